@@ -308,7 +308,7 @@ def main():
                       "step": "one frequency-model solve: re-integration + assembly of K and M, RHS, factorization, "
                               "GMRES to FP64 true residual <= 1e-8 for both polarizations; step k solves frequency "
                               "k mod 8",
-                      "path": "device multifrontal LU (FP64, nested dissection) preconditioning FP64 GMRES",
+                      "path": "device multifrontal block LDL^T (FP64, nested dissection) preconditioning FP64 GMRES",
                       "semantics": "reference arithmetic emulated (float32 Gauss points and omega, Re truncation, "
                                    "one-sided GPML, carried GPML flags) except update_sigma's linear-index range "
                                    "(geometry.f90:146-152), whose system after the first frequency cannot reach "

@@ -9,21 +9,32 @@
 // for any matrix assembled from those elements.
 //
 // Fronts: node t eliminates its n1 owned DOFs; its front also holds the n2
-// DOFs of ancestors that couple to its subtree.  The front is kept row-major
-// and split in two bands with leading dimension m = n1 + n2:
+// DOFs of ancestors that couple to its subtree.  The front is symmetric (A is)
+// and kept row-major in two bands with leading dimension m = n1 + n2:
 //   top band    T (n1 x m) = [F11 | F12]  lives in the persistent factor store
 //   bottom band B (n2 x m) = [F21 | F22]  lives in a per-level pool
-// Factorization of a front:
-//   P F11 = L U, applied to the whole top band: T = [L\U | L^-1 P F12]; the
-//   pivot of each column is searched within its 32-row panel block (with the
-//   shift below the factored matrix needs no wider search: element growth
-//   stays below ~20 and GMRES iteration counts match full partial pivoting);  then Y = U^-1 (L^-1 P F12) =
-//   F11^-1 F12 overwrites F12, and the Schur complement S = F22 - F21 Y (lower
-//   triangle, S is symmetric because A is) is extend-added into the parent.
-// The factor of a node is its top band [L\U | Y] plus the row permutation.
-// Solve with the factor (block elimination):
-//   forward  y1 = F11^-1 b1,  b2 -= Y^T b1     (F21 F11^-1 = Y^T, F11 = F11^T)
-//   backward x1 = y1 - Y x2
+// Only entries on or above the diagonal are assembled and updated.
+// Factorization of a front: block L D L^T with 64-wide diagonal blocks A_kk,
+// each factored by itself as P A_kk = L U with the pivot of every column
+// searched among the block's rows (with the shift below the factored matrix
+// needs no wider search).  For block row k, with R = A_k,rest its entries right
+// of the block,
+//   V = A_kk^-1 R = U^-1 (L^-1 P R)   overwrites R in T,
+//   R^T                               goes below the diagonal (T and F21),
+//   trailing part -= R^T V            on or above the diagonal only.
+// The Schur complement F22 -= F21 [V]_2 follows once for all block rows and is
+// extend-added into the parent.  The pivots are those of an LU with the same
+// restricted pivot search, but the symmetric form does half of its F11 work and
+// needs no second triangular solve with the whole of F11 for the n2 columns
+// (20-node 48 x 48 x 36 step: 1018 -> 744 ms, 64 x 64 x 48: 4.15 -> 3.17 s).
+// U is only ever applied by substitution: its last pivots can be ~1e-11 of the
+// largest (the shift below), and an explicit inverse of them would spread
+// rounding errors of every row that substitution keeps in the null directions.
+// The factor of a node is its top band [D blocks as L\U | V] and the blocks'
+// row permutations.  Solve with the factor:
+//   forward  b_rest -= V_k^T b_k for every block row k, front by front,
+//   y_k = A_kk^-1 b_k            for all block rows of all fronts at once,
+//   backward x_k = y_k - V_k x_rest.
 //
 // The matrix factored is A_pc = A + i*eps*|K_ii| on the diagonal of DOFs with
 // no mass (all-air DOFs), eps = kRegEps * omega * min_i(M_ii/|K_ii|): the air
@@ -49,8 +60,6 @@ constexpr int kLeafMax = 16;       // elements per leaf box
 constexpr int kNB = 64;            // panel width / triangular block size
 constexpr double kRegEps = 1e-4;   // air regularization relative to the smallest omega*M/K
 constexpr int kTile = 64;          // GEMM tile edge
-// threads of the kernels that keep one column (row) per thread in LDS
-constexpr int kColT = kNB <= 32 ? 128 : 64;
 
 struct DNode {
   int64_t n1, n2, m;
@@ -58,7 +67,7 @@ struct DNode {
   int64_t pool;  // offset of B in the level pool
   int64_t idx;   // offset of the front index list (m DOF ids, 0-based)
   int64_t rel;   // offset of the parent-relative map of the update DOFs (n2 entries)
-  int64_t pos0;  // elimination position of the first owned DOF (also pivot offset)
+  int64_t pos0;  // elimination position of the first owned DOF (also permutation offset)
   int64_t sv;    // offset (rows) of the node's solve work vector (m rows)
   int64_t inv;   // offset of the inverses of the unit-lower diagonal blocks of L (w^2 per panel block)
   int32_t child[2];
@@ -82,7 +91,10 @@ struct DirectPlan {
   // device
   DNode *d_nodes = nullptr;
   int32_t *d_lev = nullptr, *d_idx = nullptr, *d_fpos = nullptr, *d_rel = nullptr, *d_dst = nullptr;
-  int32_t *d_piv = nullptr, *d_perm = nullptr, *d_pos = nullptr;
+  int32_t *d_perm = nullptr, *d_pos = nullptr;
+  // (node, panel block) pairs of the whole tree, for the solve's diagonal blocks
+  int2 *d_blk = nullptr;
+  int64_t nblk = 0;
   double2 *d_fac = nullptr, *d_inv = nullptr;
   // level pools (the bottom bands of a level's fronts) live in one arena:
   // even levels at its start, odd levels at its end, so a level and its
@@ -124,7 +136,7 @@ struct GemmTimer {
   int used = 0;
   double ms = 0.0, flops = 0.0;
   int64_t launches = 0;
-  double mode_ms[6] = {0, 0, 0, 0, 0, 0}, mode_fl[6] = {0, 0, 0, 0, 0, 0};  // per GEMM mode
+  double mode_ms[3] = {0, 0, 0}, mode_fl[3] = {0, 0, 0};  // per GEMM mode
   void init() {
     for (int i = 0; i < kRing; i++) {
       (void)hipEventCreate(&ev[i][0]);
@@ -165,6 +177,9 @@ struct GemmTimer {
 static double now_s() {
   return std::chrono::duration<double>(std::chrono::steady_clock::now().time_since_epoch()).count();
 }
+
+// real flops of one front's factorization (n1 = a owned, n2 = b update DOFs)
+static double node_flops(double a, double b) { return 8.0 * (a * a * a / 6.0 + a * a * b / 2.0 + a * b * b / 2.0); }
 
 // ------------------------------------------------------------ symbolic ------
 struct Box {
@@ -334,9 +349,9 @@ static int build_plan_host(DirectPlan &P, int nx, int ny, int nz, int me, const 
       err = "front too large";
       return MVF_E_UNSUPPORTED;
     }
-    double a = (double)n.n1, b = (double)n.n2, m = (double)n.m;
-    // complex FMAs: wide LU, Y = U^-1 Z, lower Schur update; 8 real flops each
-    P.flops += 8.0 * (a * a * m / 2.0 - a * a * a / 6.0 + a * a * b / 2.0 + a * b * b / 2.0);
+    const double a = (double)n.n1, b = (double)n.n2;
+    // complex FMAs: symmetric factorization of F11, F12 by it, half the Schur update; 8 real flops each
+    P.flops += node_flops(a, b);
   }
   P.nidx = idxoff;
   P.nrel = reloff;
@@ -453,6 +468,8 @@ __device__ __forceinline__ void cfmac(double2 &c, double2 a, double2 b) {
   c.y += a.x * b.y - a.y * b.x;
 }
 __device__ __forceinline__ int64_t imin(int64_t a, int64_t b) { return a < b ? a : b; }
+// accumulator of v_mfma_f64_16x16x4f64
+typedef double mvf_d4 __attribute__((ext_vector_type(4)));
 // value of v in lane q (q the same in every lane) through two scalar reads
 __device__ __forceinline__ double lane_bcast(double v, int q) {
   const unsigned long long b = (unsigned long long)__double_as_longlong(v);
@@ -473,33 +490,32 @@ __global__ void k_round_c64(double2 *p, int64_t n) {
   }
 }
 
-// zeros what the assembly and extend-add of a front accumulate into: the top
-// band's lower triangle T(i, 0..i) and the bottom band's F21 and lower F22,
-// B(r, 0..n1+r).  The rest is either written whole before it is read (the top
-// band's upper part, by k_fa_sym) or never read (F22 above the diagonal: the
-// Schur update and the extend-add use its lower triangle only), so the level
-// is cleared at half the bytes of a full fill.  One wave per row.
+// zeros what the assembly and extend-add of a front accumulate into, its upper
+// triangle: F(r, r..m).  Nothing below the diagonal is read before it is
+// written (the factored block rows' transposes), so the level is cleared at half the bytes of a full
+// fill.  One wave per row.
 __global__ __launch_bounds__(256) void k_fa_zero(const DNode *nodes, const int32_t *lev, double2 *fac, double2 *pool) {
   const DNode nd = nodes[lev[blockIdx.y]];
   const int lane = threadIdx.x & 63;
   const double2 z = make_double2(0.0, 0.0);
   for (int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); r < nd.m; r += (int64_t)gridDim.x * 4) {
     double2 *row = r < nd.n1 ? fac + nd.fac + r * nd.m : pool + nd.pool + (r - nd.n1) * nd.m;
-    for (int64_t j = lane; j <= r; j += 64) row[j] = z;
+    for (int64_t j = r + lane; j < nd.m; j += 64) row[j] = z;
   }
 }
 
-// original entries: column j of the front = owned DOF d; every CSR entry (d, k)
-// whose destination row r = dst[p] >= j lands in F(r, j)
+// original entries: row j of the front = owned DOF d; every CSR entry (d, k)
+// whose front index r = dst[p] >= j lands in F(j, r)
 __global__ __launch_bounds__(256) void k_fa_assemble(const DNode *nodes, const int32_t *lev, const int32_t *idx,
                                                      const int64_t *rowptr, const int32_t *col, const int32_t *dst,
                                                      const double *K, const double *M, double w, int c64, double reg,
-                                                     double2 *fac, double2 *pool) {
+                                                     double2 *fac) {
   const DNode nd = nodes[lev[blockIdx.y]];
   const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
   for (int64_t j = (int64_t)blockIdx.x * 4 + wv; j < nd.n1; j += (int64_t)gridDim.x * 4) {
     const int32_t d = idx[nd.idx + j];
     const int64_t p1 = rowptr[d + 1];
+    double2 *row = fac + nd.fac + j * nd.m;
     for (int64_t p = rowptr[d] + lane; p < p1; p += 64) {
       const int32_t r = dst[p];
       if (r < 0) continue;
@@ -509,14 +525,14 @@ __global__ __launch_bounds__(256) void k_fa_assemble(const DNode *nodes, const i
         vi = (double)(float)vi;
       }
       if (col[p] == d && M[p] == 0.0) vi += reg * fabs(vr);
-      double2 *q = r < nd.n1 ? fac + nd.fac + (int64_t)r * nd.m + j : pool + nd.pool + (int64_t)(r - nd.n1) * nd.m + j;
-      q->x += vr;
-      q->y += vi;
+      row[r].x += vr;
+      row[r].y += vi;
     }
   }
 }
 
-// extend-add of child `slot`'s Schur complement (lower triangle of its F22)
+// extend-add of child `slot`'s Schur complement (upper triangle of its F22;
+// the relative map increases, so it lands in the parent's upper triangle)
 __global__ __launch_bounds__(256) void k_fa_extend(const DNode *nodes, const int32_t *lev, const int32_t *rel, int slot,
                                                    double2 *fac, double2 *pool, const double2 *cpool) {
   const DNode nd = nodes[lev[blockIdx.y]];
@@ -530,8 +546,8 @@ __global__ __launch_bounds__(256) void k_fa_extend(const DNode *nodes, const int
     double2 *drow = pi < nd.n1 ? fac + nd.fac + pi * nd.m : pool + nd.pool + (pi - nd.n1) * nd.m;
     // four columns per lane in flight together; the destinations of one row
     // are distinct, so the batched read-modify-writes do not overlap
-    int64_t j = lane;
-    for (; j + 192 <= i; j += 256) {
+    int64_t j = i + lane;
+    for (; j + 192 < cn.n2; j += 256) {
       int32_t pj[4];
       double2 v[4], d[4];
 #pragma unroll
@@ -548,7 +564,7 @@ __global__ __launch_bounds__(256) void k_fa_extend(const DNode *nodes, const int
         drow[pj[u]] = d[u];
       }
     }
-    for (; j <= i; j += 64) {
+    for (; j < cn.n2; j += 64) {
       const int32_t pj = rel[cn.rel + j];
       const double2 v = src[j];
       drow[pj].x += v.x;
@@ -557,40 +573,14 @@ __global__ __launch_bounds__(256) void k_fa_extend(const DNode *nodes, const int
   }
 }
 
-// upper part of the top band from the lower parts: T(i, j) = F(j, i), j > i
-__global__ __launch_bounds__(256) void k_fa_sym(const DNode *nodes, const int32_t *lev, double2 *fac,
-                                                const double2 *pool) {
-  const DNode nd = nodes[lev[blockIdx.y]];
-  const int64_t tj_n = (nd.m + 31) / 32, ti_n = (nd.n1 + 31) / 32;
-  __shared__ double2 s[32][33];
-  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-  double2 *T = fac + nd.fac;
-  const double2 *B = pool + nd.pool;
-  for (int64_t tile = blockIdx.x; tile < ti_n * tj_n; tile += gridDim.x) {
-    const int64_t ti = tile / tj_n, tj = tile % tj_n;
-    if (tj < ti) continue;
-    const int64_t i0 = ti * 32, j0 = tj * 32;
-    for (int jj = ty; jj < 32; jj += 8) {
-      const int64_t j = j0 + jj, i = i0 + tx;
-      double2 v = make_double2(0.0, 0.0);
-      if (j < nd.m && i < nd.n1) v = j < nd.n1 ? T[j * nd.m + i] : B[(j - nd.n1) * nd.m + i];
-      s[jj][tx] = v;
-    }
-    __syncthreads();
-    for (int ii = ty; ii < 32; ii += 8) {
-      const int64_t i = i0 + ii, j = j0 + tx;
-      if (i < nd.n1 && j < nd.m && j > i) T[i * nd.m + j] = s[tx][ii];
-    }
-    __syncthreads();
-  }
-}
-
-// LU of the panel's diagonal block T[k:kend, k:kend] in LDS, pivot search
-// restricted to the block's rows (kend - k <= NB); one workgroup per front.
+// LU of the panel's diagonal block T[k:kend, k:kend] in LDS, read from its
+// upper triangle, pivot search restricted to the block's rows (kend - k <= NB);
+// one workgroup per front.  perm[pos0 + k + q] is the front row that ends in
+// row k + q.
 // A pivot below `tiny` (a singular block) is replaced by `big` and counted.
 template <int NB>
 __global__ __launch_bounds__(256) void k_fa_pdiag(const DNode *nodes, const int32_t *lev, int64_t k, double2 *fac,
-                                                  double2 *inv, int32_t *piv, int *npert, double big, double tiny) {
+                                                  double2 *inv, int32_t *perm, int *npert, double big, double tiny) {
   // Four waves: lane t of every wave stands for row t, wave g for the columns
   // c = g (mod 4) of the rank-1 updates and of the inverse's updates.  The
   // pivot search, interchange and multipliers run on wave 0: two barriers per
@@ -611,10 +601,12 @@ __global__ __launch_bounds__(256) void k_fa_pdiag(const DNode *nodes, const int3
 #pragma unroll
     for (int j = 0; j < NB / 4; j++) {
       const int r = g + 4 * j;
-      const double2 v = T[(k + (r < w ? r : w - 1)) * m + k + tc];
+      const int rc = r < w ? r : w - 1;
+      const double2 v = T[(k + (rc < tc ? rc : tc)) * m + k + (rc < tc ? tc : rc)];
       a[r][t] = (r < w && t < w) ? v : make_double2(0.0, 0.0);
     }
   }
+  int32_t prow = (int32_t)(k + t);  // wave 0: front row now in row t
   __syncthreads();
   for (int q = 0; q < w; q++) {
     // wave 0 alone: pivot search, row interchange, perturbation and the
@@ -636,7 +628,9 @@ __global__ __launch_bounds__(256) void k_fa_pdiag(const DNode *nodes, const int3
           ri = oi;
         }
       }
-      if (t == 0) piv[nd.pos0 + k + q] = (int32_t)(k + ri);
+      const int32_t pq = __shfl(prow, q, 64), pr = __shfl(prow, ri, 64);
+      if (t == q) prow = pr;
+      if (t == ri) prow = pq;
       if (ri != q && t < w) {
         const double2 e = a[q][t];
         a[q][t] = a[ri][t];
@@ -675,6 +669,7 @@ __global__ __launch_bounds__(256) void k_fa_pdiag(const DNode *nodes, const int3
     const int r = g + 4 * j;
     if (r < w && t < w) T[(k + r) * m + k + t] = a[r][t];
   }
+  if (g == 0 && t < w) perm[nd.pos0 + k + t] = prow;
   // inverse X of the unit lower L_kk.  L's multipliers are bounded by 1, so
   // the explicit inverse is safe; U_kk can hold pivots ~1e-11 of the largest
   // (the air shift) and is only ever used by substitution.  Column form:
@@ -716,141 +711,121 @@ __global__ __launch_bounds__(256) void k_fa_pdiag(const DNode *nodes, const int3
   }
 }
 
-constexpr int kTrsmThreads = 256;
-constexpr int kTrsmChunk = 16;
-
-// L rows below the diagonal block: T[i, k:kend] = T[i, k:kend] U_kk^-1 for
-// i in [kend, n1).  Four lanes per row, lane l holding columns 16 l .. 16 l + 15
-// of its row in registers (one batch of loads, 1 KB contiguous per row): for
-// each column c in order the lane that owns it scales it by the reciprocal
-// pivot, passes it to the row's other lanes, and every lane subtracts its
-// multiple of row c of U_kk (read from LDS) from its later columns.
+// Block row of panel k: V = A_kk^-1 T[k:kend, kend:m] in place, and the
+// transpose of the block row as it was into the lower part (T for the owned
+// columns, F21 for the others), where the updates read it as their left operand.
+// Each wave owns 16 columns and works alone: the block row in registers as
+// MFMA operands (lane l, register v: row 4 v + l / 16, column l % 16), L^-1 by
+// products with the block inverse, U by substitution over 16-row blocks.  The
+// MFMA result layout (row l / 16 + 4 v of its 16-row block) is the operand
+// layout of the next product, so nothing is staged; inside a diagonal block the
+// sixteen steps pass the solved row from its sixteen lanes to the others.
+// Bound by its own dependency chain (64 substitution steps, about 29 us for one
+// launch on few fronts) rather than by bytes; it does the work of the row
+// interchange, L-row, U-row and n2-column solve launches of an unsymmetric band
+// LU (20-node 21 x 19 x 17: 15.0 -> 3.2 ms per factorization).
 template <int NB>
-__global__ __launch_bounds__(256) void k_fa_prows(const DNode *nodes, const int32_t *lev, int64_t k, double2 *fac) {
-  static_assert(NB == 64, "four lanes of sixteen columns per row");
+__global__ __launch_bounds__(256) void k_fa_prow(const DNode *nodes, const int32_t *lev, int64_t k, double2 *fac,
+                                                 double2 *pool, const double2 *inv, const int32_t *perm) {
+  static_assert(NB == 64, "four 16-row blocks");
   const DNode nd = nodes[lev[blockIdx.y]];
   if (k >= nd.n1) return;
-  const int64_t m = nd.m, kend = (k + NB < nd.n1) ? k + NB : nd.n1;
-  if (kend + (int64_t)blockIdx.x * 64 >= nd.n1) return;
-  const int w = (int)(kend - k);
+  const int64_t m = nd.m, n1 = nd.n1, ke = (k + NB < n1) ? k + NB : n1;
+  const int64_t c0 = ke + (int64_t)blockIdx.x * 64;
+  if (c0 >= m) return;
+  const int w = (int)(ke - k);
   double2 *T = fac + nd.fac;
-  __shared__ double2 U[NB][NB];
+  __shared__ double2 Us[4][16][16];  // Us[b][c][r] = U[16 b + r][16 b + c], r < c
   __shared__ double2 dinv[NB];
-  for (int e = threadIdx.x; e < NB * NB; e += 256) {
-    const int r = e / NB, c = e % NB;
-    const double2 v = T[(k + (r < w ? r : w - 1)) * m + k + (c < w ? c : w - 1)];
-    U[r][c] = (r < w && c < w && c >= r) ? v : make_double2(0.0, 0.0);
+  __shared__ int32_t sp[NB];
+  const int tid = threadIdx.x;
+  for (int e = tid; e < 1024; e += 256) {
+    const int b = e >> 8, r = (e >> 4) & 15, c = e & 15, R = 16 * b + r, C = 16 * b + c;
+    const double2 v = T[(k + (R < w ? R : w - 1)) * m + k + (C < w ? C : w - 1)];
+    Us[b][c][r] = (r < c && C < w) ? v : make_double2(0.0, 0.0);
+  }
+  if (tid < NB) {
+    const int64_t d = k + (tid < w ? tid : w - 1);
+    dinv[tid] = tid < w ? cinv(T[d * m + d]) : make_double2(0.0, 0.0);
+    sp[tid] = perm[nd.pos0 + d];
   }
   __syncthreads();
-  if (threadIdx.x < NB) dinv[threadIdx.x] = threadIdx.x < w ? cinv(U[threadIdx.x][threadIdx.x]) : make_double2(0, 0);
-  __syncthreads();
-  const int l = threadIdx.x & 3, rr = threadIdx.x >> 2;
-  for (int64_t i0 = kend + (int64_t)blockIdx.x * 64; i0 < nd.n1; i0 += (int64_t)gridDim.x * 64) {
-    const int64_t i = i0 + rr;
-    if (i >= nd.n1) continue;  // the row's four lanes leave together
-    double2 *row = T + i * m + k;
-    double2 x[16];
+  const int wv = tid >> 6, l = tid & 63, li = l & 15, lk = l >> 4;
+  if (c0 + wv * 16 >= m) return;
+  const int64_t j = c0 + wv * 16 + li, jc = j < m ? j : m - 1;
+  double2 x[16];
 #pragma unroll
-    for (int j = 0; j < 16; j++) {
-      const int c = 16 * l + j;
-      const double2 v = row[c < w ? c : w - 1];
-      x[j] = c < w ? v : make_double2(0.0, 0.0);
-    }
+  for (int v = 0; v < 16; v++) x[v] = T[(k + (4 * v + lk < w ? 4 * v + lk : w - 1)) * m + jc];
+  if (j < m) {
+    double2 *q = (j < n1 ? T + j * m : pool + nd.pool + (j - n1) * m) + k;
 #pragma unroll
-    for (int c = 0; c < NB; c++) {
-      if (c < w) {  // uniform; c stays a compile-time register index
-        const int o = c >> 4, jj = c & 15;
-        if (l == o) x[jj] = cmul(x[jj], dinv[c]);
-        const double2 xc = make_double2(__shfl(x[jj].x, o, 4), __shfl(x[jj].y, o, 4));
-#pragma unroll
-        for (int j = 0; j < 16; j++)
-          if (16 * l + j > c) cfms(x[j], xc, U[c][16 * l + j]);
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < 16; j++)
-      if (16 * l + j < w) row[16 * l + j] = x[j];
+    for (int v = 0; v < 16; v++)
+      if (4 * v + lk < w) q[4 * v + lk] = x[v];
   }
-}
-
-// Y block rows by back substitution, panel blocks from the last one (b = nb-1-step):
-// T[r0:r0+w, n1:m] = U_bb^-1 T[r0:r0+w, n1:m].  One thread per column walks
-// the block in 16-row chunks from the bottom: a chunk is loaded into
-// registers, reduced by the chunks solved before it (read back from the
-// band, where the thread itself stored them), solved by substitution and
-// stored.  U_bb and the reciprocal pivots are read from LDS as broadcasts.
-template <int NB>
-__global__ __launch_bounds__(kTrsmThreads, 2) void k_fa_trsm_y(const DNode *nodes, const int32_t *lev, int64_t step,
-                                                             double2 *fac) {
-  const DNode nd = nodes[lev[blockIdx.y]];
-  const int64_t b = (nd.n1 + NB - 1) / NB - 1 - step;
-  if (b < 0 || nd.n2 == 0) return;
-  const int64_t r0 = b * NB, r1 = r0 + NB < nd.n1 ? r0 + NB : nd.n1, m = nd.m;
-  const int w = (int)(r1 - r0);
-  double2 *T = fac + nd.fac;
-  __shared__ double2 U[NB][NB];
-  __shared__ double2 dinv[NB];
-  for (int e = threadIdx.x; e < NB * NB; e += kTrsmThreads) {
-    const int r = e / NB, c = e % NB;
-    U[r][c] = (r < w && c < w && c >= r) ? T[(r0 + r) * m + r0 + c] : make_double2(0.0, 0.0);
+#pragma unroll
+  for (int v = 0; v < 16; v++) {
+    const double2 t = T[sp[4 * v + lk] * m + jc];
+    x[v] = 4 * v + lk < w ? t : make_double2(0.0, 0.0);
   }
-  __syncthreads();
-  if (threadIdx.x < NB) dinv[threadIdx.x] = threadIdx.x < w ? cinv(U[threadIdx.x][threadIdx.x]) : make_double2(0, 0);
-  __syncthreads();
-  constexpr int C = kTrsmChunk, NQ = NB / kTrsmChunk;
-  for (int64_t j0 = nd.n1 + (int64_t)blockIdx.x * kTrsmThreads; j0 < m; j0 += (int64_t)gridDim.x * kTrsmThreads) {
-    const int64_t j = j0 + threadIdx.x;
-    if (j >= m) continue;
-    double2 *col = T + r0 * m + j;
-    #pragma unroll 1
-    for (int q = NQ - 1; q >= 0; q--) {
-      if (q * C >= w) continue;
-      double2 x[C];
+  // Z = L^-1 P R
+  const double2 *Li = inv + nd.inv + (int64_t)NB * NB * (k / NB);
+  mvf_d4 zr[4], zi[4];
 #pragma unroll
-      for (int r = 0; r < C; r++) x[r] = (q * C + r < w) ? col[(int64_t)(q * C + r) * m] : make_double2(0.0, 0.0);
-      #pragma unroll 1
-      for (int q2 = q + 1; q2 < NQ && q2 * C < w; q2++) {
-        double2 y[C];
+  for (int b = 0; b < 4; b++) {
+    zr[b] = zi[b] = mvf_d4{0.0, 0.0, 0.0, 0.0};
+    const int row = 16 * b + li;
 #pragma unroll
-        for (int c = 0; c < C; c++) y[c] = (q2 * C + c < w) ? col[(int64_t)(q2 * C + c) * m] : make_double2(0.0, 0.0);
-#pragma unroll
-        for (int r = 0; r < C; r++)
-#pragma unroll
-          for (int c = 0; c < C; c++) cfms(x[r], U[q * C + r][q2 * C + c], y[c]);
-      }
-      // rows past w hold zeros and zero U entries, so they stay zero
-#pragma unroll
-      for (int r = C - 1; r >= 0; r--) {
-        double2 v = x[r];
-#pragma unroll
-        for (int c = r + 1; c < C; c++) cfms(v, U[q * C + r][q * C + c], x[c]);
-        x[r] = cmul(v, dinv[q * C + r]);
-      }
-#pragma unroll
-      for (int r = 0; r < C; r++)
-        if (q * C + r < w) col[(int64_t)(q * C + r) * m] = x[r];
+    for (int q = 0; q < 4 * (b + 1); q++) {
+      const int col = 4 * q + lk;
+      const double2 t = Li[(row < w ? row : w - 1) * w + (col < w ? col : w - 1)];
+      const double2 a = (row < w && col < w) ? t : make_double2(0.0, 0.0);
+      zr[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, x[q].x, zr[b], 0, 0, 0);
+      zi[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, x[q].y, zi[b], 0, 0, 0);
+      zr[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(-a.y, x[q].y, zr[b], 0, 0, 0);
+      zi[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, x[q].x, zi[b], 0, 0, 0);
     }
   }
-}
-
-// the panel's row interchanges applied to the top band outside the panel
-template <int NB>
-__global__ __launch_bounds__(256) void k_fa_swap(const DNode *nodes, const int32_t *lev, int64_t k, double2 *fac,
-                                                 const int32_t *piv) {
-  const DNode nd = nodes[lev[blockIdx.y]];
-  if (k >= nd.n1) return;
-  const int64_t m = nd.m, kend = (k + NB < nd.n1) ? k + NB : nd.n1;
-  double2 *T = fac + nd.fac;
-  for (int64_t j = blockIdx.x * 256 + threadIdx.x; j < m; j += (int64_t)gridDim.x * 256) {
-    if (j >= k && j < kend) continue;
-    for (int64_t q = k; q < kend; q++) {
-      const int64_t r = piv[nd.pos0 + q];
-      if (r != q) {
-        const double2 a = T[q * m + j];
-        T[q * m + j] = T[r * m + j];
-        T[r * m + j] = a;
+  // V = U^-1 Z, 16-row blocks from the last
+#pragma unroll
+  for (int b = 3; b >= 0; b--) {
+    const int row = 16 * b + li;
+#pragma unroll
+    for (int jb = b + 1; jb < 4; jb++)
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const int col = 16 * jb + 4 * q + lk;
+        const double2 t = T[(k + (row < w ? row : w - 1)) * m + k + (col < w ? col : w - 1)];
+        const double2 a = (row < w && col < w) ? t : make_double2(0.0, 0.0);
+        zr[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(-a.x, zr[jb][q], zr[b], 0, 0, 0);
+        zi[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(-a.x, zi[jb][q], zi[b], 0, 0, 0);
+        zr[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, zi[jb][q], zr[b], 0, 0, 0);
+        zi[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(-a.y, zr[jb][q], zi[b], 0, 0, 0);
+      }
+#pragma unroll
+    for (int r = 15; r >= 0; r--) {
+      const int o = r & 3, v = r >> 2;
+      const double2 y = cmul(make_double2(zr[b][v], zi[b][v]), dinv[16 * b + r]);
+      const double2 s = make_double2(__shfl(y.x, li + 16 * o, 64), __shfl(y.y, li + 16 * o, 64));
+      if (lk == o) {
+        zr[b][v] = y.x;
+        zi[b][v] = y.y;
+      }
+#pragma unroll
+      for (int v2 = 0; v2 <= v; v2++) {  // rows lk + 4 v2 < r (Us is zero from r on)
+        const double2 u = Us[b][r][lk + 4 * v2];
+        zr[b][v2] -= u.x * s.x - u.y * s.y;
+        zi[b][v2] -= u.x * s.y + u.y * s.x;
       }
     }
+  }
+  if (j < m) {
+#pragma unroll
+    for (int b = 0; b < 4; b++)
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        const int r = 16 * b + lk + 4 * v;
+        if (r < w) T[(k + r) * m + j] = make_double2(zr[b][v], zi[b][v]);
+      }
   }
 }
 
@@ -860,25 +835,37 @@ __global__ __launch_bounds__(256) void k_fa_swap(const DNode *nodes, const int32
 // D[l / 16 + 4 v][l % 16] (checked on the device against a host product).  A complex product is four real MFMAs:
 // Cre += Are Bre - Aim Bim, Cim += Are Bim + Aim Bre.  Each of the four waves
 // owns a 32 x 32 quarter of the 64 x 64 tile (2 x 2 MFMA blocks).
-typedef double mvf_d4 __attribute__((ext_vector_type(4)));
+// The updates touch tiles on or above the diagonal only: C's first row and first
+// column are the same front index and Mr <= Nc.  With a tile's rows S times its
+// columns (S = 1, 2), row ti of tiles holds the columns S ti .. tn - 1.
+template <int S>
+__host__ __device__ inline int64_t upper_tiles(int64_t tm, int64_t tn) {
+  return tm * tn - S * tm * (tm - 1) / 2;
+}
+template <int S>
+__device__ __forceinline__ void upper_tile(int64_t tile, int64_t tm, int64_t tn, int64_t &ti, int64_t &tj) {
+  const double b = 2.0 * (double)tn + S;
+  ti = (int64_t)((b - sqrt(fmax(b * b - 8.0 * S * (double)tile, 0.0))) / (2.0 * S));
+  ti = ti < 0 ? 0 : (ti >= tm ? tm - 1 : ti);
+  while (ti > 0 && upper_tiles<S>(ti, tn) > tile) ti--;
+  while (ti + 1 < tm && upper_tiles<S>(ti + 1, tn) <= tile) ti++;
+  tj = S * ti + tile - upper_tiles<S>(ti, tn);
+}
 
-// C (Mr x Nc) -= A (Mr x Kd) B (Kd x Nc), or C = A B with OVERWRITE (in place
-// over B allowed: each workgroup reads its whole B column tile before it
-// writes); row-major operands with leading dimensions lda, ldb, ldc; 64 x 64
-// tiles, tile t handled by workgroup t mod gridDim.x; LOWER skips tiles above
-// the diagonal.
-template <bool OVERWRITE>
-__device__ __forceinline__ void mfma_tiles(const double2 *A, int64_t lda, const double2 *B, int64_t ldb, double2 *C,
-                                  int64_t ldc, int64_t Mr, int64_t Nc, int64_t Kd, bool lower) {
-  const int64_t tn = (Nc + kTile - 1) / kTile, tm = (Mr + kTile - 1) / kTile;
+// C (Mr x Nc) -= A (Mr x Kd) B (Kd x Nc) on or above the diagonal; row-major
+// operands with one leading dimension ld; 64 x 64 tiles, tile t handled by
+// workgroup t mod gridDim.x.
+__device__ __forceinline__ void mfma_tiles(const double2 *A, const double2 *B, double2 *C, int64_t ld, int64_t Mr,
+                                           int64_t Nc, int64_t Kd) {
+  const int64_t tn = (Nc + kTile - 1) / kTile, tm = (Mr + kTile - 1) / kTile, ntiles = upper_tiles<1>(tm, tn);
   __shared__ double2 As[kTile][17];
   __shared__ double2 Bs[16][kTile + 1];
   const int tid = threadIdx.x, wv = tid >> 6, l = tid & 63;
   const int wr = (wv >> 1) * 32, wc = (wv & 1) * 32;  // wave's quarter of the tile
   const int li = l & 15, lk = l >> 4;
-  for (int64_t tile = blockIdx.x; tile < tm * tn; tile += gridDim.x) {
-    const int64_t ti = tile / tn, tj = tile % tn;
-    if (lower && tj > ti) continue;
+  for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+    int64_t ti, tj;
+    upper_tile<1>(tile, tm, tn, ti, tj);
     const int64_t i0 = ti * kTile, j0 = tj * kTile;
     mvf_d4 cre[2][2], cim[2][2];
 #pragma unroll
@@ -896,9 +883,9 @@ __device__ __forceinline__ void mfma_tiles(const double2 *A, int64_t lda, const 
 #pragma unroll
       for (int j = 0; j < kTile * 16 / 256; j++) {
         const int e = tid + 256 * j, r = e >> 4, q = e & 15;
-        va[j] = A[imin(i0 + r, Mr - 1) * lda + imin(kk + q, Kd - 1)];
+        va[j] = A[imin(i0 + r, Mr - 1) * ld + imin(kk + q, Kd - 1)];
         const int qb = e >> 6, c = e & 63;
-        vb[j] = B[imin(kk + qb, Kd - 1) * ldb + imin(j0 + c, Nc - 1)];
+        vb[j] = B[imin(kk + qb, Kd - 1) * ld + imin(j0 + c, Nc - 1)];
       }
 #pragma unroll
       for (int j = 0; j < kTile * 16 / 256; j++) {
@@ -931,28 +918,23 @@ __device__ __forceinline__ void mfma_tiles(const double2 *A, int64_t lda, const 
     for (int rb = 0; rb < 2; rb++) {
       // C reads of one row block issued together (clamped addresses), then the updates
       double2 cv[2][4];
-      if (!OVERWRITE)
 #pragma unroll
-        for (int cb = 0; cb < 2; cb++)
+      for (int cb = 0; cb < 2; cb++)
 #pragma unroll
-          for (int v = 0; v < 4; v++) {
-            const int64_t i = i0 + wr + rb * 16 + lk + 4 * v, j = j0 + wc + cb * 16 + li;
-            cv[cb][v] = C[imin(i, Mr - 1) * ldc + imin(j, Nc - 1)];
-          }
+        for (int v = 0; v < 4; v++) {
+          const int64_t i = i0 + wr + rb * 16 + lk + 4 * v, j = j0 + wc + cb * 16 + li;
+          cv[cb][v] = C[imin(i, Mr - 1) * ld + imin(j, Nc - 1)];
+        }
 #pragma unroll
       for (int cb = 0; cb < 2; cb++)
 #pragma unroll
         for (int v = 0; v < 4; v++) {
           const int64_t i = i0 + wr + rb * 16 + lk + 4 * v, j = j0 + wc + cb * 16 + li;
           if (i < Mr && j < Nc) {
-            if (OVERWRITE) {
-              C[i * ldc + j] = make_double2(cre[rb][cb][v], cim[rb][cb][v]);
-            } else {
-              double2 o = cv[cb][v];
-              o.x -= cre[rb][cb][v];
-              o.y -= cim[rb][cb][v];
-              C[i * ldc + j] = o;
-            }
+            double2 o = cv[cb][v];
+            o.x -= cre[rb][cb][v];
+            o.y -= cim[rb][cb][v];
+            C[i * ld + j] = o;
           }
         }
     }
@@ -969,19 +951,17 @@ __device__ __forceinline__ void mfma_tiles(const double2 *A, int64_t lda, const 
 // 96 registers per lane, two waves per SIMD), 16-deep K chunks through two
 // LDS buffers with the next chunk's global loads in flight.  A is staged
 // transposed (k-major) so that both operands are read as 256-byte rows per
-// 16-lane group.  With lower set only the tiles that reach the lower triangle
-// are enumerated (row ti holds min(2 ti + 2, tn) of them; this needs Mr == Nc),
-// so no workgroup is spent on tiles above the diagonal.  When every workgroup
+// 16-lane group.  Only the tiles that reach the upper triangle are enumerated,
+// so no workgroup is spent on tiles below the diagonal.  When every workgroup
 // takes one tile, workgroups are renumbered so that each XCD (workgroups are
 // dealt round-robin to the 8 XCDs) walks an equal contiguous range of the
 // front's tiles and shares the A row panels in its L2.
 constexpr int kBig = 128;        // tile rows of the large-front GEMM
 constexpr int kBigN = 64;        // tile columns
 constexpr int kBigThreads = 512;
-static_assert(kBig == 2 * kBigN, "the lower-tile count assumes two tile columns per tile row");
-__device__ __forceinline__ void mfma_tiles3m(const double2 *A, int64_t lda, const double2 *B, int64_t ldb,
-                                             double2 *C, int64_t ldc, int64_t Mr, int64_t Nc, int64_t Kd,
-                                             bool lower) {
+static_assert(kBig == 2 * kBigN, "upper_tiles<2> counts two tile columns per tile row");
+__device__ __forceinline__ void mfma_tiles3m(const double2 *A, const double2 *B, double2 *C, int64_t ld, int64_t Mr,
+                                             int64_t Nc, int64_t Kd) {
   const int64_t tn = (Nc + kBigN - 1) / kBigN, tm = (Mr + kBig - 1) / kBig;
   __shared__ double2 As[2][16][kBig + 1];
   __shared__ double2 Bs[2][16][kBigN];
@@ -989,7 +969,7 @@ __device__ __forceinline__ void mfma_tiles3m(const double2 *A, int64_t lda, cons
   const int wr = (wv >> 1) * 32, wc = (wv & 1) * 32;
   const int li = l & 15, lk = l >> 4;
   const unsigned G = gridDim.x;
-  const int64_t ntiles = lower ? (tm - 1) * tm + tn : tm * tn;
+  const int64_t ntiles = upper_tiles<2>(tm, tn);
   // global -> register staging: A rows ar + 32 j at column aq; B rows bq + 8 j at column bc
   const int aq = tid & 15, ar = tid >> 4, bc = tid & 63, bq = tid >> 6;
   for (int64_t it = blockIdx.x; it < ntiles; it += G) {
@@ -999,15 +979,7 @@ __device__ __forceinline__ void mfma_tiles3m(const double2 *A, int64_t lda, cons
       tile = x * q + (x < rem ? x : rem) + it / 8;
     }
     int64_t ti, tj;
-    if (lower) {  // rows before ti hold ti (ti + 1) lower tiles
-      ti = (int64_t)((sqrt(4.0 * (double)tile + 1.0) - 1.0) * 0.5);
-      while (ti > 0 && ti * (ti + 1) > tile) ti--;
-      while (ti + 1 < tm && (ti + 1) * (ti + 2) <= tile) ti++;
-      tj = tile - ti * (ti + 1);
-    } else {
-      ti = tile / tn;
-      tj = tile % tn;
-    }
+    upper_tile<2>(tile, tm, tn, ti, tj);
     const int64_t i0 = ti * kBig, j0 = tj * kBigN;
     mvf_d4 t1[2][2], t2[2][2], t3[2][2];
 #pragma unroll
@@ -1021,12 +993,12 @@ __device__ __forceinline__ void mfma_tiles3m(const double2 *A, int64_t lda, cons
 #pragma unroll
       for (int j = 0; j < 4; j++) {
         const int64_t r = i0 + ar + 32 * j, q = kk + aq;
-        ra[set][j] = (r < Mr && q < Kd) ? A[r * lda + q] : make_double2(0.0, 0.0);
+        ra[set][j] = (r < Mr && q < Kd) ? A[r * ld + q] : make_double2(0.0, 0.0);
       }
 #pragma unroll
       for (int j = 0; j < 2; j++) {
         const int64_t qb = kk + bq + 8 * j, c = j0 + bc;
-        rb[set][j] = (qb < Kd && c < Nc) ? B[qb * ldb + c] : make_double2(0.0, 0.0);
+        rb[set][j] = (qb < Kd && c < Nc) ? B[qb * ld + c] : make_double2(0.0, 0.0);
       }
     };
     auto stash = [&](int set, int buf) {
@@ -1084,7 +1056,7 @@ __device__ __forceinline__ void mfma_tiles3m(const double2 *A, int64_t lda, cons
 #pragma unroll
         for (int v = 0; v < 4; v++) {
           const int64_t i = i0 + wr + r * 16 + lk + 4 * v, j = j0 + wc + c * 16 + li;
-          cv[c][v] = C[imin(i, Mr - 1) * ldc + imin(j, Nc - 1)];
+          cv[c][v] = C[imin(i, Mr - 1) * ld + imin(j, Nc - 1)];
         }
 #pragma unroll
       for (int c = 0; c < 2; c++)
@@ -1095,29 +1067,27 @@ __device__ __forceinline__ void mfma_tiles3m(const double2 *A, int64_t lda, cons
             double2 o = cv[c][v];
             o.x -= t1[r][c][v] - t2[r][c][v];
             o.y -= t3[r][c][v] - t1[r][c][v] - t2[r][c][v];
-            C[i * ldc + j] = o;
+            C[i * ld + j] = o;
           }
         }
     }
   }
 }
 
-// Two-level blocking of the top band's LU and of the Y solve: 64-wide panels
-// (kNB) inside outer blocks of kOuter columns (rows for Y).  Updates that
-// reach past the outer block are deferred and applied once per outer block
-// with K = kOuter, so the trailing part of a front is read and written
-// kOuter/kNB times less often than by rank-64 updates.
+// Two-level blocking of the top band: 64-wide panels (kNB) inside outer blocks
+// of kOuter rows.  A panel updates the rows of its outer block; the rows past
+// it are updated once per outer block with K = kOuter, so the trailing part of
+// a front is read and written kOuter/kNB times less often than by rank-64
+// updates.
 constexpr int64_t kGroup = 4;  // panels per outer block
 constexpr int64_t kOuter = kGroup * kNB;
 
 // operands of the batched GEMM launches, as offsets into the front's top
-// band T (or its pool band for the Schur update), all with leading dimension m
-//   MODE 0: LU, inner: T[ke:n1, ke:K1] -= T[ke:n1, k:ke] T[k:ke, ke:K1]
-//   MODE 3: LU, rows of the outer block past it: T[ke:K1, K1:m] -= T[ke:K1, k:ke] T[k:ke, K1:m]
-//   MODE 4: LU, outer: T[K1:n1, K1:m] -= T[K1:n1, K0:K1] T[K0:K1, K1:m]
-//   MODE 1: Y, inner: rows [R0, r0) of the outer group of block b = nb-1-step
-//   MODE 5: Y, outer: rows [0, R0) once the group's first block b = R0/kNB is solved
-//   MODE 2: Schur complement F22 -= F21 Y (lower tiles only)
+// band T (or its pool band for the Schur update), all with leading dimension m,
+// on or above the diagonal:
+//   MODE 0: inner: T[ke:K1, ke:m] -= T[ke:K1, k:ke] T[k:ke, ke:m]
+//   MODE 1: outer: T[K1:n1, K1:m] -= T[K1:n1, K0:K1] T[K0:K1, K1:m]
+//   MODE 2: Schur complement F22 -= F21 T[0:n1, n1:m]
 // with ke = min(k + kNB, n1) and K1 = min(K0 + kOuter, n1).
 struct GemmArgs {
   int64_t a, b, c, Mr, Nc, Kd;
@@ -1126,69 +1096,28 @@ struct GemmArgs {
 __host__ __device__ inline GemmArgs gemm_args(int mode, const DNode &nd, int64_t step, int64_t K0) {
   const int64_t n1 = nd.n1, n2 = nd.n2, m = nd.m;
   GemmArgs g{0, 0, 0, 0, 0, 0, false};
-  if (mode == 0 || mode == 3) {
+  if (mode == 0) {
     const int64_t k = step;
     if (k >= n1) return g;
     const int64_t ke = (k + kNB < n1) ? k + kNB : n1, K1 = (K0 + kOuter < n1) ? K0 + kOuter : n1;
     g.a = ke * m + k;
+    g.b = k * m + ke;
+    g.c = ke * m + ke;
+    g.Mr = K1 - ke;
+    g.Nc = m - ke;
     g.Kd = ke - k;
-    if (mode == 0) {
-      g.b = k * m + ke;
-      g.c = ke * m + ke;
-      g.Mr = n1 - ke;
-      g.Nc = K1 - ke;
-    } else {
-      g.b = k * m + K1;
-      g.c = ke * m + K1;
-      g.Mr = K1 - ke;
-      g.Nc = m - K1;
-    }
-  } else if (mode == 4) {
+  } else if (mode == 1) {
     // step selects the part: 0 the whole update; with K1n = min(K1 + kOuter, n1),
-    // 1 the next outer block's columns T[K1:n1, K1:K1n], 2 its rows past them
-    // T[K1:K1n, K1n:m], 3 the trailing rest T[K1n:n1, K1n:m]
+    // 1 the next outer block's rows T[K1:K1n, K1:m], 2 the rows past them T[K1n:n1, K1n:m]
     if (K0 >= n1) return g;
     const int64_t K1 = (K0 + kOuter < n1) ? K0 + kOuter : n1, K1n = (K1 + kOuter < n1) ? K1 + kOuter : n1;
-    int64_t r0 = K1, r1 = n1, c0 = K1, c1 = m;
-    if (step == 1) {
-      c1 = K1n;
-    } else if (step == 2) {
-      r1 = K1n;
-      c0 = K1n;
-    } else if (step == 3) {
-      r0 = K1n;
-      c0 = K1n;
-    }
+    const int64_t r0 = step == 2 ? K1n : K1, r1 = step == 1 ? K1n : n1;
     g.a = r0 * m + K0;
-    g.b = K0 * m + c0;
-    g.c = r0 * m + c0;
+    g.b = K0 * m + r0;
+    g.c = r0 * m + r0;
     g.Mr = r1 - r0;
-    g.Nc = c1 - c0;
+    g.Nc = m - r0;
     g.Kd = K1 - K0;
-  } else if (mode == 1 || mode == 5) {
-    const int64_t nbk = (n1 + kNB - 1) / kNB, bb = nbk - 1 - step;
-    if (bb < 0 || n2 == 0) return g;
-    const int64_t r0 = bb * kNB, r1 = (r0 + kNB < n1) ? r0 + kNB : n1;
-    g.Nc = n2;
-    if (mode == 1) {
-      const int64_t R0 = (bb / kGroup) * kOuter;
-      g.a = R0 * m + r0;
-      g.b = r0 * m + n1;
-      g.c = R0 * m + n1;
-      g.Mr = r0 - R0;
-      g.Kd = r1 - r0;
-    } else {
-      // K0 selects the part: 0 all rows [0, r0); 1 the next group's rows
-      // [r0 - kOuter, r0); 2 the rows above them [0, r0 - kOuter)
-      if (bb % kGroup != 0) return g;
-      const int64_t R1 = (r0 + kOuter < n1) ? r0 + kOuter : n1, rs = r0 > kOuter ? r0 - kOuter : 0;
-      const int64_t q0 = K0 == 1 ? rs : 0, q1 = K0 == 2 ? rs : r0;
-      g.a = q0 * m + r0;
-      g.b = r0 * m + n1;
-      g.c = q0 * m + n1;
-      g.Mr = q1 - q0;
-      g.Kd = R1 - r0;
-    }
   } else {
     g.a = 0;
     g.b = n1;
@@ -1212,47 +1141,8 @@ __global__ __launch_bounds__(BIG ? kBigThreads : 256, 2) void k_fa_gemm_mfma(con
   const int64_t m = nd.m;
   double2 *T = fac + nd.fac;
   double2 *AC = (MODE == 2) ? pool + nd.pool : T;  // the Schur update reads F21 and writes F22 in the pool band
-  if constexpr (BIG) mfma_tiles3m(AC + g.a, m, T + g.b, m, AC + g.c, m, g.Mr, g.Nc, g.Kd, MODE == 2);
-  else mfma_tiles<false>(AC + g.a, m, T + g.b, m, AC + g.c, m, g.Mr, g.Nc, g.Kd, MODE == 2);
-}
-
-// U row block on the matrix cores, in place, for columns [c0, c1):
-//   T[k:k+w, c0:c1] = Linv_b T[k:k+w, c0:c1],  b = k / kNB
-// part 0: c0 = k + w, c1 = K1 (inside the outer block); part 1: c0 = K1, c1 = m
-__host__ __device__ inline void urow_cols(const DNode &nd, int64_t k, int64_t K0, int part, int64_t &c0, int64_t &c1) {
-  const int64_t n1 = nd.n1, w = (k + kNB < n1) ? kNB : n1 - k, K1 = (K0 + kOuter < n1) ? K0 + kOuter : n1;
-  c0 = part ? K1 : k + w;
-  c1 = part ? nd.m : K1;
-}
-__global__ __launch_bounds__(256) void k_fa_urow(const DNode *nodes, const int32_t *lev, int64_t k, int64_t K0,
-                                                 int part, double2 *fac, const double2 *inv) {
-  const DNode nd = nodes[lev[blockIdx.y]];
-  const int64_t n1 = nd.n1, m = nd.m;
-  if (k >= n1) return;
-  const int64_t b = k / kNB, w = (k + kNB < n1) ? kNB : n1 - k;
-  int64_t c0, c1;
-  urow_cols(nd, k, K0, part, c0, c1);
-  if (c0 >= c1) return;
-  double2 *T = fac + nd.fac;
-  mfma_tiles<true>(inv + nd.inv + kNB * kNB * b, w, T + k * m + c0, m, T + k * m + c0, m, w, c1 - c0, w, false);
-}
-
-// row permutation of each front from its interchange sequence.  The pivot
-// search never leaves a kNB-row panel block, so the blocks' permutations are
-// independent: one thread per (block, front), kNB interchanges each.
-__global__ void k_fa_perm(const DNode *nodes, const int32_t *lev, const int32_t *piv, int32_t *perm) {
-  const DNode nd = nodes[lev[blockIdx.y]];
-  const int64_t b0 = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * kNB;
-  if (b0 >= nd.n1) return;
-  const int64_t b1 = b0 + kNB < nd.n1 ? b0 + kNB : nd.n1;
-  int32_t *p = perm + nd.pos0;
-  for (int64_t q = b0; q < b1; q++) p[q] = (int32_t)q;
-  for (int64_t q = b0; q < b1; q++) {
-    const int64_t r = piv[nd.pos0 + q];
-    const int32_t a = p[q];
-    p[q] = p[r];
-    p[r] = a;
-  }
+  if constexpr (BIG) mfma_tiles3m(AC + g.a, T + g.b, AC + g.c, m, g.Mr, g.Nc, g.Kd);
+  else mfma_tiles(AC + g.a, T + g.b, AC + g.c, m, g.Mr, g.Nc, g.Kd);
 }
 
 // ----------------------------------------------------------- solve kernels --
@@ -1285,212 +1175,188 @@ __global__ __launch_bounds__(256) void k_sv_extend(const DNode *nodes, const int
   }
 }
 
-// W2[j] -= sum_i Y[i][j] W1[i]
+// Forward sweep inside an outer block of rows [K0, K1), K1 = min(K0 + kOuter,
+// n1): W[j] -= sum_r V[r][j] W[r] over the block's panels in order, for the
+// columns j of the block right of each panel.  One workgroup per front; a wave
+// takes 16 columns with four lanes of 16 rows each per column.
 template <int NC>
-__global__ __launch_bounds__(256) void k_sv_contrib(const DNode *nodes, const int32_t *lev, const double2 *fac,
-                                                    double2 *W) {
-  const DNode nd = nodes[lev[blockIdx.y]];
-  if (nd.n1 == 0) return;
-  const double2 *T = fac + nd.fac;
-  __shared__ double2 s[256][NC];
-  for (int64_t jb = blockIdx.x; jb * 256 < nd.n2; jb += gridDim.x) {
-    const int64_t j = jb * 256 + threadIdx.x;
+__global__ __launch_bounds__(768) void k_sv_fblock(const DNode *nodes, const int32_t *lev, int64_t K0,
+                                                   const double2 *fac, double2 *W) {
+  const DNode nd = nodes[lev[blockIdx.x]];
+  const int64_t K1 = K0 + kOuter < nd.n1 ? K0 + kOuter : nd.n1;
+  if (K0 + kNB >= K1) return;
+  const int nb = (int)(K1 - K0);
+  const int64_t m = nd.m;
+  const double2 *T = fac + nd.fac + K0 * m + K0;
+  double2 *Wb = W + (nd.sv + K0) * NC;
+  __shared__ double2 s[kOuter][NC];
+  for (int e = threadIdx.x; e < nb * NC; e += 768) s[e / NC][e % NC] = Wb[e];
+  __syncthreads();
+  const int l = threadIdx.x & 63, li = l & 15, lq = l >> 4, wv = threadIdx.x >> 6;
+  for (int p = 0; p + kNB < nb; p += kNB) {
+    const int j = p + kNB + wv * 16 + li, jc = j < nb ? j : nb - 1;
     double2 acc[NC];
 #pragma unroll
     for (int c = 0; c < NC; c++) acc[c] = make_double2(0.0, 0.0);
-    for (int64_t i0 = 0; i0 < nd.n1; i0 += 256) {
-      for (int e = threadIdx.x; e < 256 * NC; e += 256) {
-        const int r = e / NC, c = e % NC;
-        s[r][c] = i0 + r < nd.n1 ? W[(nd.sv + i0 + r) * NC + c] : make_double2(0.0, 0.0);
+    const double2 *V = T + (int64_t)(p + 16 * lq) * m + jc;
+    if (p + kNB + wv * 16 < nb) {
+#pragma unroll
+      for (int r0 = 0; r0 < 16; r0 += 8) {
+        double2 v[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) v[u] = V[(r0 + u) * m];
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+#pragma unroll
+          for (int c = 0; c < NC; c++) cfma(acc[c], v[u], s[p + 16 * lq + r0 + u][c]);
       }
-      __syncthreads();
-      if (j < nd.n2) {
-        const int64_t lim = (nd.n1 - i0) < 256 ? nd.n1 - i0 : 256;
-        int64_t r = 0;
-        for (; r + 8 <= lim; r += 8) {  // eight rows' loads in flight together
-          double2 y[8];
 #pragma unroll
-          for (int u = 0; u < 8; u++) y[u] = T[(i0 + r + u) * nd.m + nd.n1 + j];
+      for (int c = 0; c < NC; c++)
 #pragma unroll
-          for (int u = 0; u < 8; u++)
-#pragma unroll
-            for (int c = 0; c < NC; c++) cfma(acc[c], y[u], s[r + u][c]);
+        for (int off = 16; off < 64; off <<= 1) {
+          acc[c].x += __shfl_xor(acc[c].x, off, 64);
+          acc[c].y += __shfl_xor(acc[c].y, off, 64);
         }
-        for (; r < lim; r++) {
-          const double2 y = T[(i0 + r) * nd.m + nd.n1 + j];
+      if (lq == 0 && j < nb)
 #pragma unroll
-          for (int c = 0; c < NC; c++) cfma(acc[c], y, s[r][c]);
+        for (int c = 0; c < NC; c++) {
+          s[j][c].x -= acc[c].x;
+          s[j][c].y -= acc[c].y;
         }
-      }
-      __syncthreads();
     }
-    if (j < nd.n2)
+    __syncthreads();
+  }
+  for (int e = threadIdx.x; e < nb * NC; e += 768) Wb[e] = s[e / NC][e % NC];
+}
+
+// the same block's contribution to the columns past it: W[j] -= sum_r V[r][j]
+// W[r], r in [K0, K1), j in [K1, m); 16 columns per wave, four lanes per
+// column, each over a quarter of the rows
+template <int NC>
+__global__ __launch_bounds__(256) void k_sv_frest(const DNode *nodes, const int32_t *lev, int64_t K0,
+                                                  const double2 *fac, double2 *W) {
+  const DNode nd = nodes[lev[blockIdx.y]];
+  if (K0 >= nd.n1) return;
+  const int64_t K1 = K0 + kOuter < nd.n1 ? K0 + kOuter : nd.n1, m = nd.m;
+  if (K1 + (int64_t)blockIdx.x * 64 >= m) return;
+  const int nb = (int)(K1 - K0);
+  __shared__ double2 s[kOuter][NC];
+  for (int e = threadIdx.x; e < nb * NC; e += 256) s[e / NC][e % NC] = W[(nd.sv + K0) * NC + e];
+  __syncthreads();
+  const int l = threadIdx.x & 63, li = l & 15, lq = l >> 4, wv = threadIdx.x >> 6;
+  const int nq = (nb + 3) / 4, ra = lq * nq < nb ? lq * nq : nb, rb = ra + nq < nb ? ra + nq : nb;
+  for (int64_t j0 = K1 + (int64_t)blockIdx.x * 64 + wv * 16; j0 < m; j0 += (int64_t)gridDim.x * 64) {
+    const int64_t j = j0 + li, jc = j < m ? j : m - 1;
+    const double2 *V = fac + nd.fac + K0 * m + jc;
+    double2 acc[NC];
+#pragma unroll
+    for (int c = 0; c < NC; c++) acc[c] = make_double2(0.0, 0.0);
+    int r = ra;
+    for (; r + 8 <= rb; r += 8) {  // eight rows' loads in flight together
+      double2 v[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) v[u] = V[(r + u) * m];
+#pragma unroll
+      for (int u = 0; u < 8; u++)
+#pragma unroll
+        for (int c = 0; c < NC; c++) cfma(acc[c], v[u], s[r + u][c]);
+    }
+    for (; r < rb; r++) {
+      const double2 v = V[r * m];
+#pragma unroll
+      for (int c = 0; c < NC; c++) cfma(acc[c], v, s[r][c]);
+    }
+#pragma unroll
+    for (int c = 0; c < NC; c++)
+#pragma unroll
+      for (int off = 16; off < 64; off <<= 1) {
+        acc[c].x += __shfl_xor(acc[c].x, off, 64);
+        acc[c].y += __shfl_xor(acc[c].y, off, 64);
+      }
+    if (lq == 0 && j < m)
 #pragma unroll
       for (int c = 0; c < NC; c++) {
-        double2 &o = W[(nd.sv + nd.n1 + j) * NC + c];
+        double2 &o = W[(nd.sv + j) * NC + c];
         o.x -= acc[c].x;
         o.y -= acc[c].y;
       }
   }
 }
 
-template <int NC>
-__global__ __launch_bounds__(256) void k_sv_perm(const DNode *nodes, const int32_t *lev, const int32_t *perm,
-                                                 const double2 *W, double2 *zb) {
-  const DNode nd = nodes[lev[blockIdx.y]];
-  for (int64_t e = blockIdx.x * 256 + threadIdx.x; e < nd.n1 * NC; e += (int64_t)gridDim.x * 256) {
-    const int64_t q = e / NC;
-    const int c = (int)(e % NC);
-    zb[(nd.pos0 + q) * NC + c] = W[(nd.sv + perm[nd.pos0 + q]) * NC + c];
-  }
-}
-
-// z_b = Linv_b z_b for panel block b of each front: a (w x w) by (w x NC)
-// product, one workgroup per front
+// y = A_kk^-1 b for every panel block of the tree at once, one workgroup per
+// block: L through its stored inverse (four lanes per row), then U by
+// substitution on one wave, lane r holding row r of the strict upper block
+// column-major in LDS, the solved value broadcast by scalar lane reads.
 template <int NC, int NB>
-__global__ __launch_bounds__(256) void k_sv_ldiag(const DNode *nodes, const int32_t *lev, int64_t b,
-                                                  const double2 *inv, double2 *zb) {
-  const DNode nd = nodes[lev[blockIdx.x]];
-  const int64_t r0 = b * NB;
-  if (r0 >= nd.n1) return;
-  const int w = (int)((r0 + NB < nd.n1) ? NB : nd.n1 - r0);
-  const double2 *Ai = inv + nd.inv + (int64_t)NB * NB * b;
-  __shared__ double2 z[NB][NC];
-  for (int e = threadIdx.x; e < w * NC; e += 256) z[e / NC][e % NC] = zb[(nd.pos0 + r0) * NC + e];
-  __syncthreads();
-  for (int e = threadIdx.x; e < w * NC; e += 256) {
+__global__ __launch_bounds__(256) void k_sv_diag(const DNode *nodes, const int2 *blk, const double2 *fac,
+                                                 const double2 *inv, const int32_t *perm, const double2 *W,
+                                                 double2 *zb) {
+  static_assert(NB == 64, "one lane per row of the diagonal block");
+  const int2 nb = blk[blockIdx.x];
+  const DNode nd = nodes[nb.x];
+  const int64_t r0 = (int64_t)nb.y * NB, r1 = r0 + NB < nd.n1 ? r0 + NB : nd.n1;
+  const int w = (int)(r1 - r0);
+  const double2 *T = fac + nd.fac;
+  const double2 *Ai = inv + nd.inv + (int64_t)NB * NB * nb.y;
+  __shared__ double2 S[NB][NB + 1];  // S[col][row] = U[row][col], row < col; padded for conflict-free writes
+  __shared__ double2 z[NB][NC], y[NB][NC];
+  const int tid = threadIdx.x;
+  for (int e = tid; e < NB * NC; e += 256) {
     const int r = e / NC, c = e % NC;
-    double2 acc = make_double2(0.0, 0.0);
-    for (int q = 0; q <= r; q++) cfma(acc, Ai[r * w + q], z[q][c]);
-    zb[(nd.pos0 + r0) * NC + e] = acc;
+    z[r][c] = r < w ? W[(nd.sv + perm[nd.pos0 + r0 + r]) * NC + c] : make_double2(0.0, 0.0);
   }
-}
-
-// z[r] -= sum_{q<w} M[r][q] zblk[q] for the rows r in [rb, re) of a front,
-// M[r] = M0 + r m: sixteen lanes per row, lane l taking columns l, l + 16,
-// l + 32, l + 48 (each load instruction reads 256 contiguous bytes per row),
-// then a reduction over the sixteen lanes.  zblk rows past w are zero.
-template <int NC, int NB>
-__device__ __forceinline__ void sv_rows_update(const double2 *M0, int64_t m, int w, int64_t rb, int64_t re,
-                                               const double2 (*zblk)[NC], double2 *zrows) {
-  static_assert(NB == 64, "four columns per lane");
-  const int l16 = threadIdx.x & 15, rr = threadIdx.x >> 4;
-  for (int64_t r0 = rb + (int64_t)blockIdx.x * 16; r0 < re; r0 += (int64_t)gridDim.x * 16) {
-    const int64_t r = r0 + rr;
+#pragma unroll 16
+  for (int q = tid >> 6; q < NB; q += 4) {
+    const int r = tid & 63;  // column r of row q
+    const double2 u = T[(r0 + (q < w ? q : w - 1)) * nd.m + r0 + (r < w ? r : w - 1)];
+    S[r][q] = (q < w && r < w && r > q) ? u : make_double2(0.0, 0.0);
+  }
+  __syncthreads();
+  {
+    const int r = tid >> 2, l4 = tid & 3, rc = r < w ? r : w - 1;
     double2 acc[NC];
 #pragma unroll
     for (int c = 0; c < NC; c++) acc[c] = make_double2(0.0, 0.0);
-    if (r < re) {
-      const double2 *Mr = M0 + r * m;
-      double2 v[4];
+#pragma unroll 8
+    for (int q = l4; q < NB; q += 4) {
+      const double2 a = Ai[rc * w + (q < w ? q : w - 1)];
+      if (q < w)
 #pragma unroll
-      for (int u = 0; u < 4; u++) v[u] = Mr[l16 + 16 * u < w ? l16 + 16 * u : w - 1];
-#pragma unroll
-      for (int u = 0; u < 4; u++)
-        if (l16 + 16 * u < w)
-#pragma unroll
-          for (int c = 0; c < NC; c++) cfma(acc[c], v[u], zblk[l16 + 16 * u][c]);
+        for (int c = 0; c < NC; c++) cfma(acc[c], a, z[q][c]);
     }
 #pragma unroll
     for (int c = 0; c < NC; c++)
 #pragma unroll
-      for (int off = 8; off > 0; off >>= 1) {
-        acc[c].x += __shfl_xor(acc[c].x, off, 16);
-        acc[c].y += __shfl_xor(acc[c].y, off, 16);
+      for (int off = 1; off < 4; off <<= 1) {
+        acc[c].x += __shfl_xor(acc[c].x, off, 4);
+        acc[c].y += __shfl_xor(acc[c].y, off, 4);
       }
-    if (r < re)
+    if (l4 == 0)
 #pragma unroll
-      for (int c = 0; c < NC; c++)
-        if (l16 == c) {  // lane c of the group writes column c
-          double2 &o = zrows[r * NC + c];
-          o.x -= acc[c].x;
-          o.y -= acc[c].y;
-        }
-  }
-}
-
-// rows below block b: z[r] -= L[r][b0:b1] z[b0:b1]
-template <int NC, int NB>
-__global__ __launch_bounds__(256) void k_sv_lupd(const DNode *nodes, const int32_t *lev, int64_t b, const double2 *fac,
-                                                 double2 *zb) {
-  const DNode nd = nodes[lev[blockIdx.y]];
-  const int64_t b0 = b * NB;
-  if (b0 >= nd.n1) return;
-  const int64_t b1 = b0 + NB < nd.n1 ? b0 + NB : nd.n1;
-  const int w = (int)(b1 - b0);
-  if (b1 + (int64_t)blockIdx.x * 16 >= nd.n1) return;
-  __shared__ double2 z[NB][NC];
-  for (int e = threadIdx.x; e < NB * NC; e += 256) {
-    const int r = e / NC, c = e % NC;
-    z[r][c] = r < w ? zb[(nd.pos0 + b0 + r) * NC + c] : make_double2(0.0, 0.0);
+      for (int c = 0; c < NC; c++) y[r][c] = acc[c];
   }
   __syncthreads();
-  sv_rows_update<NC, NB>(fac + nd.fac + b0, nd.m, w, b1, nd.n1, z, zb + nd.pos0 * NC);
-}
-
-// back substitution (upper U) inside panel block b = nb-1-step: one wave per
-// front, lane r owns row r.  The strict upper block is staged column-major in
-// LDS by one batch of independent loads; each step scales row q by its
-// precomputed diagonal reciprocal, broadcasts it across the wave and updates
-// the rows above it, with no barrier inside the substitution.
-template <int NC, int NB>
-__global__ __launch_bounds__(64) void k_sv_udiag(const DNode *nodes, const int32_t *lev, int64_t step,
-                                                 const double2 *fac, double2 *zb) {
-  static_assert(NB == 64, "one lane per row of the diagonal block");
-  const DNode nd = nodes[lev[blockIdx.x]];
-  const int64_t b = (nd.n1 + NB - 1) / NB - 1 - step;
-  if (b < 0) return;
-  const int64_t r0 = b * NB, r1 = r0 + NB < nd.n1 ? r0 + NB : nd.n1;
-  const int w = (int)(r1 - r0);
-  const double2 *T = fac + nd.fac;
-  __shared__ double2 S[NB][NB + 1];  // S[col][row] = U[row][col], row < col; padded for conflict-free writes
-  const int r = threadIdx.x;
-  const int rc = r < w ? r : w - 1;
-#pragma unroll 16
-  for (int q = 0; q < NB; q++) {
-    // lane r reads U[q][r] of row q (coalesced, clamped address, padding selected afterwards)
-    const double2 u = T[(r0 + (q < w ? q : w - 1)) * nd.m + r0 + rc];
-    S[r][q] = (q < w && r < w && r > q) ? u : make_double2(0.0, 0.0);
-  }
+  if (tid >= 64) return;
+  const int r = tid;
   const double2 dinv = r < w ? cinv(T[(r0 + r) * nd.m + r0 + r]) : make_double2(0.0, 0.0);
-  double2 z[NC];
+  double2 zc[NC];
 #pragma unroll
-  for (int c = 0; c < NC; c++) z[c] = r < w ? zb[(nd.pos0 + r0 + r) * NC + c] : make_double2(0.0, 0.0);
-  __syncthreads();
+  for (int c = 0; c < NC; c++) zc[c] = y[r][c];
   for (int q = w - 1; q >= 0; q--) {
     const double2 u = S[q][r];
 #pragma unroll
     for (int c = 0; c < NC; c++) {
-      if (r == q) z[c] = cmul(z[c], dinv);
-      const double2 zq = make_double2(lane_bcast(z[c].x, q), lane_bcast(z[c].y, q));
-      if (r < q) cfms(z[c], u, zq);
+      if (r == q) zc[c] = cmul(zc[c], dinv);
+      const double2 zq = make_double2(lane_bcast(zc[c].x, q), lane_bcast(zc[c].y, q));
+      if (r < q) cfms(zc[c], u, zq);
     }
   }
   if (r < w)
 #pragma unroll
-    for (int c = 0; c < NC; c++) zb[(nd.pos0 + r0 + r) * NC + c] = z[c];
+    for (int c = 0; c < NC; c++) zb[(nd.pos0 + r0 + r) * NC + c] = zc[c];
 }
 
-// rows above block b = nb-1-step: z[r] -= U[r][r0:r1] z[r0:r1]
-template <int NC, int NB>
-__global__ __launch_bounds__(256) void k_sv_uupd(const DNode *nodes, const int32_t *lev, int64_t step,
-                                                 const double2 *fac, double2 *zb) {
-  const DNode nd = nodes[lev[blockIdx.y]];
-  const int64_t b = (nd.n1 + NB - 1) / NB - 1 - step;
-  if (b <= 0) return;
-  const int64_t r0 = b * NB, r1 = r0 + NB < nd.n1 ? r0 + NB : nd.n1;
-  const int w = (int)(r1 - r0);
-  if ((int64_t)blockIdx.x * 16 >= r0) return;
-  __shared__ double2 z[NB][NC];
-  for (int e = threadIdx.x; e < NB * NC; e += 256) {
-    const int r = e / NC, c = e % NC;
-    z[r][c] = r < w ? zb[(nd.pos0 + r0 + r) * NC + c] : make_double2(0.0, 0.0);
-  }
-  __syncthreads();
-  sv_rows_update<NC, NB>(fac + nd.fac + r0, nd.m, w, 0, r0, z, zb + nd.pos0 * NC);
-}
-
-// backward: x1[i] = y1[i] - sum_j Y[i][j] x2[j]; one wave per row
+// backward, update columns: z[i] -= sum_j V[i][n1 + j] x2[j]; one wave per row
 template <int NC>
 __global__ __launch_bounds__(256) void k_sv_back(const DNode *nodes, const int32_t *lev, const int32_t *fpos,
                                                  const double2 *fac, double2 *zb) {
@@ -1523,6 +1389,96 @@ __global__ __launch_bounds__(256) void k_sv_back(const DNode *nodes, const int32
   }
 }
 
+// backward, owned columns past the outer block at K0: z[i] -= sum_j V[i][j] z[j],
+// i in [K0, K1), j in [K1, n1); one workgroup per row
+template <int NC>
+__global__ __launch_bounds__(256) void k_sv_brest(const DNode *nodes, const int32_t *lev, int64_t K0,
+                                                  const double2 *fac, double2 *zb) {
+  const DNode nd = nodes[lev[blockIdx.y]];
+  const int64_t K1 = K0 + kOuter, i = K0 + blockIdx.x;
+  if (K1 >= nd.n1) return;  // uniform; rows i < K0 + kOuter = K1 < n1 all exist
+  const double2 *Vr = fac + nd.fac + i * nd.m;
+  const double2 *z = zb + nd.pos0 * NC;
+  const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  double2 acc[NC];
+#pragma unroll
+  for (int c = 0; c < NC; c++) acc[c] = make_double2(0.0, 0.0);
+#pragma unroll 4
+  for (int64_t j = K1 + threadIdx.x; j < nd.n1; j += 256) {
+    const double2 v = Vr[j];
+#pragma unroll
+    for (int c = 0; c < NC; c++) cfma(acc[c], v, z[j * NC + c]);
+  }
+  __shared__ double2 s[4][NC];
+#pragma unroll
+  for (int c = 0; c < NC; c++) {
+    for (int off = 32; off > 0; off >>= 1) {
+      acc[c].x += __shfl_xor(acc[c].x, off, 64);
+      acc[c].y += __shfl_xor(acc[c].y, off, 64);
+    }
+    if (lane == 0) s[wv][c] = acc[c];
+  }
+  __syncthreads();
+  if (threadIdx.x < NC) {
+    const int c = threadIdx.x;
+    double2 &o = zb[(nd.pos0 + i) * NC + c];
+    o.x -= s[0][c].x + s[1][c].x + s[2][c].x + s[3][c].x;
+    o.y -= s[0][c].y + s[1][c].y + s[2][c].y + s[3][c].y;
+  }
+}
+
+// backward inside an outer block: its panels from the last, z[r] -= sum_c
+// V[r][c] z[c] over the block's columns right of the panel; one workgroup per
+// front, four rows per wave
+template <int NC>
+__global__ __launch_bounds__(1024) void k_sv_bblock(const DNode *nodes, const int32_t *lev, int64_t K0,
+                                                    const double2 *fac, double2 *zb) {
+  const DNode nd = nodes[lev[blockIdx.x]];
+  const int64_t K1 = K0 + kOuter < nd.n1 ? K0 + kOuter : nd.n1;
+  if (K0 + kNB >= K1) return;
+  const int nb = (int)(K1 - K0);
+  const int64_t m = nd.m;
+  const double2 *T = fac + nd.fac + K0 * m + K0;
+  double2 *Zb = zb + (nd.pos0 + K0) * NC;
+  __shared__ double2 s[kOuter][NC];
+  for (int e = threadIdx.x; e < nb * NC; e += 1024) s[e / NC][e % NC] = Zb[e];
+  __syncthreads();
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  for (int p = (nb - 1) / kNB - 1; p >= 0; p--) {
+    const int j0 = (p + 1) * kNB;
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const int r = p * kNB + wv * 4 + u;
+      double2 v[3];
+#pragma unroll
+      for (int q = 0; q < 3; q++) v[q] = T[(int64_t)r * m + (j0 + 64 * q + lane < nb ? j0 + 64 * q + lane : nb - 1)];
+      double2 acc[NC];
+#pragma unroll
+      for (int c = 0; c < NC; c++) acc[c] = make_double2(0.0, 0.0);
+#pragma unroll
+      for (int q = 0; q < 3; q++)
+        if (j0 + 64 * q + lane < nb)
+#pragma unroll
+          for (int c = 0; c < NC; c++) cfma(acc[c], v[q], s[j0 + 64 * q + lane][c]);
+#pragma unroll
+      for (int c = 0; c < NC; c++)
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) {
+          acc[c].x += __shfl_xor(acc[c].x, off, 64);
+          acc[c].y += __shfl_xor(acc[c].y, off, 64);
+        }
+#pragma unroll
+      for (int c = 0; c < NC; c++)
+        if (lane == c) {
+          s[r][c].x -= acc[c].x;
+          s[r][c].y -= acc[c].y;
+        }
+    }
+    __syncthreads();
+  }
+  for (int e = threadIdx.x; e < nb * NC; e += 1024) Zb[e] = s[e / NC][e % NC];
+}
+
 template <int NC>
 __global__ void k_sv_out(int64_t n, const int32_t *pos, const double2 *zb, double2 *x) {
   for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < n * NC; e += (int64_t)gridDim.x * blockDim.x) {
@@ -1539,7 +1495,7 @@ void direct_free(mvf_handle *h) {
   DirectPlan *P = (DirectPlan *)h->direct;
   if (!P) return;
   dfree(P->d_nodes); dfree(P->d_lev); dfree(P->d_idx); dfree(P->d_fpos); dfree(P->d_rel); dfree(P->d_dst);
-  dfree(P->d_piv); dfree(P->d_perm); dfree(P->d_pos); dfree(P->d_fac); dfree(P->d_inv); dfree(P->d_npert);
+  dfree(P->d_perm); dfree(P->d_pos); dfree(P->d_fac); dfree(P->d_inv); dfree(P->d_npert); dfree(P->d_blk);
   dfree(P->d_sv);
   dfree(P->d_zb);
   dfree(P->d_gin);
@@ -1613,7 +1569,6 @@ static int direct_plan(mvf_handle *h) {
   MVF_TRY(dalloc(h, &P->d_rel, P->nrel));
   MVF_TRY(dalloc(h, &P->d_dst, nnz));
   MVF_TRY(dalloc(h, &P->d_pos, nne));
-  MVF_TRY(dalloc(h, &P->d_piv, nne));
   MVF_TRY(dalloc(h, &P->d_perm, nne));
   MVF_TRY(dalloc(h, &P->d_npert, 1));
   MVF_TRY(dalloc(h, &P->d_fac, P->fac_entries));
@@ -1629,6 +1584,12 @@ static int direct_plan(mvf_handle *h) {
   MVF_HIP(h, hipMemcpy(P->d_rel, A.rel.data(), A.rel.size() * 4, hipMemcpyHostToDevice));
   MVF_HIP(h, hipMemcpy(P->d_dst, A.dst.data(), A.dst.size() * 4, hipMemcpyHostToDevice));
   MVF_HIP(h, hipMemcpy(P->d_pos, A.pos.data(), A.pos.size() * 4, hipMemcpyHostToDevice));
+  std::vector<int2> blk;
+  for (int t = 0; t < P->T; t++)
+    for (int64_t b = 0; b * kNB < P->nodes[t].n1; b++) blk.push_back(int2{t, (int)b});
+  P->nblk = (int64_t)blk.size();
+  MVF_TRY(dalloc(h, &P->d_blk, blk.size()));
+  MVF_HIP(h, hipMemcpy(P->d_blk, blk.data(), sizeof(int2) * blk.size(), hipMemcpyHostToDevice));
   P->t_symbolic = now_s() - t0;
   return 0;
 }
@@ -1650,8 +1611,8 @@ static void launch_gemm(bool big, unsigned gx, unsigned gy, hipStream_t st, cons
 
 // f32: emulated complex64 factorization.  Every front entry (top band in the
 // factor store, bottom band in the level pool) and the block inverses are
-// rounded to complex64 after the assembly, after each outer-block update, after
-// the Y solve and after the Schur update; the arithmetic between roundings is
+// rounded to complex64 after the assembly, after each outer-block update and
+// after the Schur update; the arithmetic between roundings is
 // FP64 and the lookahead is off, so the rounding points are ordered on one
 // stream.  A factorization in complex64 arithmetic rounds at least as often.
 static int direct_factor(mvf_handle *h, double w, int c64, int f32 = 0) {
@@ -1688,7 +1649,7 @@ static int direct_factor(mvf_handle *h, double w, int c64, int f32 = 0) {
     const int64_t mn1 = P->lev_maxn1[d], mn2 = P->lev_maxn2[d], mm = P->lev_maxm[d];
     hipLaunchKernelGGL(k_fa_zero, dim3(cap_grid((mm + 3) / 4), nl), dim3(256), 0, st, P->d_nodes, lev, P->d_fac, pool);
     hipLaunchKernelGGL(k_fa_assemble, dim3(cap_grid((mn1 + 3) / 4), nl), dim3(256), 0, st, P->d_nodes, lev, P->d_idx,
-                       h->d_rowptr, h->d_col, P->d_dst, h->d_K, h->d_M, w, c64, reg, P->d_fac, pool);
+                       h->d_rowptr, h->d_col, P->d_dst, h->d_K, h->d_M, w, c64, reg, P->d_fac);
     if (d < P->maxdepth) {
       int64_t cn2 = P->lev_maxn2[d + 1];
       for (int s = 0; s < 2; s++)
@@ -1710,8 +1671,6 @@ static int direct_factor(mvf_handle *h, double w, int c64, int f32 = 0) {
     const int64_t tile = big ? kBig : kTile;
     const int64_t tile_n = big ? kBigN : kTile;
     if (mn1 > 0) {
-      hipLaunchKernelGGL(k_fa_sym, dim3(cap_grid(((mn1 + 31) / 32) * ((mm + 31) / 32)), nl), dim3(256), 0, st,
-                         P->d_nodes, lev, P->d_fac, pool);
       // one GEMM launch over the level's fronts: grid from the largest operand, algorithmic flops summed
       auto gemm = [&](auto mode_tag, int64_t step, int64_t K0, hipStream_t s) {
         constexpr int MODE = decltype(mode_tag)::value;
@@ -1721,131 +1680,58 @@ static int direct_factor(mvf_handle *h, double w, int c64, int f32 = 0) {
           const GemmArgs g = gemm_args(MODE, P->nodes[t], step, K0);
           if (!g.ok) continue;
           const int64_t tm = (g.Mr + tile - 1) / tile, tn = (g.Nc + tile_n - 1) / tile_n;
-          // the large-front Schur update enumerates its lower tiles only
-          gt = std::max(gt, (MODE == 2 && big) ? (tm - 1) * tm + tn : tm * tn);
-          gfl += MODE == 2 ? 8.0 * (double)g.Mr * (double)(g.Mr + 1) / 2.0 * (double)g.Kd
-                           : 8.0 * (double)g.Mr * (double)g.Nc * (double)g.Kd;
+          gt = std::max(gt, big ? upper_tiles<2>(tm, tn) : upper_tiles<1>(tm, tn));
+          gfl += 8.0 * ((double)g.Mr * (double)g.Nc - (double)g.Mr * (double)(g.Mr - 1) / 2.0) * (double)g.Kd;
         }
         if (gt == 0) return;
         gemm_begin(gfl, MODE, s);
         launch_gemm<MODE>(big, cap_grid(gt), nl, s, P->d_nodes, lev, step, K0, P->d_fac, pool);
         gemm_end(s);
       };
-      auto urow = [&](int64_t k, int64_t K0, int part) {
-        int64_t gu = 0;
-        for (int t : P->levels[d]) {
-          const DNode &n = P->nodes[t];
-          if (k >= n.n1) continue;
-          int64_t c0, c1;
-          urow_cols(n, k, K0, part, c0, c1);
-          if (c1 > c0) gu = std::max(gu, (c1 - c0 + kTile - 1) / kTile);
-        }
-        if (gu > 0)
-          hipLaunchKernelGGL(k_fa_urow, dim3(cap_grid(gu), nl), dim3(256), 0, st, P->d_nodes, lev, k, K0, part,
-                             P->d_fac, P->d_inv);
-      };
       using M0 = std::integral_constant<int, 0>;
       using M1 = std::integral_constant<int, 1>;
       using M2 = std::integral_constant<int, 2>;
-      using M3 = std::integral_constant<int, 3>;
-      using M4 = std::integral_constant<int, 4>;
-      using M5 = std::integral_constant<int, 5>;
-      // LU of the top bands, two-level: panels of kNB inside outer blocks of kOuter.
-      // With more than one outer block, the trailing part of each outer update
-      // (rows and columns past the next outer block) runs on the side stream
+      // block rows of the top bands, two-level: panels of kNB inside outer blocks
+      // of kOuter.  With more than one outer block, the trailing part of each
+      // outer update (rows past the next outer block) runs on the side stream
       // while the next block's panels are factored on the handle's stream:
-      // pivoting is restricted to the panel's rows, so those panels touch
-      // neither the trailing part's rows nor its columns.  The next outer
-      // update waits for it.
+      // those write its block rows, and their transposes into its columns below
+      // the diagonal, and the trailing part lies right of its columns and
+      // reads the block before it.  The next outer update waits for it.
       const bool ahead = !f32 && mn1 > kOuter;
       bool pending = false;
       for (int64_t K0 = 0; K0 < mn1; K0 += kOuter) {
         const int64_t Kend = std::min(K0 + kOuter, mn1);
         for (int64_t k = K0; k < Kend; k += kNB) {
-          int64_t gc = 0, gr = 0;
+          int64_t gc = 0;  // widest block row right of the panel
           for (int t : P->levels[d]) {
             const DNode &n = P->nodes[t];
-            if (k >= n.n1) continue;
-            gc = std::max(gc, n.m);
-            gr = std::max(gr, n.n1 - std::min(k + kNB, n.n1));
+            if (k < n.n1) gc = std::max(gc, n.m - std::min(k + kNB, n.n1));
           }
           hipLaunchKernelGGL((k_fa_pdiag<kNB>), dim3(nl), dim3(256), 0, st, P->d_nodes, lev, k, P->d_fac, P->d_inv,
-                             P->d_piv, P->d_npert, big, tiny);
-          if (gr > 0)
-            hipLaunchKernelGGL((k_fa_prows<kNB>), dim3(cap_grid((gr + 63) / 64), nl), dim3(256), 0, st,
-                               P->d_nodes, lev, k, P->d_fac);
-          hipLaunchKernelGGL((k_fa_swap<kNB>), dim3(cap_grid((gc + 255) / 256), nl), dim3(256), 0, st, P->d_nodes,
-                             lev, k, P->d_fac, P->d_piv);
-          urow(k, K0, 0);
+                             P->d_perm, P->d_npert, big, tiny);
+          if (gc > 0)
+            hipLaunchKernelGGL((k_fa_prow<kNB>), dim3(cap_grid((gc + 63) / 64), nl), dim3(256), 0, st, P->d_nodes,
+                               lev, k, P->d_fac, pool, P->d_inv, P->d_perm);
           gemm(M0{}, k, K0, st);
-        }
-        // deferred part of the outer block's rows past it, then the rest of the front with K = kOuter
-        for (int64_t k = K0; k < Kend; k += kNB) {
-          urow(k, K0, 1);
-          gemm(M3{}, k, K0, st);
         }
         if (ahead) {
           if (pending) MVF_HIP(h, hipStreamWaitEvent(st, P->ev_join, 0));
           MVF_HIP(h, hipEventRecord(P->ev_fork, st));
           MVF_HIP(h, hipStreamWaitEvent(P->st2, P->ev_fork, 0));
-          gemm(M4{}, 3, K0, P->st2);
+          gemm(M1{}, 2, K0, P->st2);
           MVF_HIP(h, hipEventRecord(P->ev_join, P->st2));
           pending = true;
-          gemm(M4{}, 1, K0, st);
-          gemm(M4{}, 2, K0, st);
+          gemm(M1{}, 1, K0, st);
         } else {
-          gemm(M4{}, 0, K0, st);
+          gemm(M1{}, 0, K0, st);
         }
         round_level();
       }
       if (pending) MVF_HIP(h, hipStreamWaitEvent(st, P->ev_join, 0));
       if (mn2 > 0) {
-        // Y = U^-1 (L^-1 P F12), blocks from the bottom, outer groups of kGroup blocks
-        const int64_t nsteps = (mn1 + kNB - 1) / kNB;
-        // lookahead as in the LU: the outer Y update of the rows above the next
-        // group runs on the side stream while that group is solved
-        bool ypend = false;
-        for (int64_t s = 0; s < nsteps; s++) {
-          hipLaunchKernelGGL((k_fa_trsm_y<kNB>), dim3(cap_grid((mn2 + kTrsmThreads - 1) / kTrsmThreads), nl),
-                             dim3(kTrsmThreads), 0, st,
-                             P->d_nodes, lev, s, P->d_fac);
-          gemm(M1{}, s, 0, st);
-          if (ahead) {
-            // at a group boundary the side stream's pending update (rows above
-            // the previous group's next group) must end before this stream
-            // touches those rows again: part 1 here writes the next group,
-            // which the pending part 2 covered, and the top group has no part 2
-            // of its own to carry the wait
-            bool any1 = false, any2 = false;
-            for (int t : P->levels[d]) {
-              any1 = any1 || gemm_args(5, P->nodes[t], s, 1).ok;
-              any2 = any2 || gemm_args(5, P->nodes[t], s, 2).ok;
-            }
-            if ((any1 || any2) && ypend) {
-              MVF_HIP(h, hipStreamWaitEvent(st, P->ev_join, 0));
-              ypend = false;
-            }
-            if (any2) {
-              MVF_HIP(h, hipEventRecord(P->ev_fork, st));
-              MVF_HIP(h, hipStreamWaitEvent(P->st2, P->ev_fork, 0));
-              gemm(M5{}, s, 2, P->st2);
-              MVF_HIP(h, hipEventRecord(P->ev_join, P->st2));
-              ypend = true;
-            }
-            gemm(M5{}, s, 1, st);
-          } else {
-            gemm(M5{}, s, 0, st);
-          }
-        }
-        if (ypend) MVF_HIP(h, hipStreamWaitEvent(st, P->ev_join, 0));
-        round_level();
         gemm(M2{}, 0, 0, st);
         round_level();
-      }
-      {
-        const int64_t nbk = (mn1 + kNB - 1) / kNB;
-        hipLaunchKernelGGL(k_fa_perm, dim3((unsigned)((nbk + 63) / 64), nl), dim3(64), 0, st, P->d_nodes, lev, P->d_piv,
-                           P->d_perm);
       }
     }
     MVF_HIP(h, hipGetLastError());
@@ -1855,8 +1741,7 @@ static int direct_factor(mvf_handle *h, double w, int c64, int f32 = 0) {
       double lf = 0.0;
       for (int t : P->levels[d]) {
         const DNode &n = P->nodes[t];
-        const double a = (double)n.n1, b = (double)n.n2, mm2 = (double)n.m;
-        lf += 8.0 * (a * a * mm2 / 2.0 - a * a * a / 6.0 + a * a * b / 2.0 + a * b * b / 2.0);
+        lf += node_flops((double)n.n1, (double)n.n2);
       }
       const double tl = now_s() - t0;
       fprintf(stderr, "[direct] level %2d fronts %6d max n1 %6lld n2 %6lld  %.3e flop  t=%.3f s\n", d, nl,
@@ -1866,7 +1751,7 @@ static int direct_factor(mvf_handle *h, double w, int c64, int f32 = 0) {
   MVF_HIP(h, hipStreamSynchronize(st));
   gt_->destroy();
   if (h->verbose)
-    for (int q = 0; q < 6; q++)
+    for (int q = 0; q < 3; q++)
       if (gt_->mode_ms[q] > 0)
         fprintf(stderr, "[direct] GEMM mode %d: %.1f ms, %.3e flop, %.1f TFLOP/s\n", q, gt_->mode_ms[q],
                 gt_->mode_fl[q], gt_->mode_fl[q] / (gt_->mode_ms[q] * 1e-3) / 1e12);
@@ -1920,7 +1805,7 @@ static int direct_sweeps(mvf_handle *h, const double2 *in, double2 *out) {
   for (int d = P->maxdepth; d >= 0; d--) {
     const int nl = (int)P->levels[d].size();
     const int32_t *lev = P->d_lev + P->lev_off[d];
-    const int64_t mn1 = P->lev_maxn1[d], mn2 = P->lev_maxn2[d], mm = P->lev_maxm[d];
+    const int64_t mn1 = P->lev_maxn1[d], mm = P->lev_maxm[d];
     hipLaunchKernelGGL((k_sv_gather<NC>), dim3(cap_grid((mm * NC + 255) / 256), nl), dim3(256), 0, st, P->d_nodes, lev,
                        P->d_idx, in, W);
     if (d < P->maxdepth) {
@@ -1929,33 +1814,30 @@ static int direct_sweeps(mvf_handle *h, const double2 *in, double2 *out) {
         hipLaunchKernelGGL((k_sv_extend<NC>), dim3(cap_grid((cn2 * NC + 255) / 256), nl), dim3(256), 0, st,
                            P->d_nodes, lev, P->d_rel, s, W);
     }
-    if (mn1 == 0) continue;
-    if (mn2 > 0)
-      hipLaunchKernelGGL((k_sv_contrib<NC>), dim3(cap_grid((mn2 + 255) / 256), nl), dim3(256), 0, st, P->d_nodes, lev,
-                         P->d_fac, W);
-    hipLaunchKernelGGL((k_sv_perm<NC>), dim3(cap_grid((mn1 * NC + 255) / 256), nl), dim3(256), 0, st, P->d_nodes, lev,
-                       P->d_perm, W, zb);
-    const int64_t nb = (mn1 + kNB - 1) / kNB;
-    for (int64_t b = 0; b < nb; b++) {
-      hipLaunchKernelGGL((k_sv_ldiag<NC, kNB>), dim3(nl), dim3(256), 0, st, P->d_nodes, lev, b, P->d_inv, zb);
-      if ((b + 1) * kNB < mn1)
-        hipLaunchKernelGGL((k_sv_lupd<NC, kNB>), dim3(cap_grid((mn1 - (b + 1) * kNB + 15) / 16), nl), dim3(256), 0,
-                           st, P->d_nodes, lev, b, P->d_fac, zb);
-    }
-    for (int64_t s = 0; s < nb; s++) {
-      hipLaunchKernelGGL((k_sv_udiag<NC, kNB>), dim3(nl), dim3(64), 0, st, P->d_nodes, lev, s, P->d_fac, zb);
-      if (s + 1 < nb)
-        hipLaunchKernelGGL((k_sv_uupd<NC, kNB>), dim3(cap_grid((mn1 + 15) / 16), nl), dim3(256), 0, st, P->d_nodes,
-                           lev, s, P->d_fac, zb);
+    for (int64_t K0 = 0; K0 < mn1; K0 += kOuter) {
+      if (K0 + kNB < mn1)
+        hipLaunchKernelGGL((k_sv_fblock<NC>), dim3(nl), dim3(768), 0, st, P->d_nodes, lev, K0, P->d_fac, W);
+      hipLaunchKernelGGL((k_sv_frest<NC>), dim3(cap_grid((mm - K0 + 63) / 64), nl), dim3(256), 0, st, P->d_nodes,
+                         lev, K0, P->d_fac, W);
     }
   }
+  hipLaunchKernelGGL((k_sv_diag<NC, kNB>), dim3((unsigned)P->nblk), dim3(256), 0, st, P->d_nodes, P->d_blk, P->d_fac,
+                     P->d_inv, P->d_perm, W, zb);
   for (int d = 0; d <= P->maxdepth; d++) {
     const int nl = (int)P->levels[d].size();
     const int32_t *lev = P->d_lev + P->lev_off[d];
     const int64_t mn1 = P->lev_maxn1[d], mn2 = P->lev_maxn2[d];
-    if (mn1 == 0 || mn2 == 0) continue;
-    hipLaunchKernelGGL((k_sv_back<NC>), dim3(cap_grid((mn1 + 3) / 4), nl), dim3(256), 0, st, P->d_nodes, lev,
-                       P->d_fpos, P->d_fac, zb);
+    if (mn1 == 0) continue;
+    if (mn2 > 0)
+      hipLaunchKernelGGL((k_sv_back<NC>), dim3(cap_grid((mn1 + 3) / 4), nl), dim3(256), 0, st, P->d_nodes, lev,
+                         P->d_fpos, P->d_fac, zb);
+    for (int64_t K0 = (mn1 - 1) / kOuter * kOuter; K0 >= 0; K0 -= kOuter) {
+      if (K0 + kOuter < mn1)
+        hipLaunchKernelGGL((k_sv_brest<NC>), dim3((unsigned)kOuter, nl), dim3(256), 0, st, P->d_nodes, lev, K0,
+                           P->d_fac, zb);
+      if (K0 + kNB < mn1)
+        hipLaunchKernelGGL((k_sv_bblock<NC>), dim3(nl), dim3(1024), 0, st, P->d_nodes, lev, K0, P->d_fac, zb);
+    }
   }
   hipLaunchKernelGGL((k_sv_out<NC>), dim3(cap_grid((P->nne * NC + 255) / 256)), dim3(256), 0, st, P->nne, P->d_pos, zb,
                      out);

@@ -138,3 +138,32 @@ def test_direct_lookahead_fronts(need_gpu):
         for d in range(2):
             r = np.linalg.norm(b[d] - A @ x[d]) / np.linalg.norm(b[d])
             assert r <= 1e-8 * 1.0001, (f, d, r)
+
+
+@pytest.mark.parametrize("nodes,sides", [
+    (8, (5, 3, 2)),    # a root of one partial panel with nothing right of it
+    (8, (9, 7, 6)),    # last panels of every width the small fronts have
+    (20, (5, 5, 3)),
+    (20, (9, 3, 3)),   # narrow separators: fronts with one partial panel
+    (27, (4, 3, 5)),
+])
+@pytest.mark.parametrize("tile", [0, 128])
+def test_direct_block_rows(nodes, sides, tile, need_gpu):
+    """Symmetric block factorization on fronts with partial panels, partial
+    column tiles and no update columns.  With every pivot block nonsingular the
+    factor is that of the matrix itself up to the air shift, so GMRES needs at
+    most four iterations, and the solution is SuperLU's to 1e-6 where it is
+    determined (a residual of 1e-10 at condition numbers below 1e4)."""
+    m = M.random_small(nodes, *sides, seed=31, nz_air=1, full_tensor=True, freqs=(10.0,))
+    g = GpuVfem(m)
+    g.set_frequency(0)
+    A, b = reference_system(g)
+    lu = spla.splu(A)
+    x, info = g.solve(b.ravel(), method="gmres", precond="direct", tol=1e-10, direct_tile=tile)
+    x = x.reshape(2, -1)
+    print(f"block rows {nodes} {sides}: nne={g.nne} its={info['iterations']}", flush=True)
+    assert info["converged"] and info["iterations"] <= 4, info
+    mask = determined_dofs(m, g.gne())
+    for d in range(2):
+        xr = lu.solve(b[d])
+        assert np.linalg.norm(x[d][mask] - xr[mask]) <= 1e-6 * np.linalg.norm(xr[mask])
