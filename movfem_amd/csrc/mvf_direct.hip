@@ -58,6 +58,8 @@ namespace mvf {
 
 constexpr int kLeafMax = 16;       // elements per leaf box
 constexpr int kNB = 64;            // panel width / triangular block size
+constexpr int kSub = 16;           // columns per sub-panel of a diagonal block
+constexpr int kInvBlk = kNB / kSub * kSub * kSub;
 constexpr double kRegEps = 1e-4;   // air regularization relative to the smallest omega*M/K
 constexpr int kTile = 64;          // GEMM tile edge
 
@@ -69,7 +71,7 @@ struct DNode {
   int64_t rel;   // offset of the parent-relative map of the update DOFs (n2 entries)
   int64_t pos0;  // elimination position of the first owned DOF (also permutation offset)
   int64_t sv;    // offset (rows) of the node's solve work vector (m rows)
-  int64_t inv;   // offset of the inverses of the unit-lower diagonal blocks of L (w^2 per panel block)
+  int64_t inv;   // offset of the inverses of L's 16 x 16 diagonal blocks (kInvBlk entries per panel block)
   int32_t child[2];
   int32_t parent;
   int32_t depth;
@@ -335,12 +337,8 @@ static int build_plan_host(DirectPlan &P, int nx, int ny, int nz, int me, const 
     n.pos0 = optr[t];
     n.sv = svoff;
     svoff += n.m;
-    {
-      // panel blocks of width kNB, the last one n1 - kNB*(nb-1) wide
-      const int64_t nbk = (n.n1 + kNB - 1) / kNB, wl = n.n1 - kNB * (nbk - 1);
-      n.inv = invoff;
-      invoff += nbk > 0 ? kNB * kNB * (nbk - 1) + wl * wl : 0;
-    }
+    n.inv = invoff;
+    invoff += (n.n1 + kNB - 1) / kNB * kInvBlk;
     n.child[0] = tb.child[t][0];
     n.child[1] = tb.child[t][1];
     n.parent = tb.parent[t];
@@ -573,150 +571,176 @@ __global__ __launch_bounds__(256) void k_fa_extend(const DNode *nodes, const int
   }
 }
 
-// LU of the panel's diagonal block T[k:kend, k:kend] in LDS, read from its
-// upper triangle, pivot search restricted to the block's rows (kend - k <= NB);
-// one workgroup per front.  perm[pos0 + k + q] is the front row that ends in
-// row k + q.
-// A pivot below `tiny` (a singular block) is replaced by `big` and counted.
+// largest key over the wave (row shifts, then row broadcasts; lane 63 ends with
+// the maximum), the same in every lane
+__device__ __forceinline__ int wave_max(int k) {
+  k = max(k, __builtin_amdgcn_update_dpp(k, k, 0x111, 0xf, 0xf, false));
+  k = max(k, __builtin_amdgcn_update_dpp(k, k, 0x112, 0xf, 0xf, false));
+  k = max(k, __builtin_amdgcn_update_dpp(k, k, 0x114, 0xf, 0xf, false));
+  k = max(k, __builtin_amdgcn_update_dpp(k, k, 0x118, 0xf, 0xf, false));
+  k = max(k, __builtin_amdgcn_update_dpp(k, k, 0x142, 0xa, 0xf, false));
+  k = max(k, __builtin_amdgcn_update_dpp(k, k, 0x143, 0xc, 0xf, false));
+  return __builtin_amdgcn_readlane(k, 63);
+}
+// LDS written by some lanes of a wave and read by others of the same wave
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// LU of the panel's diagonal block T[k:kend, k:kend], read from its upper
+// triangle, pivot search restricted to the block's rows (kend - k <= NB); one
+// workgroup per front.  perm[pos0 + k + q] is the front row that ends in row
+// k + q; inv receives the inverses of L's 16 x 16 diagonal blocks (its
+// multipliers are bounded by 1, so they are safe to form).  A pivot below `tiny`
+// (a singular block) is replaced by `big` and counted.
+//
+// Bound by the chain of 64 pivot steps, so each step is kept inside one wave.
+// The block is cut into four sub-panels of 16 columns, wave b owning the
+// columns of sub-panel b.  A sub-panel is eliminated in registers with one row
+// per lane and rows left where they are (a chosen row only drops out of the
+// search): the search is one integer maximum over the wave on the leading bits
+// of |a|^2 (14 of the mantissa, the lane below them, so equal magnitudes take
+// the lowest row), the pivot row is broadcast by lane reads.  After the one
+// barrier per sub-panel each later wave applies L^-1 to the sub-panel's rows of
+// its columns and updates the rest on the matrix cores, then the next wave goes
+// straight on to its own sub-panel.
+// One launch on few fronts: 126 -> 39 us against 64 steps of two workgroup
+// barriers each over LDS; at the 66 KB of one block two fronts share a CU
+// (20-node 33 x 33 x 25, two frequencies: 66.0 -> 20.9 ms).
 template <int NB>
 __global__ __launch_bounds__(256) void k_fa_pdiag(const DNode *nodes, const int32_t *lev, int64_t k, double2 *fac,
                                                   double2 *inv, int32_t *perm, int *npert, double big, double tiny) {
-  // Four waves: lane t of every wave stands for row t, wave g for the columns
-  // c = g (mod 4) of the rank-1 updates and of the inverse's updates.  The
-  // pivot search, interchange and multipliers run on wave 0: two barriers per
-  // column.
-  static_assert(NB == 64, "one lane per row of the diagonal block");
+  static_assert(NB == 64 && kSub == 16, "one lane per row, one wave per sub-panel");
   const DNode nd = nodes[lev[blockIdx.x]];
   if (k >= nd.n1) return;
   const int64_t m = nd.m, kend = (k + NB < nd.n1) ? k + NB : nd.n1;
-  const int w = (int)(kend - k);
+  const int w = (int)(kend - k), nsub = (w + kSub - 1) / kSub;
   double2 *T = fac + nd.fac;
+  double2 *Li = inv + nd.inv + (int64_t)kInvBlk * (k / NB);
   __shared__ double2 a[NB][NB + 1];
-  __shared__ double2 x[NB][NB + 1];
-  const int tid = threadIdx.x, t = tid & 63, g = tid >> 6;
-  // wave g reads rows g, g + 4, ...; lane t column t (coalesced, clamped
-  // addresses, padding selected afterwards)
+  __shared__ int phys[NB];                  // phys[q]: row of `a` holding row q of the factor
+  __shared__ unsigned long long gone[4];    // rows taken as pivots up to each sub-panel
+  const int tid = threadIdx.x, t = tid & 63, g = __builtin_amdgcn_readfirstlane(tid >> 6), li = t & 15, lk = t >> 4;
   {
     const int tc = t < w ? t : w - 1;
 #pragma unroll
     for (int j = 0; j < NB / 4; j++) {
-      const int r = g + 4 * j;
-      const int rc = r < w ? r : w - 1;
+      const int r = g + 4 * j, rc = r < w ? r : w - 1;
       const double2 v = T[(k + (rc < tc ? rc : tc)) * m + k + (rc < tc ? tc : rc)];
       a[r][t] = (r < w && t < w) ? v : make_double2(0.0, 0.0);
     }
+    if (g == 0) phys[t] = t;
   }
-  int32_t prow = (int32_t)(k + t);  // wave 0: front row now in row t
   __syncthreads();
-  for (int q = 0; q < w; q++) {
-    // wave 0 alone: pivot search, row interchange, perturbation and the
-    // multipliers of column q (one wave's LDS operations complete in order,
-    // so no barrier is needed between these steps)
-    if (g == 0) {
-      // pivot: largest |a[r][q]|, r in [q, w); ties to the lower row
-      double v = -1.0;
-      int ri = q;
-      if (t >= q && t < w) {
-        v = a[t][q].x * a[t][q].x + a[t][q].y * a[t][q].y;
-        ri = t;
+  // val (a 16 x 16 block, lane: rows lk + 4 v of column li) = L_bb^-1 val
+  auto lsolve = [&](int c0, const int *pr, double2 *val) {
+#pragma unroll
+    for (int j = 0; j < kSub - 1; j++) {
+      const int o = li + 16 * (j & 3);
+      const double2 s = make_double2(__shfl(val[j >> 2].x, o, 64), __shfl(val[j >> 2].y, o, 64));
+#pragma unroll
+      for (int v = j >> 2; v < 4; v++) {
+        double2 e = a[pr[v]][c0 + j];
+        if (v == (j >> 2) && lk <= (j & 3)) e = make_double2(0.0, 0.0);
+        cfms(val[v], e, s);
       }
-      for (int off = 32; off > 0; off >>= 1) {
-        const double ov = __shfl_xor(v, off, 64);
-        const int oi = __shfl_xor(ri, off, 64);
-        if (ov > v || (ov == v && oi < ri)) {
-          v = ov;
-          ri = oi;
+    }
+  };
+  for (int b = 0; b < nsub; b++) {
+    const int c0 = kSub * b;
+    if (g == b) {
+      double2 x[kSub];
+#pragma unroll
+      for (int c = 0; c < kSub; c++) x[c] = a[t][c0 + c];
+      bool done = t >= w || (b > 0 && (gone[b > 0 ? b - 1 : 0] >> t & 1));
+#pragma unroll
+      for (int q = 0; q < kSub; q++) {
+        if (c0 + q >= w) break;  // uniform
+        const double d2 = x[q].x * x[q].x + x[q].y * x[q].y;
+        const int hi = (int)((unsigned long long)__double_as_longlong(d2) >> 32);
+        const int p = 63 - (wave_max(done ? -1 : ((hi & 0x7fffffc0) | (63 - t))) & 63);
+        double2 pv = make_double2(lane_bcast(x[q].x, p), lane_bcast(x[q].y, p));
+        if (!(pv.x * pv.x + pv.y * pv.y > tiny * tiny)) {
+          pv = make_double2(big, 0.0);
+          if (t == p) x[q] = pv;
+          if (t == 0) atomicAdd(npert, 1);
+        }
+        const double rd = 1.0 / (pv.x * pv.x + pv.y * pv.y);
+        done = done || t == p;
+        if (t == 0) phys[c0 + q] = p;
+        const double2 l = done ? make_double2(0.0, 0.0) : cmul(x[q], make_double2(pv.x * rd, -pv.y * rd));
+        if (!done) x[q] = l;
+#pragma unroll
+        for (int c = q + 1; c < kSub; c++) cfms(x[c], l, make_double2(lane_bcast(x[c].x, p), lane_bcast(x[c].y, p)));
+      }
+#pragma unroll
+      for (int c = 0; c < kSub; c++) a[t][c0 + c] = x[c];
+      const unsigned long long dm = __ballot(done);
+      if (t == 0) gone[b] = dm;
+    }
+    __syncthreads();
+    int pr[4];
+#pragma unroll
+    for (int v = 0; v < 4; v++) pr[v] = phys[c0 + lk + 4 * v];
+    double2 u[4];
+    if (g == b) {
+#pragma unroll
+      for (int v = 0; v < 4; v++) u[v] = make_double2(lk + 4 * v == li ? 1.0 : 0.0, 0.0);
+      lsolve(c0, pr, u);
+#pragma unroll
+      for (int v = 0; v < 4; v++) Li[b * 256 + (lk + 4 * v) * 16 + li] = u[v];
+    } else if (g > b && g < nsub) {
+      const int cc = kSub * g + li;
+      const unsigned long long dm = gone[b];
+#pragma unroll
+      for (int v = 0; v < 4; v++) u[v] = a[pr[v]][cc];
+      lsolve(c0, pr, u);
+#pragma unroll
+      for (int v = 0; v < 4; v++) a[pr[v]][cc] = u[v];
+      // rows not yet taken: a -= L U, rows taken masked out of L and of the store
+#pragma unroll
+      for (int rb = 0; rb < 4; rb++) {
+        mvf_d4 cr, ci;
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+          const double2 e = a[16 * rb + lk + 4 * v][cc];
+          cr[v] = e.x;
+          ci[v] = e.y;
+        }
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          const double2 e = a[16 * rb + li][c0 + 4 * q + lk];
+          cr = __builtin_amdgcn_mfma_f64_16x16x4f64(-e.x, u[q].x, cr, 0, 0, 0);
+          ci = __builtin_amdgcn_mfma_f64_16x16x4f64(-e.x, u[q].y, ci, 0, 0, 0);
+          cr = __builtin_amdgcn_mfma_f64_16x16x4f64(e.y, u[q].y, cr, 0, 0, 0);
+          ci = __builtin_amdgcn_mfma_f64_16x16x4f64(-e.y, u[q].x, ci, 0, 0, 0);
+        }
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+          const int r = 16 * rb + lk + 4 * v;
+          if (!(dm >> r & 1)) a[r][cc] = make_double2(cr[v], ci[v]);
         }
       }
-      const int32_t pq = __shfl(prow, q, 64), pr = __shfl(prow, ri, 64);
-      if (t == q) prow = pr;
-      if (t == ri) prow = pq;
-      if (ri != q && t < w) {
-        const double2 e = a[q][t];
-        a[q][t] = a[ri][t];
-        a[ri][t] = e;
-      }
-      if (t == 0 && !(v > tiny * tiny)) {
-        a[q][q] = make_double2(big, 0.0);
-        atomicAdd(npert, 1);
-      }
-      if (t > q && t < w) a[t][q] = cmul(a[t][q], cinv(a[q][q]));
+      wave_lds_fence();
     }
-    __syncthreads();
-    if (t > q && t < w) {
-      const double2 l = a[t][q];
-      // row t -= l * row q over this wave's columns, four per batch
-      for (int c0 = q + 1 + g; c0 < w; c0 += 16) {
-        double2 xr[4], yr[4];
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-          if (c0 + 4 * j < w) {
-            xr[j] = a[t][c0 + 4 * j];
-            yr[j] = a[q][c0 + 4 * j];
-          }
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-          if (c0 + 4 * j < w) {
-            cfms(xr[j], l, yr[j]);
-            a[t][c0 + 4 * j] = xr[j];
-          }
-      }
-    }
-    __syncthreads();
-  }
-#pragma unroll
-  for (int j = 0; j < NB / 4; j++) {
-    const int r = g + 4 * j;
-    if (r < w && t < w) T[(k + r) * m + k + t] = a[r][t];
-  }
-  if (g == 0 && t < w) perm[nd.pos0 + k + t] = prow;
-  // inverse X of the unit lower L_kk.  L's multipliers are bounded by 1, so
-  // the explicit inverse is safe; U_kk can hold pivots ~1e-11 of the largest
-  // (the air shift) and is only ever used by substitution.  Column form:
-  // X = I, then for p = 0, 1, ...: X[r][c] -= L[r][p] X[p][c] for r > p and
-  // c <= p (row p of X is final once the steps before p are done); lane t
-  // updates row t, wave g the columns c = g (mod 4).
-#pragma unroll
-  for (int j = 0; j < NB / 4; j++) {
-    const int c = g + 4 * j;
-    x[t][c] = make_double2(t == c ? 1.0 : 0.0, 0.0);
   }
   __syncthreads();
-  for (int p = 0; p + 1 < w; p++) {
-    if (t > p && t < w) {
-      const double2 lp = a[t][p];
-      for (int c0 = g; c0 <= p; c0 += 16) {
-        double2 xr[4], yr[4];
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-          if (c0 + 4 * j <= p) {
-            xr[j] = x[t][c0 + 4 * j];
-            yr[j] = x[p][c0 + 4 * j];
-          }
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-          if (c0 + 4 * j <= p) {
-            cfms(xr[j], lp, yr[j]);
-            x[t][c0 + 4 * j] = xr[j];
-          }
-      }
-    }
-    __syncthreads();
-  }
-  double2 *Li = inv + nd.inv + (int64_t)NB * NB * (k / NB);
 #pragma unroll
   for (int j = 0; j < NB / 4; j++) {
     const int r = g + 4 * j;
-    if (r < w && t < w) Li[r * w + t] = x[r][t];
+    if (r < w && t < w) T[(k + r) * m + k + t] = a[phys[r]][t];
   }
+  if (g == 0 && t < w) perm[nd.pos0 + k + t] = (int32_t)(k + phys[t]);
 }
 
 // Block row of panel k: V = A_kk^-1 T[k:kend, kend:m] in place, and the
 // transpose of the block row as it was into the lower part (T for the owned
 // columns, F21 for the others), where the updates read it as their left operand.
 // Each wave owns 16 columns and works alone: the block row in registers as
-// MFMA operands (lane l, register v: row 4 v + l / 16, column l % 16), L^-1 by
-// products with the block inverse, U by substitution over 16-row blocks.  The
+// MFMA operands (lane l, register v: row 4 v + l / 16, column l % 16), L^-1
+// by products with the inverses of its 16 x 16 diagonal blocks, U by
+// substitution over 16-row blocks.  The
 // MFMA result layout (row l / 16 + 4 v of its 16-row block) is the operand
 // layout of the next product, so nothing is staged; inside a diagonal block the
 // sixteen steps pass the solved row from its sixteen lanes to the others.
@@ -767,23 +791,40 @@ __global__ __launch_bounds__(256) void k_fa_prow(const DNode *nodes, const int32
     const double2 t = T[sp[4 * v + lk] * m + jc];
     x[v] = 4 * v + lk < w ? t : make_double2(0.0, 0.0);
   }
-  // Z = L^-1 P R
-  const double2 *Li = inv + nd.inv + (int64_t)NB * NB * (k / NB);
+  // Z = L^-1 P R, 16-row blocks from the first: Z_b = L_bb^-1 (PR_b - sum_j L_bj Z_j)
+  const double2 *Li = inv + nd.inv + (int64_t)kInvBlk * (k / NB);
   mvf_d4 zr[4], zi[4];
 #pragma unroll
   for (int b = 0; b < 4; b++) {
-    zr[b] = zi[b] = mvf_d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      zr[b][v] = x[4 * b + v].x;
+      zi[b][v] = x[4 * b + v].y;
+    }
+    if (16 * b >= w) continue;  // rows past the panel stay zero
     const int row = 16 * b + li;
 #pragma unroll
-    for (int q = 0; q < 4 * (b + 1); q++) {
-      const int col = 4 * q + lk;
-      const double2 t = Li[(row < w ? row : w - 1) * w + (col < w ? col : w - 1)];
-      const double2 a = (row < w && col < w) ? t : make_double2(0.0, 0.0);
-      zr[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, x[q].x, zr[b], 0, 0, 0);
-      zi[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, x[q].y, zi[b], 0, 0, 0);
-      zr[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(-a.y, x[q].y, zr[b], 0, 0, 0);
-      zi[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, x[q].x, zi[b], 0, 0, 0);
+    for (int jb = 0; jb < b; jb++)
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const double2 t = T[(k + (row < w ? row : w - 1)) * m + k + 16 * jb + 4 * q + lk];
+        const double2 a = row < w ? t : make_double2(0.0, 0.0);
+        zr[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(-a.x, zr[jb][q], zr[b], 0, 0, 0);
+        zi[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(-a.x, zi[jb][q], zi[b], 0, 0, 0);
+        zr[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, zi[jb][q], zr[b], 0, 0, 0);
+        zi[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(-a.y, zr[jb][q], zi[b], 0, 0, 0);
+      }
+    mvf_d4 yr = {0.0, 0.0, 0.0, 0.0}, yi = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const double2 a = Li[b * 256 + li * 16 + 4 * q + lk];
+      yr = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, zr[b][q], yr, 0, 0, 0);
+      yi = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, zi[b][q], yi, 0, 0, 0);
+      yr = __builtin_amdgcn_mfma_f64_16x16x4f64(-a.y, zi[b][q], yr, 0, 0, 0);
+      yi = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, zr[b][q], yi, 0, 0, 0);
     }
+    zr[b] = yr;
+    zi[b] = yi;
   }
   // V = U^-1 Z, 16-row blocks from the last
 #pragma unroll
@@ -1284,76 +1325,54 @@ __global__ __launch_bounds__(256) void k_sv_frest(const DNode *nodes, const int3
 }
 
 // y = A_kk^-1 b for every panel block of the tree at once, one workgroup per
-// block: L through its stored inverse (four lanes per row), then U by
-// substitution on one wave, lane r holding row r of the strict upper block
-// column-major in LDS, the solved value broadcast by scalar lane reads.
+// block: L and then U by substitution, lane r of a wave holding row r, the
+// block column-major in LDS, the solved value broadcast by scalar lane reads;
+// the right-hand sides are dealt to the four waves.
 template <int NC, int NB>
 __global__ __launch_bounds__(256) void k_sv_diag(const DNode *nodes, const int2 *blk, const double2 *fac,
-                                                 const double2 *inv, const int32_t *perm, const double2 *W,
-                                                 double2 *zb) {
+                                                 const int32_t *perm, const double2 *W, double2 *zb) {
   static_assert(NB == 64, "one lane per row of the diagonal block");
   const int2 nb = blk[blockIdx.x];
   const DNode nd = nodes[nb.x];
   const int64_t r0 = (int64_t)nb.y * NB, r1 = r0 + NB < nd.n1 ? r0 + NB : nd.n1;
   const int w = (int)(r1 - r0);
   const double2 *T = fac + nd.fac;
-  const double2 *Ai = inv + nd.inv + (int64_t)NB * NB * nb.y;
-  __shared__ double2 S[NB][NB + 1];  // S[col][row] = U[row][col], row < col; padded for conflict-free writes
-  __shared__ double2 z[NB][NC], y[NB][NC];
-  const int tid = threadIdx.x;
-  for (int e = tid; e < NB * NC; e += 256) {
-    const int r = e / NC, c = e % NC;
-    z[r][c] = r < w ? W[(nd.sv + perm[nd.pos0 + r0 + r]) * NC + c] : make_double2(0.0, 0.0);
+  __shared__ double2 S[NB][NB + 1];  // S[col][row]: L below the diagonal, U above; padded for conflict-free writes
+  const int r = threadIdx.x & 63, g = threadIdx.x >> 6, rc = r < w ? r : w - 1;
+#pragma unroll
+  for (int j = 0; j < NB / 4; j++) {
+    const int q = g + 4 * j;  // lane r reads column r of row q
+    const double2 u = T[(r0 + (q < w ? q : w - 1)) * nd.m + r0 + rc];
+    S[r][q] = (q < w && r < w) ? u : make_double2(0.0, 0.0);
   }
-#pragma unroll 16
-  for (int q = tid >> 6; q < NB; q += 4) {
-    const int r = tid & 63;  // column r of row q
-    const double2 u = T[(r0 + (q < w ? q : w - 1)) * nd.m + r0 + (r < w ? r : w - 1)];
-    S[r][q] = (q < w && r < w && r > q) ? u : make_double2(0.0, 0.0);
-  }
-  __syncthreads();
-  {
-    const int r = tid >> 2, l4 = tid & 3, rc = r < w ? r : w - 1;
-    double2 acc[NC];
+  constexpr int NW = (NC + 3) / 4;  // columns per wave: g, g + 4, ...
+  double2 z[NW];
 #pragma unroll
-    for (int c = 0; c < NC; c++) acc[c] = make_double2(0.0, 0.0);
-#pragma unroll 8
-    for (int q = l4; q < NB; q += 4) {
-      const double2 a = Ai[rc * w + (q < w ? q : w - 1)];
-      if (q < w)
-#pragma unroll
-        for (int c = 0; c < NC; c++) cfma(acc[c], a, z[q][c]);
-    }
-#pragma unroll
-    for (int c = 0; c < NC; c++)
-#pragma unroll
-      for (int off = 1; off < 4; off <<= 1) {
-        acc[c].x += __shfl_xor(acc[c].x, off, 4);
-        acc[c].y += __shfl_xor(acc[c].y, off, 4);
-      }
-    if (l4 == 0)
-#pragma unroll
-      for (int c = 0; c < NC; c++) y[r][c] = acc[c];
+  for (int i = 0; i < NW; i++) {
+    const int c = g + 4 * i;
+    z[i] = (r < w && c < NC) ? W[(nd.sv + perm[nd.pos0 + r0 + rc]) * NC + c] : make_double2(0.0, 0.0);
   }
   __syncthreads();
-  if (tid >= 64) return;
-  const int r = tid;
-  const double2 dinv = r < w ? cinv(T[(r0 + r) * nd.m + r0 + r]) : make_double2(0.0, 0.0);
-  double2 zc[NC];
+  if (g >= NC) return;
+#pragma unroll 4
+  for (int q = 0; q + 1 < w; q++) {
+    const double2 l = r > q ? S[q][r] : make_double2(0.0, 0.0);
 #pragma unroll
-  for (int c = 0; c < NC; c++) zc[c] = y[r][c];
+    for (int i = 0; i < NW; i++) cfms(z[i], l, make_double2(lane_bcast(z[i].x, q), lane_bcast(z[i].y, q)));
+  }
+  const double2 dinv = r < w ? cinv(S[r][r]) : make_double2(0.0, 0.0);
+#pragma unroll 4
   for (int q = w - 1; q >= 0; q--) {
-    const double2 u = S[q][r];
+    const double2 u = r < q ? S[q][r] : make_double2(0.0, 0.0);
 #pragma unroll
-    for (int c = 0; c < NC; c++) {
-      if (r == q) zc[c] = cmul(zc[c], dinv);
-      const double2 zq = make_double2(lane_bcast(zc[c].x, q), lane_bcast(zc[c].y, q));
-      if (r < q) cfms(zc[c], u, zq);
+    for (int i = 0; i < NW; i++) {
+      if (r == q) z[i] = cmul(z[i], dinv);
+      cfms(z[i], u, make_double2(lane_bcast(z[i].x, q), lane_bcast(z[i].y, q)));
     }
   }
-  if (r < w)
 #pragma unroll
-    for (int c = 0; c < NC; c++) zb[(nd.pos0 + r0 + r) * NC + c] = zc[c];
+  for (int i = 0; i < NW; i++)
+    if (r < w && g + 4 * i < NC) zb[(nd.pos0 + r0 + r) * NC + g + 4 * i] = z[i];
 }
 
 // backward, update columns: z[i] -= sum_j V[i][n1 + j] x2[j]; one wave per row
@@ -1822,7 +1841,7 @@ static int direct_sweeps(mvf_handle *h, const double2 *in, double2 *out) {
     }
   }
   hipLaunchKernelGGL((k_sv_diag<NC, kNB>), dim3((unsigned)P->nblk), dim3(256), 0, st, P->d_nodes, P->d_blk, P->d_fac,
-                     P->d_inv, P->d_perm, W, zb);
+                     P->d_perm, W, zb);
   for (int d = 0; d <= P->maxdepth; d++) {
     const int nl = (int)P->levels[d].size();
     const int32_t *lev = P->d_lev + P->lev_off[d];
