@@ -16,8 +16,9 @@
 //            padding): Y[v][n] = sum_tap sum_k X[v+off(tap)][k] W[tap][n][k];
 //            the data gradient is the same product with the weights flipped
 //            and transposed (Wt[tap'][ci][co] = W[26-tap'][co][ci]).
-//   k_wgrad  weight gradient dW[tap][co][ci] = sum_v dY[v][co] X[v+off][ci],
-//            the voxel sum split over workgroups and added with FP32 atomics.
+//   k_wgrad  weight gradient dW[tap][co][ci] = sum_v dY[v][co] X[v+off][ci]
+//            and the bias gradient, the voxel sum split over workgroups whose
+//            partial sums k_wred adds in order.
 //   element-wise kernels: input packing, 2x2x2 average pooling and nearest
 //   upsampling with their adjoints, the masked MSE loss and Adam.
 #include <cstring>
@@ -75,21 +76,29 @@ __device__ inline s4v load4(const bf16 *p) { return *(const s4v *)p; }
 enum { EPI_ACT = 0, EPI_F32 = 1, EPI_MASK = 2, EPI_RAW = 3 };
 
 // Y = conv(X, W) over K = taps * cin; each wave computes 32 voxels (two row
-// tiles) x NT*16 output channels, four waves per workgroup.
+// tiles) x NT*16 output channels of channel group blockIdx.y, four waves per
+// workgroup.  SPLIT: the four waves share one set of 32 voxels and take every
+// fourth group of taps, their accumulators added in wave order at the end: the
+// coarse levels have too few voxels to fill the chip and would walk all taps in
+// one chain per wave.
 //   EPI_ACT:  Y bf16 = leaky(acc + bias)
 //   EPI_F32:  Y fp32 = acc + bias
 //   EPI_MASK: Y bf16 = acc * leaky'(mask tensor)   (data gradient inside a level)
 //   EPI_RAW:  Y bf16 = acc                          (data gradient at a level boundary)
 // X: channel stride cx (input may be a slice of a wider tensor); Y: channel
-// stride cy; mask: channel stride cm.
-template <int KS, int NT, int EPI>
-__global__ __launch_bounds__(256) void k_conv(Dims d, const bf16 *__restrict__ X, int cx, int cin,
+// stride cy; mask: channel stride cm.  The operands come straight from L2, so
+// the KS taps along z of one (dx, dy, 16 channels) are loaded together, and
+// those of the next group before the current group's products (64 x 64 x 48 x 2,
+// forward: 16 -> 16 channels 89 -> 67 us, a level of 6144 voxels 102 -> 24 us).
+template <int KS, int NT, int EPI, bool SPLIT>
+__global__ __launch_bounds__(256) void k_conv(Dims d, const bf16 *__restrict__ X, int cx, int cin, int cout,
                                               const bf16 *__restrict__ W, const float *__restrict__ bias, void *Yv,
                                               int cy, const bf16 *__restrict__ mask, int cm, float alpha) {
-  constexpr int NTAP = KS * KS * KS, R = KS / 2;
+  constexpr int R = KS / 2;
   const int wv = threadIdx.x >> 6, l = threadIdx.x & 63, q = l >> 4, r = l & 15;
   const int64_t V = d.vox();
-  const int64_t v0 = ((int64_t)blockIdx.x * 4 + wv) * 32;  // first voxel of the wave
+  const int64_t v0 = (SPLIT ? (int64_t)blockIdx.x : (int64_t)blockIdx.x * 4 + wv) * 32;  // first voxel of the wave
+  const int n0 = blockIdx.y * NT * 16;                                                    // first output channel
   f4v acc[2][NT];
 #pragma unroll
   for (int mt = 0; mt < 2; mt++)
@@ -104,34 +113,67 @@ __global__ __launch_bounds__(256) void k_conv(Dims d, const bf16 *__restrict__ X
     vsplit(d, rv[mt] ? v : 0, bb[mt], xx[mt], yy[mt], zz[mt]);
   }
   const s4v zero4 = s4v{0, 0, 0, 0};
-#pragma unroll 1
-  for (int tap = 0; tap < NTAP; tap++) {
-    const int dx = tap / (KS * KS) - R, dy = (tap / KS) % KS - R, dz = tap % KS - R;
-    const bf16 *xp[2];
-    bool ok[2];
+  s4v a[KS][2], b[KS][NT];
+  // group g = ((dx, dy), 16 input channels): its KS taps along z
+  const int nc = cin / 16, ng = KS * KS * nc;
+  auto load = [&](int g) {
+    const int xy = g / nc, c0 = (g - xy * nc) * 16;
+    const int dx = xy / KS - R, dy = xy % KS - R;
 #pragma unroll
     for (int mt = 0; mt < 2; mt++) {
-      const int x = xx[mt] + dx, y = yy[mt] + dy, z = zz[mt] + dz;
-      ok[mt] = rv[mt] && x >= 0 && x < d.nx && y >= 0 && y < d.ny && z >= 0 && z < d.nz;
-      xp[mt] = X + (ok[mt] ? vjoin(d, bb[mt], x, y, z) : 0) * cx + 4 * q;
-    }
-    const bf16 *wp = W + ((int64_t)tap * NT * 16 + r) * cin + 4 * q;
-#pragma unroll 1
-    for (int c0 = 0; c0 < cin; c0 += 16) {
-      s4v a[2];
+      const int x = xx[mt] + dx, y = yy[mt] + dy;
+      const bool okr = rv[mt] && x >= 0 && x < d.nx && y >= 0 && y < d.ny;
+      const int64_t row = okr ? vjoin(d, bb[mt], x, y, 0) : 0;
 #pragma unroll
-      for (int mt = 0; mt < 2; mt++) {
-        s4v t = load4(xp[mt] + c0);
-        a[mt] = ok[mt] ? t : zero4;
+      for (int t = 0; t < KS; t++) {
+        const int z = zz[mt] + t - R;
+        const bool ok = okr && z >= 0 && z < d.nz;
+        const s4v e = load4(X + (ok ? row + z : 0) * cx + c0 + 4 * q);
+        a[t][mt] = ok ? e : zero4;
       }
+    }
 #pragma unroll
-      for (int nt = 0; nt < NT; nt++) {
-        const s4v b = load4(wp + (int64_t)nt * 16 * cin + c0);
+    for (int t = 0; t < KS; t++)
+#pragma unroll
+      for (int nt = 0; nt < NT; nt++)
+        b[t][nt] = load4(W + ((int64_t)(xy * KS + t) * cout + n0 + 16 * nt + r) * cin + c0 + 4 * q);
+  };
+  const int g0 = SPLIT ? wv : 0, gs = SPLIT ? 4 : 1;
+  if (g0 < ng) load(g0);
+#pragma unroll 1
+  for (int g = g0; g < ng; g += gs) {
+    s4v ca[KS][2], cb[KS][NT];
+#pragma unroll
+    for (int t = 0; t < KS; t++) {
+#pragma unroll
+      for (int mt = 0; mt < 2; mt++) ca[t][mt] = a[t][mt];
+#pragma unroll
+      for (int nt = 0; nt < NT; nt++) cb[t][nt] = b[t][nt];
+    }
+    if (g + gs < ng) load(g + gs);
+#pragma unroll
+    for (int t = 0; t < KS; t++)
+#pragma unroll
+      for (int nt = 0; nt < NT; nt++)
 #pragma unroll
         for (int mt = 0; mt < 2; mt++)
-          acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[mt], b, acc[mt][nt], 0, 0, 0);
-      }
-    }
+          acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(ca[t][mt], cb[t][nt], acc[mt][nt], 0, 0, 0);
+  }
+  if constexpr (SPLIT) {
+    __shared__ f4v red[3][2 * NT][64];
+#pragma unroll
+    for (int mt = 0; mt < 2; mt++)
+#pragma unroll
+      for (int nt = 0; nt < NT; nt++)
+        if (wv > 0) red[wv - 1][mt * NT + nt][l] = acc[mt][nt];
+    __syncthreads();
+    if (wv > 0) return;
+#pragma unroll
+    for (int mt = 0; mt < 2; mt++)
+#pragma unroll
+      for (int nt = 0; nt < NT; nt++)
+#pragma unroll
+        for (int k = 0; k < 3; k++) acc[mt][nt] += red[k][mt * NT + nt][l];
   }
 #pragma unroll
   for (int mt = 0; mt < 2; mt++)
@@ -141,7 +183,7 @@ __global__ __launch_bounds__(256) void k_conv(Dims d, const bf16 *__restrict__ X
       if (vox >= V) continue;
 #pragma unroll
       for (int nt = 0; nt < NT; nt++) {
-        const int co = 16 * nt + r;
+        const int co = n0 + 16 * nt + r;
         float val = acc[mt][nt][v];
         if (EPI == EPI_ACT) {
           val += bias[co];
@@ -159,87 +201,172 @@ __global__ __launch_bounds__(256) void k_conv(Dims d, const bf16 *__restrict__ X
     }
 }
 
-// dW[tap][co][ci] += sum over a chunk of voxels of dY[v][co] X[v+off(tap)][ci].
-// Grid (chunks, taps).  With at least four (co tile, ci tile) pairs each wave
-// takes the pairs p with p % 4 == wave over the whole chunk; with fewer, every
-// wave takes all pairs over every fourth group of 16 voxels, so that no wave
-// idles on the finest level (16 x 16 channels, one pair).  A operand (rows co,
-// depth voxels) and B operand (depth voxels, columns ci) gathered four voxels
-// per lane.
-template <int KS>
-__global__ __launch_bounds__(256) void k_wgrad(Dims d, const bf16 *__restrict__ X, int cx, int cin,
-                                               const bf16 *__restrict__ dY, int cdy, int cout, int64_t chunk,
-                                               float *__restrict__ dW) {
-  constexpr int R = KS / 2;
-  constexpr int MAXP = 16;  // pairs per wave (cout/16 * cin/16 <= 64)
-  const int tap = blockIdx.y;
-  const int dx = tap / (KS * KS) - R, dy = (tap / KS) % KS - R, dz = tap % KS - R;
-  const int wv = threadIdx.x >> 6, l = threadIdx.x & 63, q = l >> 4, r = l & 15;
-  const int mtn = cout / 16, ntn = cin / 16, np = mtn * ntn;
-  const int pw = np >= 4 ? 4 : 1;            // pair stride across waves
-  const int pofs = wv % pw, vsl = wv / pw;   // this wave's first pair and voxel slice
-  const int64_t vstep = 16 * (4 / pw);
-  const int64_t V = d.vox();
-  const int64_t vb = (int64_t)blockIdx.x * chunk, ve = vb + chunk < V ? vb + chunk : V;
-  f4v acc[MAXP];
-#pragma unroll
-  for (int p = 0; p < MAXP; p++) acc[p] = f4v{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-  for (int64_t k0 = vb + 16 * vsl; k0 < ve; k0 += vstep) {
-    // the four voxels of this lane's depth slice, and their shifted partners
-    int64_t vv[4], vs[4];
-    bool okv[4], oks[4];
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      vv[j] = k0 + 4 * q + j;
-      okv[j] = vv[j] < ve;
-      int b, x, y, z;
-      vsplit(d, okv[j] ? vv[j] : 0, b, x, y, z);
-      x += dx;
-      y += dy;
-      z += dz;
-      oks[j] = okv[j] && x >= 0 && x < d.nx && y >= 0 && y < d.ny && z >= 0 && z < d.nz;
-      vs[j] = oks[j] ? vjoin(d, b, x, y, z) : 0;
-      if (!okv[j]) vv[j] = 0;
-    }
-#pragma unroll
-    for (int pp = 0; pp < MAXP; pp++) {
-      const int p = pofs + pw * pp;
-      if (p >= np) continue;
-      const int mt = p / ntn, nt = p % ntn;
-      s4v a, b;
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        const bf16 av = dY[vv[j] * cdy + 16 * mt + r];
-        const bf16 bv = X[vs[j] * cx + 16 * nt + r];
-        a[j] = (short)(okv[j] ? av : 0);
-        b[j] = (short)(oks[j] ? bv : 0);
-      }
-      acc[pp] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc[pp], 0, 0, 0);
-    }
-  }
-#pragma unroll
-  for (int pp = 0; pp < MAXP; pp++) {
-    const int p = pofs + pw * pp;
-    if (p >= np) continue;
-    const int mt = p / ntn, nt = p % ntn;
-#pragma unroll
-    for (int v = 0; v < 4; v++) {
-      const int co = 16 * mt + 4 * q + v, ci = 16 * nt + r;
-      atomicAdd(&dW[((int64_t)tap * cout + co) * cin + ci], acc[pp][v]);
-    }
-  }
+// dW[tap][co][ci] = sum_v dY[v][co] X[v+off(tap)][ci] for one pair of 16-channel
+// tiles (blockIdx.y), all taps at once, over this workgroup's share of the tiles
+// of 4 x-planes, 4 y-rows and 48 z (one y-row per wave).  The contraction runs
+// over voxels, which are not the contiguous index of either operand: the input
+// planes with their halo (zero outside the grid) are staged channel-major in
+// LDS, three planes in a ring, so that a lane finds its four consecutive z in
+// one word pair and forms the z - 1 and z + 1 operands by shifting; each lane
+// reads its gradient voxels from global memory once for all taps.  The first
+// input tile also carries the bias gradient (a product with ones).  Partial
+// sums go to part[workgroup][pair][tap][16 x 16] and are added in order by
+// k_wred.  All fifteen layers at 64 x 64 x 48 x 2:
+// 0.62 ms with k_wred, against 6.4 + 1.9 ms with one two-byte gather per tap and
+// operand element, atomics and a bias pass of its own.  What is left is staging:
+// the products alone would take about 0.1 ms.
+constexpr int kWgX = 4, kWgY = 4, kWgZ = 48;
+constexpr int kWgP = kWgZ + 8;  // positions per channel row: z - z0 + 4, halo one each side
+__host__ __device__ inline int64_t wgrad_tiles(const Dims &d) {
+  return (int64_t)d.nb * ((d.nx + kWgX - 1) / kWgX) * ((d.ny + kWgY - 1) / kWgY) * ((d.nz + kWgZ - 1) / kWgZ);
+}
+// workgroups per channel pair: one tile each, or equal shares once that would
+// exceed 2048 workgroups (and 58 MB of partial sums)
+static int wgrad_chunks(const Dims &d, int pairs) {
+  const int64_t t = wgrad_tiles(d), per = (t * pairs + 2047) / 2048;
+  return (int)((t + per - 1) / per);
 }
 
-// db[c] += sum_v dY[v][c]
-__global__ void k_bgrad(int64_t V, const bf16 *__restrict__ dY, int cdy, int c, int64_t chunk, float *db) {
-  const int t = threadIdx.x;
-  const int ch = t % c, lane0 = t / c, lanes = blockDim.x / c;
-  if (lane0 >= lanes) return;
-  const int64_t vb = (int64_t)blockIdx.x * chunk, ve = vb + chunk < V ? vb + chunk : V;
+template <int KS>
+__global__ __launch_bounds__(256) void k_wgrad(Dims d, const bf16 *__restrict__ X, int cx, int cin,
+                                               const bf16 *__restrict__ dY, int cdy, int cout,
+                                               float *__restrict__ part) {
+  constexpr int R = KS / 2, NTAP = KS * KS * KS, NROW = kWgY + 2 * R;
+  constexpr int NITEM = (NROW * (kWgZ + 2 * R) * 4 + 255) / 256;  // 4-channel items per thread and plane
+  __shared__ union {
+    bf16 x[KS][NROW][16][kWgP];
+    float red[(NTAP + 1) * 256];
+  } sh;
+  const int ntn = cin / 16, mt = blockIdx.y / ntn, nt = blockIdx.y % ntn;
+  const int tid = threadIdx.x, wv = tid >> 6, l = tid & 63, q = l >> 4, r = l & 15;
+  f4v acc[NTAP + 1];
+#pragma unroll
+  for (int p = 0; p <= NTAP; p++) acc[p] = f4v{0.f, 0.f, 0.f, 0.f};
+  const s4v ones = s4v{0x3f80, 0x3f80, 0x3f80, 0x3f80};
+  const int64_t ntile = wgrad_tiles(d);
+  const int tz = (d.nz + kWgZ - 1) / kWgZ, ty = (d.ny + kWgY - 1) / kWgY, tx = (d.nx + kWgX - 1) / kWgX;
+  for (int64_t tile = blockIdx.x; tile < ntile; tile += gridDim.x) {
+    int64_t e = tile;
+    const int z0 = (int)(e % tz) * kWgZ;
+    e /= tz;
+    const int y0 = (int)(e % ty) * kWgY;
+    e /= ty;
+    const int x0 = (int)(e % tx) * kWgX, b = (int)(e / tx);
+    const int xe = x0 + kWgX < d.nx ? x0 + kWgX : d.nx, zl = d.nz - z0 < kWgZ ? d.nz - z0 : kWgZ;
+    const int nseg = (zl + 15) / 16;
+    s4v st[NITEM];
+    // items of a plane: (row, position, four channels); outside the grid zero
+    auto fetch = [&](int x) {
+#pragma unroll
+      for (int i = 0; i < NITEM; i++) {
+        const int it = tid + 256 * i, cg = it & 3, pos = (it >> 2) % (kWgZ + 2 * R), row = (it >> 2) / (kWgZ + 2 * R);
+        const int y = y0 + row - R, z = z0 + pos - R;
+        const bool ok = row < NROW && x >= 0 && x < d.nx && y >= 0 && y < d.ny && z >= 0 && z < d.nz;
+        const s4v v = load4(X + (ok ? vjoin(d, b, x, y, z) : 0) * cx + 16 * nt + 4 * cg);
+        st[i] = ok ? v : s4v{0, 0, 0, 0};
+      }
+    };
+    auto stash = [&](int slot) {
+#pragma unroll
+      for (int i = 0; i < NITEM; i++) {
+        const int it = tid + 256 * i, cg = it & 3, pos = (it >> 2) % (kWgZ + 2 * R), row = (it >> 2) / (kWgZ + 2 * R);
+        if (row < NROW)
+#pragma unroll
+          for (int c = 0; c < 4; c++) sh.x[slot][row][4 * cg + c][pos - R + 4] = (bf16)st[i][c];
+      }
+    };
+    __syncthreads();  // the previous tile's planes are read to the end
+    for (int x = x0 - R; x < x0 + R; x++) {
+      fetch(x);
+      stash((x + KS) % KS);
+    }
+    fetch(x0 + R);
+    for (int x = x0; x < xe; x++) {
+      // gradient voxels of this wave's row: lane (r, q) holds channel r of voxels 4 q .. 4 q + 3 of each segment
+      const int y = y0 + wv;
+      s4v a[kWgZ / 16];
+#pragma unroll
+      for (int s = 0; s < kWgZ / 16; s++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          const int z = 16 * s + 4 * q + j;
+          const bool ok = y < d.ny && z < zl;
+          const bf16 v = dY[(ok ? vjoin(d, b, x, y, z0 + z) : 0) * cdy + 16 * mt + r];
+          a[s][j] = (short)(ok ? v : 0);
+        }
+      stash((x + R) % KS);
+      __syncthreads();
+      if (x + 1 < xe) fetch(x + 1 + R);
+      if (y < d.ny) {
+#pragma unroll 1
+        for (int s = 0; s < nseg; s++) {
+          const s4v as = s == 0 ? a[0] : s == 1 ? a[1] : a[2];
+          if (nt == 0) acc[NTAP] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(as, ones, acc[NTAP], 0, 0, 0);
+#pragma unroll
+          for (int dx = 0; dx < KS; dx++) {
+            const int slot = (x + dx - R + KS) % KS;
+#pragma unroll
+            for (int dy = 0; dy < KS; dy++) {
+              const bf16 *p = &sh.x[slot][wv + dy][r][16 * s + 4 * q + 4];
+              union {
+                uint32_t u[2];
+                s4v v;
+              } o, lo, hi;
+              o.u[0] = *(const uint32_t *)p;
+              o.u[1] = *(const uint32_t *)(p + 2);
+              if constexpr (KS == 3) {
+                const uint32_t pm = *(const uint32_t *)(p - 2), px = *(const uint32_t *)(p + 4);
+                lo.u[0] = __builtin_amdgcn_alignbit(o.u[0], pm, 16);
+                lo.u[1] = hi.u[0] = __builtin_amdgcn_alignbit(o.u[1], o.u[0], 16);
+                hi.u[1] = __builtin_amdgcn_alignbit(px, o.u[1], 16);
+                const int t0 = (dx * 3 + dy) * 3;
+                acc[t0] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(as, lo.v, acc[t0], 0, 0, 0);
+                acc[t0 + 1] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(as, o.v, acc[t0 + 1], 0, 0, 0);
+                acc[t0 + 2] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(as, hi.v, acc[t0 + 2], 0, 0, 0);
+              } else {
+                acc[0] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(as, o.v, acc[0], 0, 0, 0);
+              }
+            }
+          }
+        }
+      }
+      __syncthreads();
+    }
+  }
+  // the four waves' sums in wave order, then this workgroup's slice
+  for (int k = 0; k < 4; k++) {
+    if (wv == k)
+#pragma unroll
+      for (int p = 0; p <= NTAP; p++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+          float &o = sh.red[p * 256 + (4 * q + v) * 16 + r];
+          o = k == 0 ? acc[p][v] : o + acc[p][v];
+        }
+    __syncthreads();
+  }
+  float *out = part + ((int64_t)blockIdx.x * gridDim.y + blockIdx.y) * (NTAP + 1) * 256;
+  for (int i = tid; i < (NTAP + 1) * 256; i += 256) out[i] = sh.red[i];
+}
+
+// dW, db = sum over workgroups of k_wgrad's partial sums, in order within each
+// of sixteen slices: 64 entries per workgroup (grid: pairs * nt1 * 4, nt1 = taps + 1)
+__global__ __launch_bounds__(1024) void k_wred(int nch, int cin, int cout, int nt1, const float *__restrict__ part,
+                                               float *__restrict__ gw, float *__restrict__ gb) {
+  __shared__ float red[16][64];
+  const int i = threadIdx.x & 63, sl = threadIdx.x >> 6;
+  const int64_t per = (int64_t)gridDim.x * 64, e = (int64_t)blockIdx.x * 64 + i;
   float s = 0.f;
-  for (int64_t v = vb + lane0; v < ve; v += lanes) s += bf2f(dY[v * cdy + ch]);
-  atomicAdd(&db[ch], s);
+#pragma unroll 4
+  for (int c = sl; c < nch; c += 16) s += part[c * per + e];
+  red[sl][i] = s;
+  __syncthreads();
+  if (sl) return;
+  for (int k = 1; k < 16; k++) s += red[k][i];
+  const int ntn = cin / 16, pair = (int)(e / (nt1 * 256)), tap = (int)(e / 256 % nt1);
+  const int co = pair / ntn * 16 + (int)(e % 256) / 16, ci = pair % ntn * 16 + (int)(e % 16);
+  if (tap + 1 < nt1) gw[((int64_t)tap * cout + co) * cin + ci] = s;
+  else if (ci == 0) gb[co] = s;
 }
 
 // fp32 host layout [v][creal] -> bf16 [v][cpad], zero padded
@@ -312,32 +439,60 @@ __global__ void k_pool_bwd(Dims fine, const bf16 *__restrict__ dskip, int cds, c
   dh[v * c + ch] = f2bf(bf2f(h[v * ch_stride + ch]) > 0.f ? s : alpha * s);
 }
 
-// masked MSE: loss += sum m (y - t)^2 / count; dY = 2 m (y - t) / count (bf16)
-__global__ void k_loss(int64_t V, const float *__restrict__ y, int cy, const float *__restrict__ t,
-                       const float *__restrict__ m, int creal, float inv_count, bf16 *__restrict__ dY, int cdy,
-                       float *loss) {
-  __shared__ float red[256];
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  float s = 0.f;
-  if (i < V * cdy) {
-    const int64_t v = i / cdy;
-    const int c = (int)(i % cdy);
-    float g = 0.f;
-    if (c < creal) {
-      const float mm = m ? m[v * creal + c] : 1.f;
-      const float e = y[v * cy + c] - t[v * creal + c];
-      s = mm * e * e * inv_count;
-      g = 2.f * mm * e * inv_count;
-    }
-    dY[v * cdy + c] = f2bf(g);
-  }
+// sum over the workgroup's threads, the same on thread 0 (fixed order)
+__device__ inline double block_sum(double s) {
+  __shared__ double red[256];
   red[threadIdx.x] = s;
   __syncthreads();
   for (int o = 128; o > 0; o >>= 1) {
     if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
     __syncthreads();
   }
-  if (threadIdx.x == 0) atomicAdd(loss, red[0]);
+  s = red[0];
+  __syncthreads();
+  return s;
+}
+
+constexpr int kLossBlocks = 512;
+
+// per-workgroup sums of the mask entries
+__global__ __launch_bounds__(256) void k_count(int64_t n, const float *__restrict__ m, double *__restrict__ part) {
+  double s = 0.0;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) s += m[i];
+  s = block_sum(s);
+  if (threadIdx.x == 0) part[blockIdx.x] = s;
+}
+
+// masked MSE: per-workgroup sums of m (y - t)^2 / count; dY = 2 m (y - t) / count (bf16),
+// count = the mask's sum from k_count's partial sums (all entries without a mask)
+__global__ __launch_bounds__(256) void k_loss(int64_t V, const float *__restrict__ y, int cy,
+                                              const float *__restrict__ t, const float *__restrict__ m, int creal,
+                                              const double *__restrict__ cpart, bf16 *__restrict__ dY, int cdy,
+                                              double *__restrict__ lpart) {
+  double cnt = (double)V * creal;
+  if (m) cnt = block_sum(cpart[threadIdx.x] + cpart[threadIdx.x + 256]);
+  const float inv_count = cnt > 0 ? (float)(1.0 / cnt) : 0.f;
+  double s = 0.0;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < V * cdy; i += (int64_t)gridDim.x * 256) {
+    const int64_t v = i / cdy;
+    const int c = (int)(i % cdy);
+    float g = 0.f;
+    if (c < creal) {
+      const float mm = m ? m[v * creal + c] : 1.f;
+      const float e = y[v * cy + c] - t[v * creal + c];
+      s += mm * e * e * inv_count;
+      g = 2.f * mm * e * inv_count;
+    }
+    dY[v * cdy + c] = f2bf(g);
+  }
+  s = block_sum(s);
+  if (threadIdx.x == 0) lpart[blockIdx.x] = s;
+}
+static_assert(kLossBlocks == 512, "k_loss and k_loss_sum read two partial sums per thread");
+
+__global__ __launch_bounds__(256) void k_loss_sum(const double *__restrict__ lpart, double *__restrict__ loss) {
+  const double s = block_sum(lpart[threadIdx.x] + lpart[threadIdx.x + 256]);
+  if (threadIdx.x == 0) *loss = s;
 }
 
 // fp32 [v][cpad] -> host layout [v][creal]
@@ -347,37 +502,36 @@ __global__ void k_unpack(int64_t V, const float *__restrict__ in, int cpad, int 
   out[i] = in[(i / creal) * cpad + (i % creal)];
 }
 
-// Adam on one layer's fp32 master weights w[tap][co][ci] and bias, then the
+// Adam on every layer's fp32 master weights and biases (blockIdx.y: layer; w
+// [tap][co][ci] then b at the layer's offset in the arenas), then the weights'
 // bf16 copies in both layouts: Wb[tap][co][ci] and Wt[flip(tap)][ci][co]
-__global__ void k_adam(int64_t nw, int cout, int cin, int ntap, float *w, float *mw, float *vw, const float *gw,
-                       float lr, float b1, float b2, float eps, float c1, float c2, bf16 *Wb, bf16 *Wt) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nw) return;
-  const float g = gw[i];
-  const float m = b1 * mw[i] + (1.f - b1) * g;
-  const float v = b2 * vw[i] + (1.f - b2) * g * g;
-  mw[i] = m;
-  vw[i] = v;
-  const float x = w[i] - lr * (m * c1) / (sqrtf(v * c2) + eps);
-  w[i] = x;
-  const int64_t per = (int64_t)cout * cin;
+struct AdamLayer {
+  int64_t off, nw;
+  int cout, cin, ntap;
+  bf16 *Wb, *Wt;
+};
+struct AdamTable {
+  AdamLayer l[15];
+};
+__global__ void k_adam(AdamTable tab, float *__restrict__ w, float *__restrict__ mw, float *__restrict__ vw,
+                       const float *__restrict__ gw, float lr, float b1, float b2, float eps, float c1, float c2) {
+  const AdamLayer L = tab.l[blockIdx.y];
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, p = L.off + i;
+  if (i >= L.nw + L.cout) return;
+  const float g = gw[p];
+  const float m = b1 * mw[p] + (1.f - b1) * g;
+  const float v = b2 * vw[p] + (1.f - b2) * g * g;
+  mw[p] = m;
+  vw[p] = v;
+  const float x = w[p] - lr * (m * c1) / (sqrtf(v * c2) + eps);
+  w[p] = x;
+  if (i >= L.nw) return;
+  const int64_t per = (int64_t)L.cout * L.cin;
   const int tap = (int)(i / per);
-  const int co = (int)((i % per) / cin), ci = (int)(i % cin);
+  const int co = (int)((i % per) / L.cin), ci = (int)(i % L.cin);
   const bf16 xb = f2bf(x);
-  Wb[i] = xb;
-  Wt[((int64_t)(ntap - 1 - tap) * cin + ci) * cout + co] = xb;
-}
-
-__global__ void k_adam_bias(int n, float *b, float *mb, float *vb, const float *gb, float lr, float b1, float b2,
-                            float eps, float c1, float c2) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float g = gb[i];
-  const float m = b1 * mb[i] + (1.f - b1) * g;
-  const float v = b2 * vb[i] + (1.f - b2) * g * g;
-  mb[i] = m;
-  vb[i] = v;
-  b[i] -= lr * (m * c1) / (sqrtf(v * c2) + eps);
+  L.Wb[i] = xb;
+  L.Wt[((int64_t)(L.ntap - 1 - tap) * L.cin + ci) * L.cout + co] = xb;
 }
 
 // bf16 copies of fp32 master weights (after set_params)
@@ -390,11 +544,6 @@ __global__ void k_wcopy(int64_t nw, int cout, int cin, int ntap, const float *w,
   const bf16 xb = f2bf(w[i]);
   Wb[i] = xb;
   Wt[((int64_t)(ntap - 1 - tap) * cin + ci) * cout + co] = xb;
-}
-
-__global__ void k_fill_f32(int64_t n, float *p, float v) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = v;
 }
 
 }  // namespace nn
@@ -411,8 +560,8 @@ struct mvf_nn {
   struct Layer {
     int ks = 3, cin = 0, cout = 0;
     int64_t nw = 0;
-    float *w = nullptr, *b = nullptr, *mw = nullptr, *vw = nullptr, *mb = nullptr, *vb = nullptr;
-    float *gw = nullptr, *gb = nullptr;
+    int64_t off = 0;  // of w in the parameter arenas, b following
+    float *w = nullptr, *b = nullptr;
     mvf::nn::bf16 *Wb = nullptr, *Wt = nullptr;
   };
   // encoder e[k][0..1], decoder d[k][0..1] (k = 0..2), head
@@ -425,7 +574,14 @@ struct mvf_nn {
   // gradients (bf16), same shapes
   mvf::nn::bf16 *ge1[NL] = {}, *gcat[NL] = {}, *gpin[NL] = {}, *gd1[NL] = {}, *gd2[NL] = {}, *gbott = nullptr;
   mvf::nn::bf16 *gout = nullptr;
-  float *out = nullptr, *xin = nullptr, *tin = nullptr, *min_ = nullptr, *dloss = nullptr, *hout = nullptr;
+  float *out = nullptr, *xin = nullptr, *tin = nullptr, *min_ = nullptr, *hout = nullptr;
+  // all layers' parameters, gradients and moments in the host layout (per layer
+  // w then b), so that each set moves in one copy; the layers point into them
+  float *pw = nullptr, *pg = nullptr, *pm = nullptr, *pv = nullptr;
+  int64_t np = 0;
+  float *wpart = nullptr;  // k_wgrad's partial sums
+  // mask counts and losses per workgroup, then the loss itself
+  double *lpart = nullptr;
   std::vector<void *> owned;
   int64_t step = 0;
   // last forward+backward: matrix-core kernel time (HIP events) and flops
@@ -470,25 +626,26 @@ static Dims level_dims(const mvf_nn *n, int k) {
   return Dims{n->nb, n->cfg.nx >> k, n->cfg.ny >> k, n->cfg.nz >> k};
 }
 
-static int make_layer(mvf_nn *n, mvf_nn::Layer &L, int ks, int cin, int cout, std::mt19937_64 &rng) {
+// the layer's place in the parameter arenas (allocated once all shapes are known)
+static void shape_layer(mvf_nn *n, mvf_nn::Layer &L, int ks, int cin, int cout) {
   L.ks = ks;
   L.cin = cin;
   L.cout = cout;
-  const int ntap = ks * ks * ks;
-  L.nw = (int64_t)ntap * cin * cout;
-  for (float **p : {&L.w, &L.mw, &L.vw, &L.gw}) MVF_TRY(nn_alloc(n, p, L.nw));
-  for (float **p : {&L.b, &L.mb, &L.vb, &L.gb}) MVF_TRY(nn_alloc(n, p, cout));
+  L.nw = (int64_t)ks * ks * ks * cin * cout;
+  n->np += L.nw + cout;
+}
+
+static int init_layer(mvf_nn *n, mvf_nn::Layer &L, int64_t &off, std::vector<float> &host, std::mt19937_64 &rng) {
+  L.off = off;
+  L.w = n->pw + off;
+  L.b = L.w + L.nw;
   MVF_TRY(nn_alloc(n, &L.Wb, L.nw));
   MVF_TRY(nn_alloc(n, &L.Wt, L.nw));
-  // He-uniform initialisation from the seeded generator
-  std::vector<float> w(L.nw);
-  const float bound = std::sqrt(6.0f / (float)(ntap * cin));
+  // He-uniform initialisation from the seeded generator, zero biases
+  const float bound = std::sqrt(6.0f / (float)(L.ks * L.ks * L.ks * L.cin));
   std::uniform_real_distribution<float> U(-bound, bound);
-  for (auto &x : w) x = U(rng);
-  NN_HIP(n, hipMemcpy(L.w, w.data(), 4 * L.nw, hipMemcpyHostToDevice));
-  std::vector<float> z(std::max<int64_t>(L.nw, cout), 0.f);
-  for (float *p : {L.mw, L.vw, L.gw}) NN_HIP(n, hipMemcpy(p, z.data(), 4 * L.nw, hipMemcpyHostToDevice));
-  for (float *p : {L.b, L.mb, L.vb, L.gb}) NN_HIP(n, hipMemcpy(p, z.data(), 4 * cout, hipMemcpyHostToDevice));
+  for (int64_t i = 0; i < L.nw; i++) host[off + i] = U(rng);
+  off += L.nw + L.cout;
   return 0;
 }
 
@@ -538,29 +695,54 @@ static int alloc_acts(mvf_nn *n, int nb) {
   MVF_TRY(nn_alloc(n, &n->tin, V0 * n->cfg.cout));
   MVF_TRY(nn_alloc(n, &n->min_, V0 * n->cfg.cout));
   MVF_TRY(nn_alloc(n, &n->hout, V0 * n->cfg.cout));
-  MVF_TRY(nn_alloc(n, &n->dloss, 1));
+  MVF_TRY(nn_alloc(n, &n->lpart, 2 * kLossBlocks + 1));
+  // the largest partial-sum buffer any layer's weight gradient needs
+  int64_t wp = 0;
+  auto need = [&](const mvf_nn::Layer &L, int k) {
+    const Dims d = level_dims(n, k);
+    const int pairs = (L.cin / 16) * (L.cout / 16);
+    wp = std::max(wp, (int64_t)wgrad_chunks(d, pairs) * pairs * (L.ks * L.ks * L.ks + 1) * 256);
+  };
+  for (int k = 0; k < mvf_nn::NL; k++)
+    for (int s = 0; s < 2; s++) {
+      need(n->enc[k][s], k);
+      if (k + 1 < mvf_nn::NL) need(n->dec[k][s], k);
+    }
+  need(n->head, 0);
+  MVF_TRY(nn_alloc(n, &n->wpart, wp));
   return 0;
 }
 
 // conv launches: y = conv(x) with the layer's forward weights, or the data
-// gradient with its flipped transposed weights
+// gradient with its flipped transposed weights.  nt: output channels / 16.
+// Below 512 workgroups of 128 voxels (two per CU) the taps are split over the
+// four waves instead, with the channel groups as small as keeps 512 workgroups;
+// above, one wave takes as many channels as divide the count (up to 64), which
+// reads the inputs fewest times.
 template <int KS, int EPI>
 static void conv_nt(mvf_nn *n, int nt, Dims d, const bf16 *X, int cx, int cin, const bf16 *W, const float *bias,
                     void *Y, int cy, const bf16 *mask, int cm) {
-  const unsigned grid = (unsigned)((d.vox() + 127) / 128);
+  const int64_t V = d.vox();
   const float a = n->cfg.leaky;
-#define NN_CONV(NT_)                                                                                          \
-  hipLaunchKernelGGL((k_conv<KS, NT_, EPI>), dim3(grid), dim3(256), 0, n->stream, d, X, cx, cin, W, bias, Y, cy, \
-                     mask, cm, a)
-  switch (nt) {
-    case 1: NN_CONV(1); break;
-    case 2: NN_CONV(2); break;
-    case 3: NN_CONV(3); break;
-    case 4: NN_CONV(4); break;
-    case 6: NN_CONV(6); break;
-    case 10: NN_CONV(10); break;
-    default: break;
+  const bool split = KS > 1 && (V + 127) / 128 < 512;
+  const int64_t wgs = split ? (V + 31) / 32 : (V + 127) / 128;
+  int g = 1;
+  if (split) g = (nt % 2 == 0 && wgs * (nt / 2) >= 512) ? 2 : 1;
+  else g = nt % 4 == 0 ? 4 : nt % 3 == 0 ? 3 : nt % 2 == 0 ? 2 : 1;
+#define NN_CONV(NT_, S_)                                                                                      \
+  hipLaunchKernelGGL((k_conv<KS, NT_, EPI, S_>), dim3((unsigned)wgs, nt / NT_), dim3(256), 0, n->stream, d, X, \
+                     cx, cin, 16 * nt, W, bias, Y, cy, mask, cm, a)
+  if constexpr (KS > 1) {
+    if (split) {
+      if (g == 2) NN_CONV(2, true);
+      else NN_CONV(1, true);
+      return;
+    }
   }
+  if (g == 4) NN_CONV(4, false);
+  else if (g == 3) NN_CONV(3, false);
+  else if (g == 2) NN_CONV(2, false);
+  else NN_CONV(1, false);
 #undef NN_CONV
 }
 
@@ -606,24 +788,21 @@ static void conv_dgrad(mvf_nn *n, const mvf_nn::Layer &L, Dims d, const bf16 *dY
 
 static void conv_wgrad(mvf_nn *n, const mvf_nn::Layer &L, Dims d, const bf16 *X, int cx, const bf16 *dY) {
   const int64_t V = d.vox();
-  // about 16 voxel chunks of at least 256 voxels per tap and chunk, rounded to 16
-  int64_t chunk = (V + 63) / 64;
-  chunk = ((chunk + 15) / 16) * 16;
-  if (chunk < 256) chunk = 256;
-  const unsigned nch = (unsigned)((V + chunk - 1) / chunk);
+  const int pairs = (L.cin / 16) * (L.cout / 16), nch = wgrad_chunks(d, pairs);
+  float *gw = n->pg + L.off, *gb = gw + L.nw;
   tick(n);
   if (L.ks == 3)
-    hipLaunchKernelGGL((k_wgrad<3>), dim3(nch, 27), dim3(256), 0, n->stream, d, X, cx, L.cin, dY, L.cout, L.cout,
-                       chunk, L.gw);
+    hipLaunchKernelGGL((k_wgrad<3>), dim3(nch, pairs), dim3(256), 0, n->stream, d, X, cx, L.cin, dY, L.cout, L.cout,
+                       n->wpart);
   else
-    hipLaunchKernelGGL((k_wgrad<1>), dim3(nch, 1), dim3(256), 0, n->stream, d, X, cx, L.cin, dY, L.cout, L.cout, chunk,
-                       L.gw);
+    hipLaunchKernelGGL((k_wgrad<1>), dim3(nch, pairs), dim3(256), 0, n->stream, d, X, cx, L.cin, dY, L.cout, L.cout,
+                       n->wpart);
+  const int nt1 = L.ks * L.ks * L.ks + 1;
+  hipLaunchKernelGGL(k_wred, dim3((unsigned)(pairs * nt1 * 4)), dim3(1024), 0, n->stream, nch, L.cin, L.cout, nt1,
+                     n->wpart, gw, gb);
   tick(n);
   n->conv_flops += 2.0 * (double)V * L.ks * L.ks * L.ks * L.cin * L.cout;
   n->conv_launches++;
-  const int64_t bch = 4096;
-  hipLaunchKernelGGL(k_bgrad, dim3((unsigned)((V + bch - 1) / bch)), dim3(256), 0, n->stream, V, dY, L.cout, L.cout,
-                     bch, L.gb);
 }
 
 static unsigned g256(int64_t n) { return (unsigned)((n + 255) / 256); }
@@ -726,13 +905,6 @@ static int load_inputs(mvf_nn *n, int nb, const float *x, const float *t, const 
   return 0;
 }
 
-static void zero_grads(mvf_nn *n) {
-  for_layers(n, [&](mvf_nn::Layer &L) {
-    hipLaunchKernelGGL(k_fill_f32, dim3(g256(L.nw)), dim3(256), 0, n->stream, L.nw, L.gw, 0.f);
-    hipLaunchKernelGGL(k_fill_f32, dim3(1), dim3(256), 0, n->stream, (int64_t)L.cout, L.gb, 0.f);
-  });
-}
-
 static void timing_begin(mvf_nn *n) {
   for (auto e : n->evs) (void)hipEventDestroy(e);
   n->evs.clear();
@@ -794,17 +966,28 @@ int mvf_nn_create(const mvf_nn_config *cfg, mvf_nn **out) {
   n->ch[1] = 2 * w;
   n->ch[2] = 4 * w;
   n->ch[3] = 6 * w;
-  std::mt19937_64 rng(cfg->seed);
   for (int k = 0; k < mvf_nn::NL; k++) {
-    const int cin = k == 0 ? 16 : n->ch[k - 1];
-    MVF_TRY(make_layer(n, n->enc[k][0], 3, cin, n->ch[k], rng));
-    MVF_TRY(make_layer(n, n->enc[k][1], 3, n->ch[k], n->ch[k], rng));
+    shape_layer(n, n->enc[k][0], 3, k == 0 ? 16 : n->ch[k - 1], n->ch[k]);
+    shape_layer(n, n->enc[k][1], 3, n->ch[k], n->ch[k]);
   }
   for (int k = 0; k < mvf_nn::NL - 1; k++) {
-    MVF_TRY(make_layer(n, n->dec[k][0], 3, n->ch[k + 1] + n->ch[k], n->ch[k], rng));
-    MVF_TRY(make_layer(n, n->dec[k][1], 3, n->ch[k], n->ch[k], rng));
+    shape_layer(n, n->dec[k][0], 3, n->ch[k + 1] + n->ch[k], n->ch[k]);
+    shape_layer(n, n->dec[k][1], 3, n->ch[k], n->ch[k]);
   }
-  MVF_TRY(make_layer(n, n->head, 1, n->ch[0], 16, rng));
+  shape_layer(n, n->head, 1, n->ch[0], 16);
+  for (float **p : {&n->pw, &n->pg, &n->pm, &n->pv}) MVF_TRY(nn_alloc(n, p, n->np));
+  {
+    std::vector<float> host(n->np, 0.f);
+    for (float *p : {n->pg, n->pm, n->pv}) NN_HIP(n, hipMemcpy(p, host.data(), 4 * n->np, hipMemcpyHostToDevice));
+    std::mt19937_64 rng(cfg->seed);
+    int64_t off = 0;
+    int rc = 0;
+    for_layers(n, [&](mvf_nn::Layer &L) {
+      if (!rc) rc = init_layer(n, L, off, host, rng);
+    });
+    if (rc) return rc;
+    NN_HIP(n, hipMemcpy(n->pw, host.data(), 4 * n->np, hipMemcpyHostToDevice));
+  }
   for_layers(n, [&](mvf_nn::Layer &L) { refresh_bf16(n, L); });
   MVF_TRY(alloc_acts(n, cfg->batch));
   NN_HIP(n, hipStreamSynchronize(n->stream));
@@ -836,27 +1019,15 @@ static int copy_params(mvf_nn *n, float *host, bool grads, bool to_device) {
   if (!n || !host) return MVF_E_ARG;
   NN_HIP(n, hipSetDevice(n->cfg.device));
   NN_HIP(n, hipStreamSynchronize(n->stream));
-  int64_t off = 0;
-  int rc = 0;
-  for_layers(n, [&](mvf_nn::Layer &L) {
-    if (rc) return;
-    float *w = grads ? L.gw : L.w, *b = grads ? L.gb : L.b;
-    hipError_t e1, e2;
-    if (to_device) {
-      e1 = hipMemcpy(w, host + off, 4 * L.nw, hipMemcpyHostToDevice);
-      e2 = hipMemcpy(b, host + off + L.nw, 4 * L.cout, hipMemcpyHostToDevice);
-    } else {
-      e1 = hipMemcpy(host + off, w, 4 * L.nw, hipMemcpyDeviceToHost);
-      e2 = hipMemcpy(host + off + L.nw, b, 4 * L.cout, hipMemcpyDeviceToHost);
-    }
-    if (e1 != hipSuccess || e2 != hipSuccess) rc = nn_err(n, MVF_E_DEVICE, "parameter copy failed");
-    off += L.nw + L.cout;
-  });
-  if (!rc && to_device && !grads) {
+  float *dev = grads ? n->pg : n->pw;
+  const size_t bytes = 4 * (size_t)n->np;
+  NN_HIP(n, to_device ? hipMemcpy(dev, host, bytes, hipMemcpyHostToDevice)
+                      : hipMemcpy(host, dev, bytes, hipMemcpyDeviceToHost));
+  if (to_device && !grads) {
     for_layers(n, [&](mvf_nn::Layer &L) { refresh_bf16(n, L); });
     NN_HIP(n, hipStreamSynchronize(n->stream));
   }
-  return rc;
+  return 0;
 }
 
 int mvf_nn_get_params(mvf_nn *n, float *out) { return copy_params(n, out, false, false); }
@@ -872,26 +1043,19 @@ int mvf_nn_forward_backward(mvf_nn *n, int32_t nb, const float *x, const float *
   forward(n);
   const int64_t V = level_dims(n, 0).vox();
   // normalisation: the masked entry count (all entries without a mask)
-  double cnt = 0.0;
-  if (m) {
-    std::vector<float> hm(V * n->cfg.cout);
-    memcpy(hm.data(), m, 4 * hm.size());
-    for (float v : hm) cnt += v;
-  } else {
-    cnt = (double)V * n->cfg.cout;
-  }
-  const float inv = cnt > 0 ? (float)(1.0 / cnt) : 0.f;
-  hipLaunchKernelGGL(k_fill_f32, dim3(1), dim3(64), 0, n->stream, (int64_t)1, n->dloss, 0.f);
-  hipLaunchKernelGGL(k_loss, dim3(g256(V * 16)), dim3(256), 0, n->stream, V, n->out, 16, n->tin,
-                     m ? n->min_ : nullptr, n->cfg.cout, inv, n->gout, 16, n->dloss);
-  zero_grads(n);
+  if (m)
+    hipLaunchKernelGGL(k_count, dim3(kLossBlocks), dim3(256), 0, n->stream, V * n->cfg.cout, n->min_, n->lpart);
+  hipLaunchKernelGGL(k_loss, dim3(kLossBlocks), dim3(256), 0, n->stream, V, n->out, 16, n->tin, m ? n->min_ : nullptr,
+                     n->cfg.cout, n->lpart, n->gout, 16, n->lpart + kLossBlocks);
+  hipLaunchKernelGGL(k_loss_sum, dim3(1), dim3(256), 0, n->stream, n->lpart + kLossBlocks,
+                     n->lpart + 2 * kLossBlocks);
   backward(n);
-  float hl = 0.f;
-  NN_HIP(n, hipMemcpyAsync(&hl, n->dloss, 4, hipMemcpyDeviceToHost, n->stream));
+  double hl = 0.0;
+  NN_HIP(n, hipMemcpyAsync(&hl, n->lpart + 2 * kLossBlocks, 8, hipMemcpyDeviceToHost, n->stream));
   NN_HIP(n, hipStreamSynchronize(n->stream));
   NN_HIP(n, hipGetLastError());
   timing_end(n);
-  if (loss) *loss = hl;
+  if (loss) *loss = (float)hl;
   return 0;
 }
 
@@ -902,12 +1066,15 @@ int mvf_nn_adam(mvf_nn *n, float lr) {
   const float b1 = n->cfg.beta1, b2 = n->cfg.beta2;
   const float c1 = 1.f / (1.f - std::pow(b1, (float)n->step)), c2 = 1.f / (1.f - std::pow(b2, (float)n->step));
   const float eps = n->cfg.eps;
+  AdamTable tab;
+  int nl = 0;
+  int64_t mx = 0;
   for_layers(n, [&](mvf_nn::Layer &L) {
-    hipLaunchKernelGGL(k_adam, dim3(g256(L.nw)), dim3(256), 0, n->stream, L.nw, L.cout, L.cin, L.ks * L.ks * L.ks,
-                       L.w, L.mw, L.vw, L.gw, lr, b1, b2, eps, c1, c2, L.Wb, L.Wt);
-    hipLaunchKernelGGL(k_adam_bias, dim3(1), dim3(256), 0, n->stream, L.cout, L.b, L.mb, L.vb, L.gb, lr, b1, b2, eps,
-                       c1, c2);
+    tab.l[nl++] = AdamLayer{L.off, L.nw, L.cout, L.cin, L.ks * L.ks * L.ks, L.Wb, L.Wt};
+    mx = std::max(mx, L.nw + L.cout);
   });
+  hipLaunchKernelGGL(k_adam, dim3(g256(mx), nl), dim3(256), 0, n->stream, tab, n->pw, n->pm, n->pv, n->pg, lr, b1, b2,
+                     eps, c1, c2);
   NN_HIP(n, hipStreamSynchronize(n->stream));
   NN_HIP(n, hipGetLastError());
   return 0;

@@ -47,15 +47,41 @@ def test_unet_matches_torch(need_gpu):
     assert np.linalg.norm(y - yr) / np.linalg.norm(yr) <= 2e-2
 
 
+@pytest.mark.parametrize("nx,ny,nz,nb", [
+    (8, 24, 104, 1),   # three z tiles of the weight gradient, the last of 8; coarse rows of 13 z, y remainders 2 and 3
+    (24, 8, 8, 3),     # one voxel along y and z at the coarsest level
+    (40, 40, 48, 1),   # 76800 voxels: the finest level's convolutions unsplit, the others split over taps
+])
+def test_unet_matches_torch_shapes(nx, ny, nz, nb, need_gpu):
+    """Tile remainders and the split / unsplit convolutions, to the bars of
+    test_unet_matches_torch; the unmasked loss as well."""
+    net = Lm.Net(nx=nx, ny=ny, nz=nz, batch=nb, seed=11)
+    rng = np.random.default_rng(1)
+    x = rng.standard_normal((nb, nx, ny, nz, 3)).astype(np.float32)
+    t = rng.standard_normal((nb, nx, ny, nz, 12)).astype(np.float32)
+    p = net.params()
+    for m in ((rng.random(t.shape) < 0.7).astype(np.float32), None):
+        loss = net.forward_backward(x, t, m)
+        g = net.grads()
+        lr, gr, yr = unet_ref.forward_backward(p, x, t, np.ones_like(t) if m is None else m)
+        assert abs(loss - lr) <= 1e-4 * abs(lr)
+        assert g @ gr / np.linalg.norm(g) / np.linalg.norm(gr) >= 0.999
+        off = 0
+        for ks, cin, cout in unet_ref.layer_shapes():
+            n = ks ** 3 * cin * cout + cout
+            assert np.linalg.norm(g[off:off + n] - gr[off:off + n]) <= 0.1 * np.linalg.norm(gr[off:off + n])
+            off += n
+    y = net.predict(x)
+    assert np.linalg.norm(y - yr) / np.linalg.norm(yr) <= 2e-2
+
+
 def test_training_reduces_loss(need_gpu):
     """Adam on six 16 x 16 x (12 + 4) solver fields.  The targets are normalized
     per polarization, so predicting zero costs about 0.5 (computed below as the
     masked mean of t^2).  Within 300 steps (learning rate 5e-4 after a 30-step
     linear warm-up; at 2e-3 without warm-up the loss can rise) the masked loss
     falls below half of that, i.e. the network explains more than half of the
-    targets' energy.  The weight gradient's atomic sums make runs differ: after
-    150 steps one run ended at 0.253, just above the bar; after 300 steps runs
-    end near 0.085."""
+    targets' energy.  After 300 steps runs end near 0.087."""
     data = []
     for s in range(6):
         m, f = Lm.training_model(900 + s, nx=16, ny=16, nz_earth=12, nz_air=4)
