@@ -53,72 +53,239 @@ __device__ inline double ld(const T *p, int64_t i) {
 }
 
 // ---------------------------------------------------------------- SpMV -----
+// value of v in lane j of each group of N = 2 or 4 lanes
+template <int N, int J>
+__device__ __forceinline__ int group_bcast(int v) {
+  constexpr int ctrl = N == 4 ? J * 0x55 : (J ? 0xf5 : 0xa0);  // quad permutation
+  return __builtin_amdgcn_update_dpp(v, v, ctrl, 0xf, 0xf, false);
+}
+template <int N, int J>
+__device__ __forceinline__ double group_bcast(double v) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  const unsigned lo = (unsigned)group_bcast<N, J>((int)(unsigned)b), hi = (unsigned)group_bcast<N, J>((int)(b >> 32));
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+template <int N, int J>
+__device__ __forceinline__ float group_bcast(float v) {
+  return __int_as_float(group_bcast<N, J>(__float_as_int(v)));
+}
+
+template <typename T>
+struct Pair {
+  T x, y;
+};
+
+// entries per lane loaded together in one pass over a row: 33 entries of an
+// 8-node row are one pass of 8 lanes x 5, ~84 of a 20-node row one of 16 x 6
+template <int LPR>
+constexpr int spmv_unroll() {
+  return LPR <= 8 ? 5 : LPR <= 16 ? 6 : 4;
+}
+
 // y = A x (columns 0..NC-1); LPR lanes share a row.  With DOT, block partials
-// of p^T y (bilinear) are written to part[block][c].
-template <typename VT, typename MT, int NC, int LPR, bool C64, bool DOT>
+// of p^T y (bilinear) are written to part[block][c].  The rate is set by the
+// gathers of x (NC x 16 bytes per entry, three to four times the operator's own
+// bytes) rather than by HBM.  With two or four columns each lane loads its own
+// entries, then each group of NC lanes walks the group's entries together, lane
+// c taking column c: a gather reads whole NC x 16 byte runs and a lane keeps one
+// column's sum, against one lane reading all columns of its entry (64 cache
+// lines per load instruction, four sums per lane).  All entries of a pass and
+// then all their x are loaded before the first product, from clamped addresses,
+// the entries past the row as zeros, and the next row's entries are loaded
+// before the current row's are summed.  With C64 the caller passes fl32(K), which
+// is what the rounding makes of K, at half its bytes.  8-node 64 x 64 x 48, four
+// columns, with the dot product: 170 us one lane per entry, 156 us grouped, 130
+// us with the next row's loads ahead; capping the registers for a third wave per
+// SIMD spills and takes twice the time.
+template <typename VT, typename KT, typename MT, int NC, int LPR, bool C64, bool DOT>
 __device__ __forceinline__ void spmv_body(int64_t nne, const int64_t *__restrict__ rowptr,
-                                          const int32_t *__restrict__ col, const MT *__restrict__ K,
+                                          const int32_t *__restrict__ col, const KT *__restrict__ K,
                                           const MT *__restrict__ M, const ColW &w, const VT *__restrict__ x,
                                           VT *__restrict__ y, const VT *__restrict__ p, double *__restrict__ part) {
+  constexpr bool GROUP = NC == 2 || NC == 4;
   const int lane = threadIdx.x % LPR;
-  const int64_t rstride = (int64_t)gridDim.x * (kBS / LPR);
   double dr[NC], di[NC];
 #pragma unroll
   for (int c = 0; c < NC; c++) dr[c] = di[c] = 0.0;
-  const int64_t rfirst = ((int64_t)blockIdx.x * kBS + threadIdx.x) / LPR;
-  const int64_t rlast = rfirst + ((nne - rfirst + rstride - 1) / rstride) * rstride;  // uniform trip count per group
-  for (int64_t row = rfirst; row < (rlast > rfirst ? rlast : rfirst + rstride); row += rstride) {
-  double ar[NC], ai[NC];
+  // workgroups are dealt to the XCDs in turn: renumbered so that each XCD walks
+  // one contiguous eighth of the rows, each workgroup a contiguous run of it
+  const int gx = gridDim.x, bx = blockIdx.x, x8 = bx % 8;
+  const int64_t wg = (int64_t)x8 * (gx / 8) + (x8 < gx % 8 ? x8 : gx % 8) + bx / 8;
+  constexpr int RP = kBS / LPR;  // rows of one pass
+  const int64_t per = ((nne + RP - 1) / RP + gx - 1) / gx * RP;
+  const int64_t rend = (wg + 1) * per < nne ? (wg + 1) * per : nne;
+  if constexpr (GROUP) {
+    constexpr int U = spmv_unroll<LPR>();
+    const int gc = threadIdx.x % NC;
+    double wc = w.w[0], sr = 0.0, si = 0.0;
 #pragma unroll
-  for (int c = 0; c < NC; c++) ar[c] = ai[c] = 0.0;
-  if (row < nne) {
-    const int64_t k1 = rowptr[row + 1];
-    // one entry of the lane: A_k x_col(k) accumulated into (ar, ai)
-    auto entry = [&](int64_t cc, double kv, double mv) {
-      const VT *xp = x + 2 * cc * NC;
+    for (int c = 1; c < NC; c++) wc = gc == c ? w.w[c] : wc;
+    const Pair<VT> *xp = (const Pair<VT> *)x + gc;
+    int cc[U];
+    KT kv[U];
+    MT mv[U];
+    // entries kb + lane + u LPR of a row ending at k1 (kb < k1; past the row: the last one's column, zero values)
+    auto load = [&](int64_t kb, int64_t k1) {
 #pragma unroll
-      for (int c = 0; c < NC; c++) {
-        double vr = kv, vi = w.w[c] * mv;
+      for (int u = 0; u < U; u++) {
+        const int64_t k = kb + lane + u * LPR;
+        const bool in = k < k1;
+        const int64_t e = in ? k : k1 - 1;
+        cc[u] = col[e];
+        const KT ke = K[e];
+        const MT me = M[e];
+        kv[u] = in ? ke : (KT)0;
+        mv[u] = in ? me : (MT)0;
+      }
+    };
+    double ar, ai;
+    // gathers x for the loaded entries, has `ahead` issue what comes next, then sums
+    auto pass = [&](auto &&ahead) {
+      Pair<VT> xv[U][NC];
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        xv[u][0] = xp[(int64_t)group_bcast<NC, 0>(cc[u]) * NC];
+        xv[u][1] = xp[(int64_t)group_bcast<NC, 1>(cc[u]) * NC];
+        if constexpr (NC == 4) {
+          xv[u][2] = xp[(int64_t)group_bcast<NC, 2>(cc[u]) * NC];
+          xv[u][3] = xp[(int64_t)group_bcast<NC, 3>(cc[u]) * NC];
+        }
+      }
+      KT kc[U];
+      MT mc[U];
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        kc[u] = kv[u];
+        mc[u] = mv[u];
+      }
+      ahead();
+      auto entry = [&](double ke, double me, const Pair<VT> &xe) {
+        double vr = ke, vi = wc * me;
         if (C64) {
           vr = (double)(float)vr;
           vi = (double)(float)vi;
         }
-        const double xr = (double)xp[2 * c], xi = (double)xp[2 * c + 1];
-        ar[c] += vr * xr - vi * xi;
-        ai[c] += vr * xi + vi * xr;
+        const double xr = (double)xe.x, xi = (double)xe.y;
+        ar += vr * xr - vi * xi;
+        ai += vr * xi + vi * xr;
+      };
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        entry((double)group_bcast<NC, 0>(kc[u]), (double)group_bcast<NC, 0>(mc[u]), xv[u][0]);
+        entry((double)group_bcast<NC, 1>(kc[u]), (double)group_bcast<NC, 1>(mc[u]), xv[u][1]);
+        if constexpr (NC == 4) {
+          entry((double)group_bcast<NC, 2>(kc[u]), (double)group_bcast<NC, 2>(mc[u]), xv[u][2]);
+          entry((double)group_bcast<NC, 3>(kc[u]), (double)group_bcast<NC, 3>(mc[u]), xv[u][3]);
+        }
       }
     };
-    int64_t k = rowptr[row] + lane;
-    // two entries per lane in flight, accumulated in the same order
-    for (; k + LPR < k1; k += 2 * LPR) {
-      const int64_t c0 = col[k], c1 = col[k + LPR];
-      const double k0v = (double)K[k], m0v = (double)M[k], k1v = (double)K[k + LPR], m1v = (double)M[k + LPR];
-      entry(c0, k0v, m0v);
-      entry(c1, k1v, m1v);
+    // bounds of the row at rb (this thread's row; an absent one repeats the last row and is not stored)
+    auto bounds = [&](int64_t rb, int64_t &k0, int64_t &k1) {
+      const int64_t r = rb + threadIdx.x / LPR, rr = r < rend ? r : rend - 1;
+      k0 = rowptr[rr];
+      k1 = rowptr[rr + 1];
+    };
+    int64_t rb = wg * per, k0 = 0, k1 = 0, n0 = 0, n1 = 0;
+    if (rb < rend) {
+      bounds(rb, k0, k1);
+      bounds(rb + RP, n0, n1);
+      if (k0 < k1) load(k0, k1);
     }
-    if (k < k1) entry(col[k], (double)K[k], (double)M[k]);
-  }
+    for (; rb < rend; rb += RP) {
+      const int64_t row = rb + threadIdx.x / LPR, i = row * NC + lane;
+      const bool mine = row < rend && lane < NC;
+      Pair<VT> pv{};
+      if (DOT && mine) pv = ((const Pair<VT> *)p)[i];
+      ar = ai = 0.0;
+      const int64_t f0 = n0, f1 = n1;
+      if (k0 < k1) {
+#pragma unroll 1
+        for (int64_t kb = k0; kb < k1; kb += U * LPR)  // the row's lanes stay together
+          pass([&]() {
+            if (kb + U * LPR < k1) load(kb + U * LPR, k1);
+            else if (f0 < f1) load(f0, f1);
+          });
+      } else if (f0 < f1) {
+        load(f0, f1);
+      }
+      k0 = f0;
+      k1 = f1;
+      bounds(rb + 2 * RP, n0, n1);
 #pragma unroll
-  for (int off = LPR / 2; off > 0; off >>= 1)
-#pragma unroll
-    for (int c = 0; c < NC; c++) {
-      ar[c] += __shfl_xor(ar[c], off, LPR);
-      ai[c] += __shfl_xor(ai[c], off, LPR);
-    }
-  if (row < nne) {
-#pragma unroll
-    for (int c = 0; c < NC; c++) {
-      if (c % LPR == lane) {
-        y[2 * (row * NC + c)] = (VT)ar[c];
-        y[2 * (row * NC + c) + 1] = (VT)ai[c];
+      for (int off = LPR / 2; off >= NC; off >>= 1) {
+        ar += __shfl_xor(ar, off, LPR);
+        ai += __shfl_xor(ai, off, LPR);
+      }
+      if (mine) {
+        ((Pair<VT> *)y)[i] = Pair<VT>{(VT)ar, (VT)ai};
         if (DOT) {
-          const double pr = (double)p[2 * (row * NC + c)], pi = (double)p[2 * (row * NC + c) + 1];
-          dr[c] += pr * ar[c] - pi * ai[c];
-          di[c] += pr * ai[c] + pi * ar[c];
+          sr += (double)pv.x * ar - (double)pv.y * ai;
+          si += (double)pv.x * ai + (double)pv.y * ar;
         }
       }
     }
-  }
+    if (DOT)
+#pragma unroll
+      for (int c = 0; c < NC; c++) {
+        dr[c] = lane == c ? sr : 0.0;
+        di[c] = lane == c ? si : 0.0;
+      }
+  } else {
+    for (int64_t rb = wg * per; rb < rend; rb += RP) {
+      const int64_t row = rb + threadIdx.x / LPR;
+      double ar[NC], ai[NC];
+#pragma unroll
+      for (int c = 0; c < NC; c++) ar[c] = ai[c] = 0.0;
+      if (row < nne) {
+        const int64_t k1 = rowptr[row + 1];
+        // one entry of the lane: A_k x_col(k) accumulated into (ar, ai)
+        auto entry = [&](int64_t cc, double kv, double mv) {
+          const VT *xp = x + 2 * cc * NC;
+#pragma unroll
+          for (int c = 0; c < NC; c++) {
+            double vr = kv, vi = w.w[c] * mv;
+            if (C64) {
+              vr = (double)(float)vr;
+              vi = (double)(float)vi;
+            }
+            const double xr = (double)xp[2 * c], xi = (double)xp[2 * c + 1];
+            ar[c] += vr * xr - vi * xi;
+            ai[c] += vr * xi + vi * xr;
+          }
+        };
+        int64_t k = rowptr[row] + lane;
+        // two entries per lane in flight, accumulated in the same order
+        for (; k + LPR < k1; k += 2 * LPR) {
+          const int64_t c0 = col[k], c1 = col[k + LPR];
+          const double k0v = (double)K[k], m0v = (double)M[k], k1v = (double)K[k + LPR], m1v = (double)M[k + LPR];
+          entry(c0, k0v, m0v);
+          entry(c1, k1v, m1v);
+        }
+        if (k < k1) entry(col[k], (double)K[k], (double)M[k]);
+      }
+#pragma unroll
+      for (int off = LPR / 2; off > 0; off >>= 1)
+#pragma unroll
+        for (int c = 0; c < NC; c++) {
+          ar[c] += __shfl_xor(ar[c], off, LPR);
+          ai[c] += __shfl_xor(ai[c], off, LPR);
+        }
+      if (row < nne) {
+#pragma unroll
+        for (int c = 0; c < NC; c++) {
+          if (c % LPR == lane) {
+            y[2 * (row * NC + c)] = (VT)ar[c];
+            y[2 * (row * NC + c) + 1] = (VT)ai[c];
+            if (DOT) {
+              const double pr = (double)p[2 * (row * NC + c)], pi = (double)p[2 * (row * NC + c) + 1];
+              dr[c] += pr * ar[c] - pi * ai[c];
+              di[c] += pr * ai[c] + pi * ar[c];
+            }
+          }
+        }
+      }
+    }
   }
   if (DOT) {
     __shared__ double red[kBS / 64][NC][2];
@@ -144,12 +311,12 @@ __device__ __forceinline__ void spmv_body(int64_t nne, const int64_t *__restrict
   }
 }
 
-template <typename VT, typename MT, int NC, int LPR, bool C64, bool DOT>
+template <typename VT, typename KT, typename MT, int NC, int LPR, bool C64, bool DOT>
 __global__ __launch_bounds__(kBS) void k_spmv(int64_t nne, const int64_t *__restrict__ rowptr,
-                                              const int32_t *__restrict__ col, const MT *__restrict__ K,
+                                              const int32_t *__restrict__ col, const KT *__restrict__ K,
                                               const MT *__restrict__ M, ColW w, const VT *__restrict__ x,
                                               VT *__restrict__ y, const VT *__restrict__ p, double *__restrict__ part) {
-  spmv_body<VT, MT, NC, LPR, C64, DOT>(nne, rowptr, col, K, M, w, x, y, p, part);
+  spmv_body<VT, KT, MT, NC, LPR, C64, DOT>(nne, rowptr, col, K, M, w, x, y, p, part);
 }
 
 // ------------------------------------------------------- block reduction ----
@@ -181,15 +348,33 @@ __device__ inline void block_partials(double (&v)[NQ][NC][2], double *part) {
   }
 }
 
-// sum of block partials -> out[q][c][2]; one block of 1024 threads
+// sum of block partials -> out[q][c][2] by one block of whole waves.  With a
+// power of two of sums per block every thread walks the partials contiguously
+// (they stay in the same sum) and lanes of one sum are added by shuffles.
 template <int NC, int NQ>
 __device__ inline void reduce_partials(const double *part, int nblocks, double *out) {
+  constexpr int P = NQ * NC * 2;
   const int wv = threadIdx.x / 64, lane = threadIdx.x % 64, nw = blockDim.x / 64;
-  for (int pr = wv; pr < NQ * NC * 2; pr += nw) {
+  if constexpr ((P & (P - 1)) == 0 && P <= 64) {
+    __shared__ double red[16][P];
     double a = 0.0;
-    for (int b = lane; b < nblocks; b += 64) a += part[(int64_t)b * NQ * NC * 2 + pr];
-    for (int off = 32; off > 0; off >>= 1) a += __shfl_xor(a, off, 64);
-    if (lane == 0) out[pr] = a;
+#pragma unroll 8
+    for (int i = threadIdx.x; i < nblocks * P; i += blockDim.x) a += part[i];
+    for (int off = 32; off >= P; off >>= 1) a += __shfl_xor(a, off, 64);
+    if (lane < P) red[wv][lane] = a;
+    __syncthreads();
+    if ((int)threadIdx.x < P) {
+      a = red[0][threadIdx.x];
+      for (int v = 1; v < nw; v++) a += red[v][threadIdx.x];
+      out[threadIdx.x] = a;
+    }
+  } else {
+    for (int pr = wv; pr < P; pr += nw) {
+      double a = 0.0;
+      for (int b = lane; b < nblocks; b += 64) a += part[(int64_t)b * P + pr];
+      for (int off = 32; off > 0; off >>= 1) a += __shfl_xor(a, off, 64);
+      if (lane == 0) out[pr] = a;
+    }
   }
 }
 
@@ -380,6 +565,97 @@ __global__ __launch_bounds__(kBS) void k_cocg_upd2(int64_t nne, const ColState *
   }
 }
 
+// ------------------------------------- COCG updates from the diagonal -------
+// The FP64 recurrences form the Jacobi weights from the operator's diagonal (two
+// reals per DOF for all columns) instead of reading one complex weight per
+// column, and update x with the old p where p is read anyway: 9 vector passes
+// per iteration instead of 11 (8-node 64 x 64 x 48, four columns: 65 -> 57 us).
+__global__ void k_diag(int64_t n, const int64_t *diagpos, const double *K, const double *M, int unit, double *dg) {
+  const int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (r >= n) return;
+  const int64_t p = diagpos[r];
+  dg[2 * r] = unit ? 1.0 : p >= 0 ? K[p] : 0.0;
+  dg[2 * r + 1] = unit ? 0.0 : p >= 0 ? M[p] : 0.0;
+}
+
+// z = D^-1 r for a diagonal entry of K and M, as k_invdiag forms it
+template <bool C64>
+__device__ __forceinline__ void jacobi(const double *dg, double w, double rr, double ri, double &zr, double &zi) {
+  double dr = dg[0], di = w * dg[1];
+  if (C64) {
+    dr = (double)(float)dr;
+    di = (double)(float)di;
+  }
+  double qr = 1.0, qi = 0.0;
+  if (dr != 0.0 || di != 0.0) cdiv(1.0, 0.0, dr, di, qr, qi);
+  zr = qr * rr - qi * ri;
+  zi = qr * ri + qi * rr;
+}
+
+// r -= alpha q; partials rho' = r^T D^-1 r, |r|^2
+template <int NC, bool C64>
+__global__ __launch_bounds__(kBS) void k_cocg_step1(int64_t nne, const ColState *__restrict__ st, ColW w,
+                                                    double *__restrict__ r, const double *__restrict__ q,
+                                                    const double *__restrict__ dg, double *__restrict__ part) {
+  __shared__ double sa[NC][3];
+  if (threadIdx.x < NC) {
+    sa[threadIdx.x][0] = st[threadIdx.x].alpha_r;
+    sa[threadIdx.x][1] = st[threadIdx.x].alpha_i;
+    sa[threadIdx.x][2] = w.w[threadIdx.x];
+  }
+  __syncthreads();
+  double v[2][NC][2];
+  for (int a = 0; a < 2; a++)
+    for (int c = 0; c < NC; c++) v[a][c][0] = v[a][c][1] = 0.0;
+#pragma unroll 2
+  for (int64_t i = blockIdx.x * (int64_t)kBS + threadIdx.x; i < nne * NC; i += (int64_t)gridDim.x * kBS) {
+    const int c = (int)(i % NC);
+    const double alr = sa[c][0], ali = sa[c][1], qr = q[2 * i], qi = q[2 * i + 1];
+    const double rr = r[2 * i] - (alr * qr - ali * qi), ri = r[2 * i + 1] - (alr * qi + ali * qr);
+    r[2 * i] = rr;
+    r[2 * i + 1] = ri;
+    double zr, zi;
+    jacobi<C64>(dg + 2 * (i / NC), sa[c][2], rr, ri, zr, zi);
+#pragma unroll
+    for (int cc = 0; cc < NC; cc++)
+      if (cc == c) {
+        v[0][cc][0] += rr * zr - ri * zi;
+        v[0][cc][1] += rr * zi + ri * zr;
+        v[1][cc][0] += rr * rr + ri * ri;
+      }
+  }
+  block_partials<NC, 2>(v, part);
+}
+
+// x += alpha p; p = D^-1 r + beta p
+template <int NC, bool C64>
+__global__ __launch_bounds__(kBS) void k_cocg_step2(int64_t nne, const ColState *__restrict__ st, ColW w,
+                                                    double *__restrict__ x, const double *__restrict__ r,
+                                                    double *__restrict__ p, const double *__restrict__ dg) {
+  __shared__ double sa[NC][5];
+  if (threadIdx.x < NC) {
+    const ColState &s = st[threadIdx.x];
+    sa[threadIdx.x][0] = s.alpha_r;
+    sa[threadIdx.x][1] = s.alpha_i;
+    sa[threadIdx.x][2] = s.beta_r;
+    sa[threadIdx.x][3] = s.beta_i;
+    sa[threadIdx.x][4] = w.w[threadIdx.x];
+  }
+  __syncthreads();
+#pragma unroll 2
+  for (int64_t i = blockIdx.x * (int64_t)kBS + threadIdx.x; i < nne * NC; i += (int64_t)gridDim.x * kBS) {
+    const int c = (int)(i % NC);
+    const double alr = sa[c][0], ali = sa[c][1], br = sa[c][2], bi = sa[c][3];
+    const double pr = p[2 * i], pi = p[2 * i + 1];
+    x[2 * i] = x[2 * i] + alr * pr - ali * pi;
+    x[2 * i + 1] = x[2 * i + 1] + alr * pi + ali * pr;
+    double zr, zi;
+    jacobi<C64>(dg + 2 * (i / NC), sa[c][4], r[2 * i], r[2 * i + 1], zr, zi);
+    p[2 * i] = zr + br * pr - bi * pi;
+    p[2 * i + 1] = zi + br * pi + bi * pr;
+  }
+}
+
 // ------------------------------------------------------- persistent COCG ----
 // `iters` COCG iterations in one cooperative launch: the SpMV with its fused
 // p^T A p partials, alpha, the x/r update with its partials, beta and the p
@@ -403,7 +679,7 @@ __global__ __launch_bounds__(kBS) void k_cocg_persist(int iters, int64_t nne, co
   __syncthreads();
   const int nb = gridDim.x;
   for (int k = 0; k < iters; k++) {
-    spmv_body<double, double, NC, LPR, C64, true>(nne, rowptr, col, K, M, w, p, q, p, spart);
+    spmv_body<double, double, double, NC, LPR, C64, true>(nne, rowptr, col, K, M, w, p, q, p, spart);
     grid.sync();
     reduce_partials<NC, 1>(spart, nb, out1);
     __syncthreads();
@@ -876,15 +1152,20 @@ static int graph_block(Solver &S, GraphBlock &gb, int count, F &&iter) {
 }
 
 constexpr int kSpmvBlocks = 4096;
+// most workgroups an SpMV takes (sizes its partial sums)
 static int spmv_blocks(int64_t n) {
   int64_t b = (n + kBS / 16 - 1) / (kBS / 16);
   return (int)(b < kSpmvBlocks ? b : kSpmvBlocks);
+}
+// workgroups of this solver's SpMV: no more than its rows need, and eight waves
+// per SIMD at most, since one workgroup then adds up their partial sums
+static int spmv_grid(int64_t n, int lpr) {
+  return (int)std::min<int64_t>(spmv_blocks(n), std::min<int64_t>((n * lpr + kBS - 1) / kBS, 2048));
 }
 
 template <typename VT, typename MT, int NC, bool DOT>
 static void spmv_launch(const Solver &S, const MT *K, const MT *M, const VT *x, VT *y, const VT *p, double *part) {
   mvf_handle *h = S.h;
-  unsigned grid = (unsigned)spmv_blocks(S.n);
   SpmvTimer *tm = S.tm;
   if (tm && tm->on) {
     if (tm->used == SpmvTimer::kRing) tm->drain();
@@ -893,13 +1174,14 @@ static void spmv_launch(const Solver &S, const MT *K, const MT *M, const VT *x, 
   }
   // lanes per row: the autotuned choice for the FP64 operator, 16 otherwise
   const int lpr = sizeof(MT) == 8 ? S.lpr : 16;
+  const unsigned grid = (unsigned)spmv_grid(S.n, lpr);
 #define MVF_SPMV(L_)                                                                                             \
   do {                                                                                                           \
     if (S.c64)                                                                                                   \
-      hipLaunchKernelGGL((k_spmv<VT, MT, NC, L_, true, DOT>), dim3(grid), dim3(kBS), 0, h->stream, S.n,          \
-                         h->d_rowptr, h->d_col, K, M, S.w, x, y, p, part);                                       \
+      hipLaunchKernelGGL((k_spmv<VT, float, MT, NC, L_, true, DOT>), dim3(grid), dim3(kBS), 0, h->stream, S.n,   \
+                         h->d_rowptr, h->d_col, h->d_K32, M, S.w, x, y, p, part);                                \
     else                                                                                                         \
-      hipLaunchKernelGGL((k_spmv<VT, MT, NC, L_, false, DOT>), dim3(grid), dim3(kBS), 0, h->stream, S.n,         \
+      hipLaunchKernelGGL((k_spmv<VT, MT, MT, NC, L_, false, DOT>), dim3(grid), dim3(kBS), 0, h->stream, S.n,     \
                          h->d_rowptr, h->d_col, K, M, S.w, x, y, p, part);                                       \
   } while (0)
   if (sizeof(MT) == 8 && lpr == 4) MVF_SPMV(4);
@@ -1042,17 +1324,18 @@ static int run_cocg64(Solver &S, const mvf_solver_opts *o, const double *b, doub
   double *spart = part + (size_t)kRedBlocks * 3 * NC * 2;
   int pgrid = 0;
   if (persist) MVF_TRY(cocg_persist<NC>(S, true, pgrid, 0, x, r, p, q, invd, spart, part, st, o->tol));
-  if (o->precond == MVF_PC_JACOBI) {
-    if (S.c64)
+  // D^-1 per column for the start of the recurrences
+  auto fill_invd = [&]() {
+    if (o->precond != MVF_PC_JACOBI)
+      hipLaunchKernelGGL(k_unit_diag, dim3(grid1d(nv / 2, 256)), dim3(256), 0, h->stream, nv, invd);
+    else if (S.c64)
       hipLaunchKernelGGL((k_invdiag<NC, true>), dim3(grid1d(n, 256)), dim3(256), 0, h->stream, n, h->d_diagpos, h->d_K,
                          h->d_M, S.w, invd);
     else
       hipLaunchKernelGGL((k_invdiag<NC, false>), dim3(grid1d(n, 256)), dim3(256), 0, h->stream, n, h->d_diagpos,
                          h->d_K, h->d_M, S.w, invd);
-  } else {
-    hipLaunchKernelGGL(k_unit_diag, dim3(grid1d(nv / 2, 256)), dim3(256), 0, h->stream, nv, invd);
-  }
-  int nb = vec_blocks(n, NC), sb = spmv_blocks(n);
+  };
+  int nb = vec_blocks(n, NC), sb = spmv_grid(n, S.lpr);
   int it = 0, restarts = 0;
   ColState hs[NC];
   double res[NC];
@@ -1060,17 +1343,27 @@ static int run_cocg64(Solver &S, const mvf_solver_opts *o, const double *b, doub
   int rc = 0;
   while (!done) {
     // (re)start from the current x: r = b - A x
+    fill_invd();
     spmv_launch<double, double, NC, false>(S, h->d_K, h->d_M, x, q, nullptr, nullptr);
     hipLaunchKernelGGL((k_cocg_init<double, NC>), dim3(nb), dim3(kBS), 0, h->stream, n, b, q, invd, r, p, part);
     hipLaunchKernelGGL(k_cocg_fin_init<NC>, dim3(1), dim3(1024), 0, h->stream, part, nb, st);
+    // the iterations take the diagonal itself, in the same buffer
+    if (!persist)
+      hipLaunchKernelGGL(k_diag, dim3(grid1d(n, 256)), dim3(256), 0, h->stream, n, h->d_diagpos, h->d_K, h->d_M,
+                         o->precond == MVF_PC_JACOBI ? 0 : 1, invd);
     int since = 0;
     auto iter = [&]() {
       spmv_launch<double, double, NC, true>(S, h->d_K, h->d_M, p, q, p, spart);
       hipLaunchKernelGGL(k_cocg_alpha<NC>, dim3(1), dim3(1024), 0, h->stream, spart, sb, st);
-      hipLaunchKernelGGL((k_cocg_upd1<double, double, NC>), dim3(nb), dim3(kBS), 0, h->stream, n, st, x, r, p, q,
-                         invd, part);
+      if (S.c64)
+        hipLaunchKernelGGL((k_cocg_step1<NC, true>), dim3(nb), dim3(kBS), 0, h->stream, n, st, S.w, r, q, invd, part);
+      else
+        hipLaunchKernelGGL((k_cocg_step1<NC, false>), dim3(nb), dim3(kBS), 0, h->stream, n, st, S.w, r, q, invd, part);
       hipLaunchKernelGGL(k_cocg_beta<NC>, dim3(1), dim3(1024), 0, h->stream, part, nb, st, o->tol, 1);
-      hipLaunchKernelGGL((k_cocg_upd2<double, NC>), dim3(nb), dim3(kBS), 0, h->stream, n, st, r, p, invd);
+      if (S.c64)
+        hipLaunchKernelGGL((k_cocg_step2<NC, true>), dim3(nb), dim3(kBS), 0, h->stream, n, st, S.w, x, r, p, invd);
+      else
+        hipLaunchKernelGGL((k_cocg_step2<NC, false>), dim3(nb), dim3(kBS), 0, h->stream, n, st, S.w, x, r, p, invd);
     };
     while (it < o->maxit) {
       if (persist && since == 0) {
@@ -1147,7 +1440,7 @@ static int run_cocg_mixed(Solver &S, const mvf_solver_opts *o, const double *b, 
     hipLaunchKernelGGL((k_invdiag<NC, false>), dim3(grid1d(n, 256)), dim3(256), 0, h->stream, n, h->d_diagpos, h->d_K,
                        h->d_M, S.w, invd);
   MVF_HIP(h, hipMemsetAsync(x32, 0, nv * sizeof(float), h->stream));
-  int nb = vec_blocks(n, NC), sb = spmv_blocks(n);
+  int nb = vec_blocks(n, NC), sb = spmv_grid(n, 16);
   int it = 0, refinements = 0;
   ColState hs[NC];
   double res[NC];

@@ -136,3 +136,34 @@ def test_sixteen_frequencies_one_call(need_gpu):
     xref = np.stack([spla.splu(A).solve(b[d]) for d in range(2)])
     _check(A, b, xb[2 * i:2 * i + 2], xref)
     _check(A, b, x, xref)
+
+
+@pytest.mark.parametrize("matrix", ["c64ref", "fp64"])
+@pytest.mark.parametrize("nodes,sides,nf", [
+    (8, (5, 4, 3), 1),     # two columns, rows shorter than one pass of the lanes
+    (8, (11, 9, 7), 2),    # four columns, several workgroups
+    (20, (4, 3, 3), 1),    # ~84 entries per row: more than one pass at 4 and 8 lanes per row
+    (20, (4, 3, 3), 2),
+    (27, (3, 3, 2), 2),
+    (8, (5, 4, 3), 3),     # six columns padded to eight, one lane per entry
+])
+def test_cocg_columns_and_rows(nodes, sides, nf, matrix, need_gpu):
+    """The SpMV and the updates for every column count, short and long rows and
+    both matrix roundings: the residual of each column, formed on the host from
+    the entry list, is the tolerance of 1e-9 (times 1.1: the host's own sums of
+    ~100 products round at 1e-14)."""
+    freqs = tuple(20.0 * 3.0 ** k for k in range(nf))
+    m = M.random_small(nodes, *sides, seed=41, full_tensor=True, freqs=freqs)
+    g = GpuVfem(m, emulate=0)
+    info = g.solve_frequencies(freqs, method="cocg", matrix=matrix, tol=1e-9, maxit=20000, use_graph=nf == 2)
+    assert info["converged"], info
+    x, bb = g.solution(2 * nf), g.rhs(2 * nf)
+    for i in range(nf):
+        g2 = GpuVfem(m, emulate=0)
+        g2.set_frequency(i)
+        A, _ = reference_system(g2)
+        for d in range(2):
+            b = bb[2 * i + d]
+            r = np.linalg.norm(b - A @ x[2 * i + d]) / np.linalg.norm(b)
+            # the unrounded operator differs from the complex64 entry list by its rounding, 2^-24 relative
+            assert r <= (1.1e-9 if matrix == "c64ref" else 1e-5), (i, d, r)
