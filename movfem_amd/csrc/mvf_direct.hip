@@ -1226,6 +1226,7 @@ __global__ __launch_bounds__(768) void k_sv_fblock(const DNode *nodes, const int
   const DNode nd = nodes[lev[blockIdx.x]];
   const int64_t K1 = K0 + kOuter < nd.n1 ? K0 + kOuter : nd.n1;
   if (K0 + kNB >= K1) return;
+  constexpr int U = NC <= 4 ? 16 : 8;  // loads in flight per lane
   const int nb = (int)(K1 - K0);
   const int64_t m = nd.m;
   const double2 *T = fac + nd.fac + K0 * m + K0;
@@ -1242,12 +1243,12 @@ __global__ __launch_bounds__(768) void k_sv_fblock(const DNode *nodes, const int
     const double2 *V = T + (int64_t)(p + 16 * lq) * m + jc;
     if (p + kNB + wv * 16 < nb) {
 #pragma unroll
-      for (int r0 = 0; r0 < 16; r0 += 8) {
-        double2 v[8];
+      for (int r0 = 0; r0 < 16; r0 += U) {
+        double2 v[U];
 #pragma unroll
-        for (int u = 0; u < 8; u++) v[u] = V[(r0 + u) * m];
+        for (int u = 0; u < U; u++) v[u] = V[(r0 + u) * m];
 #pragma unroll
-        for (int u = 0; u < 8; u++)
+        for (int u = 0; u < U; u++)
 #pragma unroll
           for (int c = 0; c < NC; c++) cfma(acc[c], v[u], s[p + 16 * lq + r0 + u][c]);
       }
@@ -1280,6 +1281,7 @@ __global__ __launch_bounds__(256) void k_sv_frest(const DNode *nodes, const int3
   if (K0 >= nd.n1) return;
   const int64_t K1 = K0 + kOuter < nd.n1 ? K0 + kOuter : nd.n1, m = nd.m;
   if (K1 + (int64_t)blockIdx.x * 64 >= m) return;
+  constexpr int U = NC <= 4 ? 16 : 8;  // rows' loads in flight together
   const int nb = (int)(K1 - K0);
   __shared__ double2 s[kOuter][NC];
   for (int e = threadIdx.x; e < nb * NC; e += 256) s[e / NC][e % NC] = W[(nd.sv + K0) * NC + e];
@@ -1293,19 +1295,17 @@ __global__ __launch_bounds__(256) void k_sv_frest(const DNode *nodes, const int3
 #pragma unroll
     for (int c = 0; c < NC; c++) acc[c] = make_double2(0.0, 0.0);
     int r = ra;
-    for (; r + 8 <= rb; r += 8) {  // eight rows' loads in flight together
-      double2 v[8];
+    for (; r < rb; r += U) {  // rows past rb: the last row again, as zeros
+      double2 v[U];
 #pragma unroll
-      for (int u = 0; u < 8; u++) v[u] = V[(r + u) * m];
+      for (int u = 0; u < U; u++) v[u] = V[(r + u < rb ? r + u : rb - 1) * m];
 #pragma unroll
-      for (int u = 0; u < 8; u++)
+      for (int u = 0; u < U; u++) {
+        const int q = r + u < rb ? r + u : rb - 1;
+        const double2 e = r + u < rb ? v[u] : make_double2(0.0, 0.0);
 #pragma unroll
-        for (int c = 0; c < NC; c++) cfma(acc[c], v[u], s[r + u][c]);
-    }
-    for (; r < rb; r++) {
-      const double2 v = V[r * m];
-#pragma unroll
-      for (int c = 0; c < NC; c++) cfma(acc[c], v, s[r][c]);
+        for (int c = 0; c < NC; c++) cfma(acc[c], e, s[q][c]);
+      }
     }
 #pragma unroll
     for (int c = 0; c < NC; c++)
@@ -1375,12 +1375,14 @@ __global__ __launch_bounds__(256) void k_sv_diag(const DNode *nodes, const int2 
     if (r < w && g + 4 * i < NC) zb[(nd.pos0 + r0 + r) * NC + g + 4 * i] = z[i];
 }
 
-// backward, update columns: z[i] -= sum_j V[i][n1 + j] x2[j]; one wave per row
+// backward, update columns: z[i] -= sum_j V[i][n1 + j] x2[j]; one wave per row,
+// the gathers of several columns per lane in flight together
 template <int NC>
 __global__ __launch_bounds__(256) void k_sv_back(const DNode *nodes, const int32_t *lev, const int32_t *fpos,
                                                  const double2 *fac, double2 *zb) {
   const DNode nd = nodes[lev[blockIdx.y]];
   if (nd.n2 == 0) return;
+  constexpr int U = NC <= 4 ? 4 : 1;
   const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const double2 *T = fac + nd.fac;
   for (int64_t i = (int64_t)blockIdx.x * 4 + wv; i < nd.n1; i += (int64_t)gridDim.x * 4) {
@@ -1388,11 +1390,24 @@ __global__ __launch_bounds__(256) void k_sv_back(const DNode *nodes, const int32
 #pragma unroll
     for (int c = 0; c < NC; c++) acc[c] = make_double2(0.0, 0.0);
     const double2 *Yr = T + i * nd.m + nd.n1;
-    for (int64_t j = lane; j < nd.n2; j += 64) {
-      const double2 y = Yr[j];
-      const int64_t pj = fpos[nd.idx + nd.n1 + j];
+    for (int64_t j0 = lane; j0 < nd.n2; j0 += 64 * U) {
+      double2 y[U], z[U][NC];
+      int64_t pj[U];
 #pragma unroll
-      for (int c = 0; c < NC; c++) cfma(acc[c], y, zb[pj * NC + c]);
+      for (int u = 0; u < U; u++) {
+        const int64_t j = j0 + 64 * u < nd.n2 ? j0 + 64 * u : nd.n2 - 1;
+        const double2 t = Yr[j];
+        pj[u] = fpos[nd.idx + nd.n1 + j];
+        y[u] = j0 + 64 * u < nd.n2 ? t : make_double2(0.0, 0.0);
+      }
+#pragma unroll
+      for (int u = 0; u < U; u++)
+#pragma unroll
+        for (int c = 0; c < NC; c++) z[u][c] = zb[pj[u] * NC + c];
+#pragma unroll
+      for (int u = 0; u < U; u++)
+#pragma unroll
+        for (int c = 0; c < NC; c++) cfma(acc[c], y[u], z[u][c]);
     }
 #pragma unroll
     for (int c = 0; c < NC; c++)
@@ -1400,11 +1415,13 @@ __global__ __launch_bounds__(256) void k_sv_back(const DNode *nodes, const int32
         acc[c].x += __shfl_xor(acc[c].x, off, 64);
         acc[c].y += __shfl_xor(acc[c].y, off, 64);
       }
-    if (lane < NC) {
-      double2 &o = zb[(nd.pos0 + i) * NC + lane];
-      o.x -= acc[lane].x;
-      o.y -= acc[lane].y;
-    }
+#pragma unroll
+    for (int c = 0; c < NC; c++)
+      if (lane == c) {
+        double2 &o = zb[(nd.pos0 + i) * NC + c];
+        o.x -= acc[c].x;
+        o.y -= acc[c].y;
+      }
   }
 }
 
@@ -1448,7 +1465,8 @@ __global__ __launch_bounds__(256) void k_sv_brest(const DNode *nodes, const int3
 
 // backward inside an outer block: its panels from the last, z[r] -= sum_c
 // V[r][c] z[c] over the block's columns right of the panel; one workgroup per
-// front, four rows per wave
+// front, four rows per wave with sixteen lanes each (four shuffles per sum
+// instead of the six of a whole wave per row)
 template <int NC>
 __global__ __launch_bounds__(1024) void k_sv_bblock(const DNode *nodes, const int32_t *lev, int64_t K0,
                                                     const double2 *fac, double2 *zb) {
@@ -1462,37 +1480,44 @@ __global__ __launch_bounds__(1024) void k_sv_bblock(const DNode *nodes, const in
   __shared__ double2 s[kOuter][NC];
   for (int e = threadIdx.x; e < nb * NC; e += 1024) s[e / NC][e % NC] = Zb[e];
   __syncthreads();
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, l16 = lane & 15;
   for (int p = (nb - 1) / kNB - 1; p >= 0; p--) {
     const int j0 = (p + 1) * kNB;
+    const int r = p * kNB + wv * 4 + (lane >> 4);
+    constexpr int QB = NC <= 4 ? 12 : 4;  // loads in flight
+    double2 acc[NC];
 #pragma unroll
-    for (int u = 0; u < 4; u++) {
-      const int r = p * kNB + wv * 4 + u;
-      double2 v[3];
+    for (int c = 0; c < NC; c++) acc[c] = make_double2(0.0, 0.0);
+#pragma unroll 1
+    for (int q0 = 0; q0 < 12; q0 += QB) {  // at most three panels right of this one
+      double2 v[QB];
 #pragma unroll
-      for (int q = 0; q < 3; q++) v[q] = T[(int64_t)r * m + (j0 + 64 * q + lane < nb ? j0 + 64 * q + lane : nb - 1)];
-      double2 acc[NC];
+      for (int q = 0; q < QB; q++) {
+        const int j = j0 + 16 * (q0 + q) + l16;
+        v[q] = make_double2(0.0, 0.0);
+        if (j0 + 16 * (q0 + q) < nb) v[q] = T[(int64_t)r * m + (j < nb ? j : nb - 1)];
+      }
 #pragma unroll
-      for (int c = 0; c < NC; c++) acc[c] = make_double2(0.0, 0.0);
+      for (int q = 0; q < QB; q++) {
+        const int j = j0 + 16 * (q0 + q) + l16;
+        if (j < nb)
 #pragma unroll
-      for (int q = 0; q < 3; q++)
-        if (j0 + 64 * q + lane < nb)
-#pragma unroll
-          for (int c = 0; c < NC; c++) cfma(acc[c], v[q], s[j0 + 64 * q + lane][c]);
-#pragma unroll
-      for (int c = 0; c < NC; c++)
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) {
-          acc[c].x += __shfl_xor(acc[c].x, off, 64);
-          acc[c].y += __shfl_xor(acc[c].y, off, 64);
-        }
-#pragma unroll
-      for (int c = 0; c < NC; c++)
-        if (lane == c) {
-          s[r][c].x -= acc[c].x;
-          s[r][c].y -= acc[c].y;
-        }
+          for (int c = 0; c < NC; c++) cfma(acc[c], v[q], s[j][c]);
+      }
     }
+#pragma unroll
+    for (int c = 0; c < NC; c++)
+#pragma unroll
+      for (int off = 8; off > 0; off >>= 1) {
+        acc[c].x += __shfl_xor(acc[c].x, off, 16);
+        acc[c].y += __shfl_xor(acc[c].y, off, 16);
+      }
+#pragma unroll
+    for (int c = 0; c < NC; c++)
+      if (l16 == c) {
+        s[r][c].x -= acc[c].x;
+        s[r][c].y -= acc[c].y;
+      }
     __syncthreads();
   }
   for (int e = threadIdx.x; e < nb * NC; e += 1024) Zb[e] = s[e / NC][e % NC];
