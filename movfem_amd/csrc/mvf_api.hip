@@ -180,6 +180,7 @@ void mvf_free(mvf_handle *h) {
   for (void *p : h->gv_pin)
     if (p) (void)hipHostFree(p);
   direct_free(h);
+  spmv_timer_free(h);
   if (h->stream) (void)hipStreamDestroy(h->stream);
   delete h;
 }
@@ -1018,23 +1019,23 @@ int mvf_readout(mvf_handle *h, const double *x, int32_t f, int32_t ke_top, int32
   }
   double *es = nullptr, *hs = nullptr;
   const size_t nf = (size_t)2 * g.npt * 3 * 2;
-  int rc = dalloc(h, &es, nf);
-  if (!rc) rc = dalloc(h, &hs, nf);
+  int rc = ds.alloc(h, &es, nf);
+  if (!rc) rc = ds.alloc(h, &hs, nf);
   if (!rc) rc = node_fields(h, x ? dx : h->d_x, ncol, col0, omega, es, hs);
   if (!rc && nrx > 0) {
     double *drx = nullptr, *dry = nullptr, *doe = nullptr, *doh = nullptr, *doz = nullptr, *drho = nullptr,
            *dphi = nullptr, *delev = nullptr;
     int32_t *die = nullptr, *dje = nullptr;
-    rc = dalloc(h, &drx, nrx);
-    if (!rc) rc = dalloc(h, &dry, nrx);
-    if (!rc) rc = dalloc(h, &die, nrx);
-    if (!rc) rc = dalloc(h, &dje, nrx);
-    if (!rc) rc = dalloc(h, &doe, (size_t)nrx * 12);
-    if (!rc) rc = dalloc(h, &doh, (size_t)nrx * 12);
-    if (!rc) rc = dalloc(h, &doz, (size_t)nrx * 8);
-    if (!rc) rc = dalloc(h, &drho, (size_t)nrx * 4);
-    if (!rc) rc = dalloc(h, &dphi, (size_t)nrx * 4);
-    if (!rc) rc = dalloc(h, &delev, (size_t)nrx);
+    rc = ds.alloc(h, &drx, nrx);
+    if (!rc) rc = ds.alloc(h, &dry, nrx);
+    if (!rc) rc = ds.alloc(h, &die, nrx);
+    if (!rc) rc = ds.alloc(h, &dje, nrx);
+    if (!rc) rc = ds.alloc(h, &doe, (size_t)nrx * 12);
+    if (!rc) rc = ds.alloc(h, &doh, (size_t)nrx * 12);
+    if (!rc) rc = ds.alloc(h, &doz, (size_t)nrx * 8);
+    if (!rc) rc = ds.alloc(h, &drho, (size_t)nrx * 4);
+    if (!rc) rc = ds.alloc(h, &dphi, (size_t)nrx * 4);
+    if (!rc) rc = ds.alloc(h, &delev, (size_t)nrx);
     if (!rc) {
       hipError_t e = hipMemcpy(drx, rx, 8 * nrx, hipMemcpyHostToDevice);
       if (e == hipSuccess) e = hipMemcpy(dry, ry, 8 * nrx, hipMemcpyHostToDevice);
@@ -1058,9 +1059,9 @@ int mvf_readout(mvf_handle *h, const double *x, int32_t f, int32_t ke_top, int32
   }
   if (!rc && (node_z || node_rho || node_phi)) {
     double *dz = nullptr, *drh = nullptr, *dph = nullptr;
-    rc = dalloc(h, &dz, (size_t)g.npt * 8);
-    if (!rc) rc = dalloc(h, &drh, (size_t)g.npt * 4);
-    if (!rc) rc = dalloc(h, &dph, (size_t)g.npt * 4);
+    rc = ds.alloc(h, &dz, (size_t)g.npt * 8);
+    if (!rc) rc = ds.alloc(h, &drh, (size_t)g.npt * 4);
+    if (!rc) rc = ds.alloc(h, &dph, (size_t)g.npt * 4);
     if (!rc) rc = node_impedance(h, es, hs, omega, dz, drh, dph);
     if (!rc) {
       hipError_t e = hipStreamSynchronize(h->stream);

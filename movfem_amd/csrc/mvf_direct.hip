@@ -125,6 +125,7 @@ struct DirectPlan {
   double t_symbolic = 0.0, t_factor = 0.0;
   int64_t factorizations = 0;
   // GEMM launches of the last factorization: HIP-event time and algorithmic flops
+  struct GemmTimer *timer = nullptr;
   double gemm_ms = 0.0, gemm_flops = 0.0;
   int64_t gemm_launches = 0;
 };
@@ -167,8 +168,13 @@ struct GemmTimer {
     }
     used -= count;
   }
-  void destroy() {
-    drain();
+  void reset() {
+    used = 0;
+    ms = flops = 0.0;
+    launches = 0;
+    for (int q = 0; q < 3; q++) mode_ms[q] = mode_fl[q] = 0.0;
+  }
+  ~GemmTimer() {
     for (int i = 0; i < kRing; i++) {
       (void)hipEventDestroy(ev[i][0]);
       (void)hipEventDestroy(ev[i][1]);
@@ -1550,6 +1556,7 @@ void direct_free(mvf_handle *h) {
   if (P->ev_fork) (void)hipEventDestroy(P->ev_fork);
   if (P->ev_join) (void)hipEventDestroy(P->ev_join);
   if (P->st2) (void)hipStreamDestroy(P->st2);
+  delete P->timer;
   delete P;
   h->direct = nullptr;
 }
@@ -1667,8 +1674,12 @@ static int direct_factor(mvf_handle *h, double w, int c64, int f32 = 0) {
   const double big = P->maxK + w * P->maxM;
   const double tiny = 1e-14 * big;
   MVF_HIP(h, hipMemsetAsync(P->d_npert, 0, sizeof(int), st));
-  GemmTimer *gt_ = new GemmTimer();
-  gt_->init();
+  if (!P->timer) {
+    P->timer = new GemmTimer();
+    P->timer->init();
+  }
+  GemmTimer *gt_ = P->timer;
+  gt_->reset();
   auto gemm_begin = [&](double flops, int mode, hipStream_t s) {
     if (gt_->used == GemmTimer::kRing) gt_->drain(GemmTimer::kRing / 2);
     gt_->fl[gt_->used] = flops;
@@ -1793,7 +1804,7 @@ static int direct_factor(mvf_handle *h, double w, int c64, int f32 = 0) {
     }
   }
   MVF_HIP(h, hipStreamSynchronize(st));
-  gt_->destroy();
+  gt_->drain();
   if (h->verbose)
     for (int q = 0; q < 3; q++)
       if (gt_->mode_ms[q] > 0)
@@ -1802,9 +1813,9 @@ static int direct_factor(mvf_handle *h, double w, int c64, int f32 = 0) {
   P->gemm_ms = gt_->ms;
   P->gemm_flops = gt_->flops;
   P->gemm_launches = gt_->launches;
-  delete gt_;
   int np = 0;
-  MVF_HIP(h, hipMemcpy(&np, P->d_npert, sizeof(int), hipMemcpyDeviceToHost));
+  MVF_HIP(h, hipMemcpyAsync(&np, P->d_npert, sizeof(int), hipMemcpyDeviceToHost, st));
+  MVF_HIP(h, hipStreamSynchronize(st));
   P->npert = np;
   P->factored = 1;
   P->omega = w;
@@ -2052,7 +2063,8 @@ static int run_gmres_direct(Solver &S, const mvf_solver_opts *o, const double *b
     MVF_TRY(true_resid<NC>(S, b, x, (double *)Z, part + (size_t)(mres + 1) * std::max(nbk, kRedBlocks) * NC * 2,
                            dnorm, res, (double *)r));
     double hn[2 * NC];
-    MVF_HIP(h, hipMemcpy(hn, dnorm, sizeof(hn), hipMemcpyDeviceToHost));
+    MVF_HIP(h, hipMemcpyAsync(hn, dnorm, sizeof(hn), hipMemcpyDeviceToHost, st));
+    MVF_HIP(h, hipStreamSynchronize(st));
     bool ok = true;
     for (int c = 0; c < S.ncol; c++) ok &= res[c] <= o->tol;
     if (ok) break;

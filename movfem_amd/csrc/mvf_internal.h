@@ -6,6 +6,8 @@
 #include <cstdint>
 #include <cstdio>
 #include <string>
+#include <algorithm>
+#include <mutex>
 #include <vector>
 
 #include "../../include/movfem_gpu.h"
@@ -91,6 +93,90 @@ __device__ inline int64_t xcd_block(int64_t b, int64_t nb) {
   return x * q + (x < rm ? x : rm) + i;
 }
 
+// Device buffers a handle's calls took and gave back, kept for its next calls:
+// hipMalloc and hipFree cost 50-300 us each and wait for the whole device, other
+// handles' streams included.  A handle's work is ordered on its stream, so a
+// buffer can be handed out again while earlier work on it is queued.  At most
+// kMax bytes are kept (the oldest go first), and an allocation that fails
+// anywhere empties every pool and is tried again.
+struct BufPool {
+  static constexpr size_t kMax = (size_t)1 << 30;
+  struct Buf {
+    void *p;
+    size_t bytes;
+  };
+  std::mutex mu;
+  std::vector<Buf> idle;  // oldest first
+  size_t held = 0;
+  struct Registry {
+    std::mutex mu;
+    std::vector<BufPool *> pools;
+  };
+  static Registry &registry() {
+    static Registry *r = new Registry();  // never destroyed: handles may outlive static destruction
+    return *r;
+  }
+  BufPool() {
+    std::lock_guard<std::mutex> g(registry().mu);
+    registry().pools.push_back(this);
+  }
+  BufPool(const BufPool &) = delete;
+  BufPool &operator=(const BufPool &) = delete;
+  ~BufPool() {
+    {
+      std::lock_guard<std::mutex> g(registry().mu);
+      auto &v = registry().pools;
+      v.erase(std::remove(v.begin(), v.end(), this), v.end());
+    }
+    trim();
+  }
+  // the smallest kept buffer of at least `bytes` and at most twice that
+  Buf take(size_t bytes) {
+    std::lock_guard<std::mutex> g(mu);
+    size_t best = idle.size();
+    for (size_t i = 0; i < idle.size(); i++)
+      if (idle[i].bytes >= bytes && idle[i].bytes <= std::max<size_t>(2 * bytes, 4096) &&
+          (best == idle.size() || idle[i].bytes < idle[best].bytes))
+        best = i;
+    if (best == idle.size()) return Buf{nullptr, 0};
+    const Buf b = idle[best];
+    idle.erase(idle.begin() + best);
+    held -= b.bytes;
+    return b;
+  }
+  void give(Buf b) {
+    std::vector<Buf> out;
+    {
+      std::lock_guard<std::mutex> g(mu);
+      if (b.bytes > kMax) {
+        out.push_back(b);
+      } else {
+        while (held + b.bytes > kMax) {
+          held -= idle.front().bytes;
+          out.push_back(idle.front());
+          idle.erase(idle.begin());
+        }
+        idle.push_back(b);
+        held += b.bytes;
+      }
+    }
+    for (const Buf &o : out) (void)hipFree(o.p);
+  }
+  void trim() {
+    std::vector<Buf> out;
+    {
+      std::lock_guard<std::mutex> g(mu);
+      out.swap(idle);
+      held = 0;
+    }
+    for (const Buf &o : out) (void)hipFree(o.p);  // waits for the work queued on it
+  }
+  static void trim_all() {
+    std::lock_guard<std::mutex> g(registry().mu);
+    for (BufPool *q : registry().pools) q->trim();
+  }
+};
+
 }  // namespace mvf
 
 struct mvf_handle {
@@ -173,6 +259,9 @@ struct mvf_handle {
   std::vector<double> last_freqs;
   // scratch
   std::vector<void *> owned;
+  mvf::BufPool pool;
+  // event ring of the SpMV timer (mvf_solver.hip)
+  void *spmv_timer = nullptr;
 };
 
 namespace mvf {
@@ -208,6 +297,11 @@ inline int dalloc(mvf_handle *h, T **p, size_t n) {
   void *q = nullptr;
   size_t bytes = (n ? n : 1) * sizeof(T);
   hipError_t e = hipMalloc(&q, bytes);
+  if (e == hipErrorOutOfMemory) {
+    (void)hipGetLastError();
+    BufPool::trim_all();
+    e = hipMalloc(&q, bytes);
+  }
   if (e != hipSuccess)
     return set_err(h, MVF_E_MEMORY, "hipMalloc(%zu bytes) failed: %s", bytes, hipGetErrorString(e));
   *p = (T *)q;
@@ -221,26 +315,41 @@ inline void dfree(void *p) {
 // Temporary device buffers of one call: whatever is allocated through it is
 // freed when the call returns, on every return path (errors included).
 struct DevScope {
-  std::vector<void *> bufs;
+  mvf_handle *h = nullptr;
+  std::vector<BufPool::Buf> bufs;
   DevScope() = default;
   DevScope(const DevScope &) = delete;
   DevScope &operator=(const DevScope &) = delete;
+  // back to the handle's pool, once the work queued on them is done: a call
+  // returns with its device work finished
   ~DevScope() {
-    for (void *p : bufs)
-      if (p) (void)hipFree(p);
+    if (!h) return;
+    (void)hipStreamSynchronize(h->stream);
+    for (const BufPool::Buf &b : bufs) h->pool.give(b);
   }
   template <typename T>
-  int alloc(mvf_handle *h, T **p, size_t n) {
-    int rc = dalloc(h, p, n);
-    if (!rc) bufs.push_back((void *)*p);
-    return rc;
+  int alloc(mvf_handle *hd, T **p, size_t n) {
+    const size_t bytes = (n ? n : 1) * sizeof(T);
+    BufPool::Buf b = hd->pool.take(bytes);
+    if (!b.p) {
+      T *q = nullptr;
+      MVF_TRY(dalloc(hd, &q, n));
+      b = BufPool::Buf{(void *)q, bytes};
+    }
+    h = hd;
+    bufs.push_back(b);
+    *p = (T *)b.p;
+    return 0;
   }
-  // free one buffer before the call ends (lowers the peak)
+  // give one buffer back before the call ends (lowers the peak; later work of
+  // this handle is ordered after what is queued on it)
   void drop(void *p) {
-    if (!p) return;
-    for (auto &q : bufs)
-      if (q == p) q = nullptr;
-    (void)hipFree(p);
+    for (size_t i = 0; p && i < bufs.size(); i++)
+      if (bufs[i].p == p) {
+        h->pool.give(bufs[i]);
+        bufs.erase(bufs.begin() + i);
+        return;
+      }
   }
 };
 
@@ -258,6 +367,7 @@ int element_rhs_range(mvf_handle *h, double omega, int first_flags, int64_t e0, 
 int assemble_rhs(mvf_handle *h, const double *d_be, double *d_b, int ncol, int col0);
 int update_sigma(mvf_handle *h, double omega);
 void direct_free(mvf_handle *h);
+void spmv_timer_free(mvf_handle *h);
 int node_table(mvf_handle *h);
 int node_fields(mvf_handle *h, const double *x, int ncol, int col0, double omega, double *es, double *hs);
 int problem_fields(mvf_handle *h, double omega, double *ep, double *hp, double *src);

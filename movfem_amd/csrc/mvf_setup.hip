@@ -292,6 +292,7 @@ int setup_pattern(mvf_handle *h) {
     // (32 bytes per pair) at once: by rows when that exceeds a quarter of the
     // free memory, or when MVF_SETUP says so
     size_t fr = 0, tot = 0;
+    BufPool::trim_all();  // buffers kept for reuse count as free
     (void)hipMemGetInfo(&fr, &tot);
     const char *sv = getenv("MVF_SETUP");
     h->setup_rows = (sv && strcmp(sv, "rows") == 0) ? 1

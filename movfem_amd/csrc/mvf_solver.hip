@@ -1050,14 +1050,20 @@ struct SpmvTimer {
     }
     used = 0;
   }
-  void destroy() {
-    if (!on) return;
-    drain();
-    for (int i = 0; i < kRing; i++) {
-      (void)hipEventDestroy(ev[i][0]);
-      (void)hipEventDestroy(ev[i][1]);
+  // counters back to zero for the next solve; the events stay
+  void reset() {
+    used = 0;
+    for (int k = 0; k < 2; k++) {
+      launches[k] = 0;
+      ms[k] = 0;
     }
-    on = false;
+  }
+  ~SpmvTimer() {
+    if (on)
+      for (int i = 0; i < kRing; i++) {
+        (void)hipEventDestroy(ev[i][0]);
+        (void)hipEventDestroy(ev[i][1]);
+      }
   }
 };
 
@@ -1760,8 +1766,12 @@ static int tune_lpr(Solver &S) {
 template <int NC>
 static int solve_nc(mvf_handle *h, const double *omegas, int ncol, const mvf_solver_opts *o, const double *b,
                     double *x, mvf_solve_info *info, double *alpha_out = nullptr) {
-  SpmvTimer *tm = new SpmvTimer();
-  tm->init();
+  SpmvTimer *tm = (SpmvTimer *)h->spmv_timer;
+  if (!tm) {
+    h->spmv_timer = tm = new SpmvTimer();
+    tm->init();
+  }
+  tm->reset();
   Solver S{h, ncol, {}, o->matrix == MVF_MATRIX_C64REF, 16, (int64_t)h->nne, tm};
   for (int c = 0; c < NC; c++) S.w.w[c] = c < ncol ? (double)(float)omegas[c] : 0.0;
   int rc = h->autotune ? tune_lpr<NC>(S) : 0;
@@ -1771,7 +1781,7 @@ static int solve_nc(mvf_handle *h, const double *omegas, int ncol, const mvf_sol
   else if (o->precision == MVF_PREC_MIXED) rc = run_cocg_mixed<NC>(S, o, b, x, info);
   else if (o->method == MVF_KRYLOV_BICGSTAB) rc = run_bicgstab<NC>(S, o, b, x, info);
   else rc = run_cocg64<NC>(S, o, b, x, info);
-  tm->destroy();
+  tm->drain();
   const double n = (double)h->nne, nnz = (double)h->nnz;
   for (int k = 0; k < 2; k++) {
     info->spmv_launches[k] = tm->launches[k];
@@ -1783,8 +1793,12 @@ static int solve_nc(mvf_handle *h, const double *omegas, int ncol, const mvf_sol
   info->spmv_bytes[1] = nnz * (4 + 4 + 4) + n * (8 + NC * (8 + 8));
   info->spmv_ncol = NC;
   info->spmv_lpr = S.lpr;
-  delete tm;
   return rc;
+}
+
+void spmv_timer_free(mvf_handle *h) {
+  delete (SpmvTimer *)h->spmv_timer;
+  h->spmv_timer = nullptr;
 }
 
 // b, x: device [nne][ncol_pad] with ncol_pad in {2,4,8,16}

@@ -111,3 +111,28 @@ def test_persistent_cocg(need_gpu):
         assert ip["converged"] and max(ip["true_resid"][:2]) <= 1e-10 and ip["graph_launches"] > 0
         assert d <= 1e-8
         g.close()
+
+
+@pytest.mark.parametrize("method,precond", [("cocg", "jacobi"), ("gmres", "direct")])
+def test_reused_buffers(method, precond, need_gpu):
+    """Work buffers a handle keeps between calls: calls with one and three
+    frequencies (other buffer sizes) in turn on two handles repeat the first
+    results bit for bit, readout included, and closing the handles gives the
+    memory back."""
+    import torch
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    freqs = (20.0, 50.0, 90.0)
+    gs = [GpuVfem(M.random_small(n, 5, 4, 4, seed=51, full_tensor=True, freqs=freqs), emulate=0) for n in (8, 20)]
+    first = {}
+    for _ in range(3):
+        for nf in (1, 3):
+            for i, g in enumerate(gs):
+                g.assemble()
+                g.solve_frequencies(freqs[:nf], method=method, precond=precond, tol=1e-10, maxit=20000)
+                got = [g.solution(2 * nf)] + [np.asarray(v) for v in g.readout(None, f=0)[:2]]
+                for a, b in zip(first.setdefault((nf, i), got), got):
+                    assert np.array_equal(a, b)
+    for g in gs:
+        g.close()
+    assert torch.cuda.mem_get_info()[0] >= before - (64 << 20)
