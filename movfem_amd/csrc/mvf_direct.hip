@@ -457,20 +457,16 @@ static int build_plan_host(DirectPlan &P, int nx, int ny, int nz, int me, const 
 __device__ __forceinline__ double2 cmul(double2 a, double2 b) {
   return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
 }
-// c -= a * b
+// c -= a * b, four fused multiply-adds (written as a difference of products it
+// takes six operations)
 __device__ __forceinline__ void cfms(double2 &c, double2 a, double2 b) {
-  c.x -= a.x * b.x - a.y * b.y;
-  c.y -= a.x * b.y + a.y * b.x;
+  c.x = fma(a.y, b.y, fma(-a.x, b.x, c.x));
+  c.y = fma(-a.y, b.x, fma(-a.x, b.y, c.y));
 }
 // c += a * b
 __device__ __forceinline__ void cfma(double2 &c, double2 a, double2 b) {
-  c.x += a.x * b.x - a.y * b.y;
-  c.y += a.x * b.y + a.y * b.x;
-}
-// c += conj(a) * b
-__device__ __forceinline__ void cfmac(double2 &c, double2 a, double2 b) {
-  c.x += a.x * b.x + a.y * b.y;
-  c.y += a.x * b.y - a.y * b.x;
+  c.x = fma(-a.y, b.y, fma(a.x, b.x, c.x));
+  c.y = fma(a.y, b.x, fma(a.x, b.y, c.y));
 }
 __device__ __forceinline__ int64_t imin(int64_t a, int64_t b) { return a < b ? a : b; }
 // accumulator of v_mfma_f64_16x16x4f64
@@ -865,8 +861,8 @@ __global__ __launch_bounds__(256) void k_fa_prow(const DNode *nodes, const int32
 #pragma unroll
       for (int v2 = 0; v2 <= v; v2++) {  // rows lk + 4 v2 < r (Us is zero from r on)
         const double2 u = Us[b][r][lk + 4 * v2];
-        zr[b][v2] -= u.x * s.x - u.y * s.y;
-        zi[b][v2] -= u.x * s.y + u.y * s.x;
+        zr[b][v2] = fma(u.y, s.y, fma(-u.x, s.x, zr[b][v2]));
+        zi[b][v2] = fma(-u.y, s.x, fma(-u.x, s.y, zi[b][v2]));
       }
     }
   }
