@@ -11,7 +11,7 @@ and top 4 cells.  Inputs are synthetic and resident in HBM before timing.
 One step = one frequency-model solve, the reference's unit of work per pass of
 its frequency loop (MoVFEM_3DMT.f90:62-143): re-integrate every element's K
 and M on the device and re-assemble them (global_vfem's element loop), the
-device RHS of that frequency, one numeric multifrontal LU factorization (FP64,
+device RHS of that frequency, one numeric multifrontal factorization (FP64,
 nested dissection) of the operator and right-preconditioned FP64 GMRES to a
 true relative residual <= 1e-8 for both polarizations (the reference factors
 every frequency with MUMPS, MoVFEM_3DMT.f90:113-115).  Step k solves frequency

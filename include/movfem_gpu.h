@@ -158,7 +158,7 @@ enum { MVF_KRYLOV_COCG = 0, MVF_KRYLOV_BICGSTAB = 1, MVF_KRYLOV_GMRES = 2 };
  * factorization, FP64 arithmetic between the roundings), FP64 GMRES outside */
 enum { MVF_PREC_FP64 = 0, MVF_PREC_MIXED = 1 };
 enum { MVF_MATRIX_C64REF = 0, MVF_MATRIX_FP64 = 1 };/* which operator the residual is judged on */
-/* MVF_PC_DIRECT: multifrontal LU (FP64, nested dissection of the element box)
+/* MVF_PC_DIRECT: multifrontal block LDL^T (FP64, nested dissection of the element box)
  * of the operator at the geometric mean of the batch's frequencies, with a small imaginary
  * shift on the diagonal of massless (all-air) DOFs; the outer method is then
  * right-preconditioned GMRES on the unshifted operator whatever `method` says.

@@ -113,7 +113,7 @@ def test_direct_frequency_sweep(need_gpu):
 def test_direct_lookahead_fronts(need_gpu):
     """20-node 14 x 14 x 11 GPML model whose largest fronts own 974 DOFs:
     four outer blocks of 256, so the factorization overlaps the trailing
-    part of each outer LU update and of each outer Y update with the next
+    part of each outer update with the next
     block's panels on its second stream, and the fronts above 512 run the
     128 x 64 three-product tiles.  An error in either split or in the stream
     ordering corrupts the factor that preconditions GMRES: the bar is the
