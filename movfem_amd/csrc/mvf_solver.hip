@@ -1787,9 +1787,9 @@ static int solve_nc(mvf_handle *h, const double *omegas, int ncol, const mvf_sol
     info->spmv_launches[k] = tm->launches[k];
     info->spmv_ms[k] = tm->ms[k];
   }
-  // algorithmic bytes: K, M and column index per entry, row pointer per row,
-  // x read once and y written once per column
-  info->spmv_bytes[0] = nnz * (8 + 8 + 4) + n * (8 + NC * (16 + 16));
+  // algorithmic bytes: K (fl32(K) for the complex64 operator), M and column index
+  // per entry, row pointer per row, x read once and y written once per column
+  info->spmv_bytes[0] = nnz * ((S.c64 ? 4 : 8) + 8 + 4) + n * (8 + NC * (16 + 16));
   info->spmv_bytes[1] = nnz * (4 + 4 + 4) + n * (8 + NC * (8 + 8));
   info->spmv_ncol = NC;
   info->spmv_lpr = S.lpr;
