@@ -367,6 +367,7 @@ int mvf_init(const mvf_grid *grid, const mvf_model *model, const mvf_bc *bc, con
   h->t_setup[2] = t4 - t3;
   h->t_setup[3] = t5 - t4;
   (void)t0;
+  h->pool.trim();  // no later call takes buffers of the setup's sizes
   return 0;
 }
 
