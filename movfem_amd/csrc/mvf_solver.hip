@@ -79,43 +79,46 @@ struct Pair {
 // entries per lane loaded together in one pass over a row: 33 entries of an
 // 8-node row are one pass of 8 lanes x 5, ~84 of a 20-node row one of 16 x 6
 template <int LPR>
-constexpr int spmv_unroll() {
+__host__ __device__ constexpr int spmv_unroll() {
   return LPR <= 8 ? 5 : LPR <= 16 ? 6 : 4;
 }
 
 // y = A x (columns 0..NC-1); LPR lanes share a row.  With DOT, block partials
-// of p^T y (bilinear) are written to part[block][c].  The rate is set by the
-// gathers of x (NC x 16 bytes per entry, three to four times the operator's own
-// bytes) rather than by HBM.  With two or four columns each lane loads its own
-// entries, then each group of NC lanes walks the group's entries together, lane
-// c taking column c: a gather reads whole NC x 16 byte runs and a lane keeps one
-// column's sum, against one lane reading all columns of its entry (64 cache
-// lines per load instruction, four sums per lane).  All entries of a pass and
-// then all their x are loaded before the first product, from clamped addresses,
-// the entries past the row as zeros, and the next row's entries are loaded
-// before the current row's are summed.  With C64 the caller passes fl32(K), which
-// is what the rounding makes of K, at half its bytes.  8-node 64 x 64 x 48, four
-// columns, with the dot product: 170 us one lane per entry, 156 us grouped, 130
-// us with the next row's loads ahead; capping the registers for a third wave per
-// SIMD spills and takes twice the time.
-template <typename VT, typename KT, typename MT, int NC, int LPR, bool C64, bool DOT>
+// of p^T y (bilinear) are written to part[block][c].  With C64 the caller may pass
+// fl32(K), which is what the rounding makes of K, at half its bytes.  The rate is
+// set by the gathers of x (NC x 16 bytes per entry, three to four times the
+// operator's own bytes) rather than by HBM.
+//
+// Plain form: a lane reads all columns of its entry, two entries in flight, and
+// the workgroups stride over the rows.
+// GRP (two or four columns): each lane loads its own entries, then each group of
+// NC lanes walks the group's entries together, lane c taking column c: a gather
+// reads whole NC x 16 byte runs and a lane keeps one column's sum, against 64
+// cache lines per load instruction and NC sums per lane.  All entries of a pass
+// and then all their x are loaded before the first product, from clamped
+// addresses, the entries past the row as zeros, and the next row's entries are
+// loaded before the current row's are summed; 8-node 64 x 64 x 48, four columns,
+// with the dot product: 156 us plain, 156 us grouped without the next row's loads
+// ahead, 126 us with them; capping the registers for a third wave per SIMD spills
+// and takes twice the time.  spmv_grouped_rows says where it is used.
+template <typename VT, typename KT, typename MT, int NC, int LPR, bool C64, bool DOT, bool GRP>
 __device__ __forceinline__ void spmv_body(int64_t nne, const int64_t *__restrict__ rowptr,
                                           const int32_t *__restrict__ col, const KT *__restrict__ K,
                                           const MT *__restrict__ M, const ColW &w, const VT *__restrict__ x,
                                           VT *__restrict__ y, const VT *__restrict__ p, double *__restrict__ part) {
-  constexpr bool GROUP = NC == 2 || NC == 4;
+  static_assert(!GRP || NC == 2 || NC == 4, "a group is two or four lanes");
   const int lane = threadIdx.x % LPR;
+  constexpr int RP = kBS / LPR;  // rows of one pass
   double dr[NC], di[NC];
 #pragma unroll
   for (int c = 0; c < NC; c++) dr[c] = di[c] = 0.0;
-  // workgroups are dealt to the XCDs in turn: renumbered so that each XCD walks
-  // one contiguous eighth of the rows, each workgroup a contiguous run of it
-  const int gx = gridDim.x, bx = blockIdx.x, x8 = bx % 8;
-  const int64_t wg = (int64_t)x8 * (gx / 8) + (x8 < gx % 8 ? x8 : gx % 8) + bx / 8;
-  constexpr int RP = kBS / LPR;  // rows of one pass
-  const int64_t per = ((nne + RP - 1) / RP + gx - 1) / gx * RP;
-  const int64_t rend = (wg + 1) * per < nne ? (wg + 1) * per : nne;
-  if constexpr (GROUP) {
+  if constexpr (GRP) {
+    // workgroups are dealt to the XCDs in turn: renumbered so that each XCD walks
+    // one contiguous eighth of the rows, each workgroup a contiguous run of it
+    const int gx = gridDim.x, bx = blockIdx.x, x8 = bx % 8;
+    const int64_t wg = (int64_t)x8 * (gx / 8) + (x8 < gx % 8 ? x8 : gx % 8) + bx / 8;
+    const int64_t per = ((nne + RP - 1) / RP + gx - 1) / gx * RP;
+    const int64_t rend = (wg + 1) * per < nne ? (wg + 1) * per : nne;
     constexpr int U = spmv_unroll<LPR>();
     const int gc = threadIdx.x % NC;
     double wc = w.w[0], sr = 0.0, si = 0.0;
@@ -232,7 +235,7 @@ __device__ __forceinline__ void spmv_body(int64_t nne, const int64_t *__restrict
         di[c] = lane == c ? si : 0.0;
       }
   } else {
-    for (int64_t rb = wg * per; rb < rend; rb += RP) {
+    for (int64_t rb = (int64_t)blockIdx.x * RP; rb < nne; rb += (int64_t)gridDim.x * RP) {
       const int64_t row = rb + threadIdx.x / LPR;
       double ar[NC], ai[NC];
 #pragma unroll
@@ -311,12 +314,12 @@ __device__ __forceinline__ void spmv_body(int64_t nne, const int64_t *__restrict
   }
 }
 
-template <typename VT, typename KT, typename MT, int NC, int LPR, bool C64, bool DOT>
+template <typename VT, typename KT, typename MT, int NC, int LPR, bool C64, bool DOT, bool GRP>
 __global__ __launch_bounds__(kBS) void k_spmv(int64_t nne, const int64_t *__restrict__ rowptr,
                                               const int32_t *__restrict__ col, const KT *__restrict__ K,
                                               const MT *__restrict__ M, ColW w, const VT *__restrict__ x,
                                               VT *__restrict__ y, const VT *__restrict__ p, double *__restrict__ part) {
-  spmv_body<VT, KT, MT, NC, LPR, C64, DOT>(nne, rowptr, col, K, M, w, x, y, p, part);
+  spmv_body<VT, KT, MT, NC, LPR, C64, DOT, GRP>(nne, rowptr, col, K, M, w, x, y, p, part);
 }
 
 // ------------------------------------------------------- block reduction ----
@@ -665,7 +668,7 @@ __global__ __launch_bounds__(kBS) void k_cocg_step2(int64_t nne, const ColState 
 // writes the state back at the end.  Every block runs every iteration: inactive
 // columns only carry zero alpha and beta.
 template <int NC, int LPR, bool C64>
-__global__ __launch_bounds__(kBS) void k_cocg_persist(int iters, int64_t nne, const int64_t *__restrict__ rowptr,
+__global__ __launch_bounds__(kBS, 2) void k_cocg_persist(int iters, int64_t nne, const int64_t *__restrict__ rowptr,
                                                       const int32_t *__restrict__ col, const double *__restrict__ K,
                                                       const double *__restrict__ M, ColW w, double *__restrict__ x,
                                                       double *__restrict__ r, double *__restrict__ p,
@@ -679,7 +682,7 @@ __global__ __launch_bounds__(kBS) void k_cocg_persist(int iters, int64_t nne, co
   __syncthreads();
   const int nb = gridDim.x;
   for (int k = 0; k < iters; k++) {
-    spmv_body<double, double, double, NC, LPR, C64, true>(nne, rowptr, col, K, M, w, p, q, p, spart);
+    spmv_body<double, double, double, NC, LPR, C64, true, NC <= 4>(nne, rowptr, col, K, M, w, p, q, p, spart);
     grid.sync();
     reduce_partials<NC, 1>(spart, nb, out1);
     __syncthreads();
@@ -1092,6 +1095,7 @@ struct Solver {
   int lpr;
   int64_t n;  // nne
   SpmvTimer *tm;
+  bool grp = false;  // rows for the grouped SpMV (spmv_grouped_rows)
   // device block the Krylov buffers are carved from; nullptr: allocated per call
   char *ws = nullptr;
   size_t ws_cap = 0;
@@ -1163,10 +1167,40 @@ static int spmv_blocks(int64_t n) {
   int64_t b = (n + kBS / 16 - 1) / (kBS / 16);
   return (int)(b < kSpmvBlocks ? b : kSpmvBlocks);
 }
-// workgroups of this solver's SpMV: no more than its rows need, and eight waves
-// per SIMD at most, since one workgroup then adds up their partial sums
-static int spmv_grid(int64_t n, int lpr) {
-  return (int)std::min<int64_t>(spmv_blocks(n), std::min<int64_t>((n * lpr + kBS - 1) / kBS, 2048));
+// The grouped form pays only where the plain form's gathers of x leave the L2s:
+// 8-node rows (one pass of eight lanes holds them) of systems above about 220k
+// DOFs, with four columns, or with two and no dot product (which costs the
+// grouped form's longer row chains more).  us plain / grouped, complex64, four
+// columns with the dot product: 199k DOFs 55.5 / 54.8 (44 / 50 without), 237k
+// 63 / 54, 570k 156 / 126, 2.3M 633 / 467; two columns without it: 199k 29.4 /
+// 33.5, 237k 33.5 / 32.2, 570k 95 / 86; with it 570k 98 / 103.  Longer rows leave
+// a second pass nearly empty (two columns with the dot product: 20-node 129k 41 /
+// 52, 27-node 69k 32 / 45), and float vectors halve the plain form's lines (8-node
+// 570k, four columns: 182 / 248).
+constexpr int kGrpLanes = 8;
+constexpr int64_t kGrpMinRows = 220000;
+static bool short_rows(const mvf_handle *h) {
+  return h->nnz <= (int64_t)kGrpLanes * spmv_unroll<kGrpLanes>() * h->nne;
+}
+static bool spmv_grouped_rows(const mvf_handle *h) { return h->nne >= kGrpMinRows && short_rows(h); }
+template <typename MT, int NC, bool DOT>
+constexpr bool spmv_grouped_call() {
+  return sizeof(MT) == 8 && (NC == 4 || (NC == 2 && !DOT));
+}
+
+// workgroups of an SpMV (and of its partial sums): no more than its rows need.
+// The grouped form takes eight waves per SIMD at most.  The plain form with the
+// dot product takes four workgroups per CU: one workgroup adds up the partial sums
+// afterwards, and more of them do not run side by side anyway (us at 1024 / 4096
+// workgroups, sixteen columns: 8-node 145k DOFs 171 / 209, 570k 656 / 693, 27-node
+// 69k 264 / 297; four: 8-node 145k 39 / 44; two: 25.4 / 24.7).  Without it the
+// last workgroups to finish count more (sixteen columns, 145k: 191 / 153).
+template <typename MT, int NC, bool DOT>
+static int spmv_grid(const Solver &S) {
+  const bool grp = spmv_grouped_call<MT, NC, DOT>() && S.grp;
+  const int64_t lpr = grp ? kGrpLanes : sizeof(MT) == 8 ? S.lpr : 16;
+  const int most = grp ? 2048 : DOT ? 1024 : kSpmvBlocks;
+  return (int)std::min<int64_t>(std::min(spmv_blocks(S.n), most), (S.n * lpr + kBS - 1) / kBS);
 }
 
 template <typename VT, typename MT, int NC, bool DOT>
@@ -1180,20 +1214,22 @@ static void spmv_launch(const Solver &S, const MT *K, const MT *M, const VT *x, 
   }
   // lanes per row: the autotuned choice for the FP64 operator, 16 otherwise
   const int lpr = sizeof(MT) == 8 ? S.lpr : 16;
-  const unsigned grid = (unsigned)spmv_grid(S.n, lpr);
-#define MVF_SPMV(L_)                                                                                             \
+  constexpr bool grp = spmv_grouped_call<MT, NC, DOT>();
+  const unsigned grid = (unsigned)spmv_grid<MT, NC, DOT>(S);
+#define MVF_SPMV(L_, G_)                                                                                         \
   do {                                                                                                           \
     if (S.c64)                                                                                                   \
-      hipLaunchKernelGGL((k_spmv<VT, float, MT, NC, L_, true, DOT>), dim3(grid), dim3(kBS), 0, h->stream, S.n,   \
-                         h->d_rowptr, h->d_col, h->d_K32, M, S.w, x, y, p, part);                                \
+      hipLaunchKernelGGL((k_spmv<VT, float, MT, NC, L_, true, DOT, G_>), dim3(grid), dim3(kBS), 0, h->stream,    \
+                         S.n, h->d_rowptr, h->d_col, h->d_K32, M, S.w, x, y, p, part);                           \
     else                                                                                                         \
-      hipLaunchKernelGGL((k_spmv<VT, MT, MT, NC, L_, false, DOT>), dim3(grid), dim3(kBS), 0, h->stream, S.n,     \
+      hipLaunchKernelGGL((k_spmv<VT, MT, MT, NC, L_, false, DOT, G_>), dim3(grid), dim3(kBS), 0, h->stream, S.n, \
                          h->d_rowptr, h->d_col, K, M, S.w, x, y, p, part);                                       \
   } while (0)
-  if (sizeof(MT) == 8 && lpr == 4) MVF_SPMV(4);
-  else if (sizeof(MT) == 8 && lpr == 8) MVF_SPMV(8);
-  else if (sizeof(MT) == 8 && lpr == 32) MVF_SPMV(32);
-  else MVF_SPMV(16);
+  if (grp && S.grp) MVF_SPMV(kGrpLanes, grp);
+  else if (sizeof(MT) == 8 && lpr == 4) MVF_SPMV(4, false);
+  else if (sizeof(MT) == 8 && lpr == 8) MVF_SPMV(8, false);
+  else if (sizeof(MT) == 8 && lpr == 32) MVF_SPMV(32, false);
+  else MVF_SPMV(16, false);
 #undef MVF_SPMV
   if (tm && tm->on) {
     (void)hipEventRecord(tm->ev[tm->used][1], h->stream);
@@ -1286,26 +1322,29 @@ static int cocg_persist_run(Solver &S, int grid, int iters, double *x, double *r
   return 0;
 }
 
-// dispatch over the autotuned lane width and the matrix rounding
+// dispatch over the lane width and the matrix rounding: two and four columns take
+// the grouped SpMV at any size (8 lanes for short rows, 32 for longer ones: one
+// pass each), eight and sixteen the plain one at the autotuned width
 template <int NC>
 static int cocg_persist(Solver &S, bool grid_only, int &grid, int iters, double *x, double *r, double *p, double *q,
                         const double *invd, double *spart, double *part, ColState *st, double tol) {
-#define MVF_PERSIST(LPR_, C64_)                                                                                    \
-  return grid_only ? cocg_persist_grid<NC, LPR_, C64_>(S.h, S.n, grid)                                            \
-                   : cocg_persist_run<NC, LPR_, C64_>(S, grid, iters, x, r, p, q, invd, spart, part, st, tol)
-  if (S.c64) {
-    switch (S.lpr) {
-      case 4: MVF_PERSIST(4, true);
-      case 8: MVF_PERSIST(8, true);
-      case 32: MVF_PERSIST(32, true);
-      default: MVF_PERSIST(16, true);
-    }
+#define MVF_PERSIST(LPR_)                                                                                          \
+  do {                                                                                                             \
+    if (S.c64)                                                                                                     \
+      return grid_only ? cocg_persist_grid<NC, LPR_, true>(S.h, S.n, grid)                                        \
+                       : cocg_persist_run<NC, LPR_, true>(S, grid, iters, x, r, p, q, invd, spart, part, st, tol); \
+    return grid_only ? cocg_persist_grid<NC, LPR_, false>(S.h, S.n, grid)                                         \
+                     : cocg_persist_run<NC, LPR_, false>(S, grid, iters, x, r, p, q, invd, spart, part, st, tol);  \
+  } while (0)
+  if constexpr (NC <= 4) {
+    if (short_rows(S.h)) MVF_PERSIST(kGrpLanes);
+    MVF_PERSIST(32);
   } else {
     switch (S.lpr) {
-      case 4: MVF_PERSIST(4, false);
-      case 8: MVF_PERSIST(8, false);
-      case 32: MVF_PERSIST(32, false);
-      default: MVF_PERSIST(16, false);
+      case 4: MVF_PERSIST(4);
+      case 8: MVF_PERSIST(8);
+      case 32: MVF_PERSIST(32);
+      default: MVF_PERSIST(16);
     }
   }
 #undef MVF_PERSIST
@@ -1341,7 +1380,7 @@ static int run_cocg64(Solver &S, const mvf_solver_opts *o, const double *b, doub
       hipLaunchKernelGGL((k_invdiag<NC, false>), dim3(grid1d(n, 256)), dim3(256), 0, h->stream, n, h->d_diagpos,
                          h->d_K, h->d_M, S.w, invd);
   };
-  int nb = vec_blocks(n, NC), sb = spmv_grid(n, S.lpr);
+  int nb = vec_blocks(n, NC), sb = spmv_grid<double, NC, true>(S);
   int it = 0, restarts = 0;
   ColState hs[NC];
   double res[NC];
@@ -1446,7 +1485,7 @@ static int run_cocg_mixed(Solver &S, const mvf_solver_opts *o, const double *b, 
     hipLaunchKernelGGL((k_invdiag<NC, false>), dim3(grid1d(n, 256)), dim3(256), 0, h->stream, n, h->d_diagpos, h->d_K,
                        h->d_M, S.w, invd);
   MVF_HIP(h, hipMemsetAsync(x32, 0, nv * sizeof(float), h->stream));
-  int nb = vec_blocks(n, NC), sb = spmv_grid(n, 16);
+  int nb = vec_blocks(n, NC), sb = spmv_grid<float, NC, true>(S);
   int it = 0, refinements = 0;
   ColState hs[NC];
   double res[NC];
@@ -1717,36 +1756,40 @@ static int guess_scale(Solver &S, const double *b, double *x, double *alpha_out)
 constexpr int nc_slot(int nc) { return nc == 2 ? 0 : (nc == 4 ? 1 : (nc == 8 ? 2 : 3)); }
 
 // SpMV autotuner: the FP64 operator's lanes per row (4, 8, 16 or 32) timed
-// once per handle and column count with HIP events (one warm-up and three
-// timed launches each), the fastest kept in the handle.  Rows of 8-node
-// systems hold <= 33 entries, 20-node ~84, 27-node ~104: the best width
-// follows the row length and the column count.
-template <int NC>
+// once per handle, column count and form (COCG runs the one with the dot product)
+// with HIP events (one warm-up and three timed launches each), the fastest kept
+// in the handle.  Rows of 8-node systems hold <= 33 entries, 20-node ~84, 27-node
+// ~104: the best width follows the row length and the column count.
+template <int NC, bool DOT>
 static int tune_lpr(Solver &S) {
   mvf_handle *h = S.h;
-  int &slot = h->spmv_lpr[nc_slot(NC)];
+  int &slot = h->spmv_lpr[DOT][nc_slot(NC)];
   if (slot) {
     S.lpr = slot;
     return 0;
   }
   DevScope ds;
-  double *xa, *ya;
+  double *xa, *ya, *part = nullptr;
   const int64_t nv = S.n * NC * 2;
   MVF_TRY(ds.alloc(h, &xa, nv));
   MVF_TRY(ds.alloc(h, &ya, nv));
+  if (DOT) MVF_TRY(ds.alloc(h, &part, (size_t)spmv_blocks(S.n) * NC * 2));
   hipLaunchKernelGGL(k_fill_d, dim3(grid1d(nv, 256)), dim3(256), 0, h->stream, nv, xa, 1.0);
   hipEvent_t e0, e1;
   MVF_HIP(h, hipEventCreate(&e0));
   MVF_HIP(h, hipEventCreate(&e1));
   SpmvTimer *tm = S.tm;
   S.tm = nullptr;
+  const bool grp = S.grp;
+  S.grp = false;  // the plain form's width
   int best = 16;
   float best_ms = 1e30f;
   for (int L : {4, 8, 16, 32}) {
     S.lpr = L;
-    spmv_launch<double, double, NC, false>(S, h->d_K, h->d_M, xa, ya, nullptr, nullptr);
+    auto apply = [&]() { spmv_launch<double, double, NC, DOT>(S, h->d_K, h->d_M, xa, ya, DOT ? xa : nullptr, part); };
+    apply();
     (void)hipEventRecord(e0, h->stream);
-    for (int k = 0; k < 3; k++) spmv_launch<double, double, NC, false>(S, h->d_K, h->d_M, xa, ya, nullptr, nullptr);
+    for (int k = 0; k < 3; k++) apply();
     (void)hipEventRecord(e1, h->stream);
     float ms = 0.f;
     if (hipEventSynchronize(e1) == hipSuccess && hipEventElapsedTime(&ms, e0, e1) == hipSuccess && ms < best_ms) {
@@ -1755,6 +1798,7 @@ static int tune_lpr(Solver &S) {
     }
   }
   S.tm = tm;
+  S.grp = grp;
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   MVF_HIP(h, hipGetLastError());
@@ -1774,7 +1818,10 @@ static int solve_nc(mvf_handle *h, const double *omegas, int ncol, const mvf_sol
   tm->reset();
   Solver S{h, ncol, {}, o->matrix == MVF_MATRIX_C64REF, 16, (int64_t)h->nne, tm};
   for (int c = 0; c < NC; c++) S.w.w[c] = c < ncol ? (double)(float)omegas[c] : 0.0;
-  int rc = h->autotune ? tune_lpr<NC>(S) : 0;
+  S.grp = spmv_grouped_rows(h);
+  const bool cocg64 =
+      o->precond != MVF_PC_DIRECT && o->precision != MVF_PREC_MIXED && o->method != MVF_KRYLOV_BICGSTAB;
+  int rc = !h->autotune ? 0 : cocg64 ? tune_lpr<NC, true>(S) : tune_lpr<NC, false>(S);
   if (!rc && alpha_out) rc = guess_scale<NC>(S, b, x, alpha_out);
   if (rc) {
   } else if (o->precond == MVF_PC_DIRECT) rc = run_gmres_direct<NC>(S, o, b, x, info);
@@ -1792,7 +1839,7 @@ static int solve_nc(mvf_handle *h, const double *omegas, int ncol, const mvf_sol
   info->spmv_bytes[0] = nnz * ((S.c64 ? 4 : 8) + 8 + 4) + n * (8 + NC * (16 + 16));
   info->spmv_bytes[1] = nnz * (4 + 4 + 4) + n * (8 + NC * (8 + 8));
   info->spmv_ncol = NC;
-  info->spmv_lpr = S.lpr;
+  info->spmv_lpr = NC == 4 && S.grp ? kGrpLanes : S.lpr;
   return rc;
 }
 

@@ -167,3 +167,27 @@ def test_cocg_columns_and_rows(nodes, sides, nf, matrix, need_gpu):
             r = np.linalg.norm(b - A @ x[2 * i + d]) / np.linalg.norm(b)
             # the unrounded operator differs from the complex64 entry list by its rounding, 2^-24 relative
             assert r <= (1.1e-9 if matrix == "c64ref" else 1e-5), (i, d, r)
+
+
+@pytest.mark.parametrize("sides", [(44, 44, 36), (47, 50, 37)])  # 199k and 249k DOFs: on either side of the rule
+@pytest.mark.parametrize("method,nf", [("cocg", 2), ("cocg", 1), ("bicgstab", 1)])
+def test_spmv_large_grids(sides, method, nf, need_gpu):
+    """The SpMV's two forms at the sizes where the choice between them lies: four
+    and two columns with the dot product, two without it; the second grid's rows
+    fill no whole pass of the workgroups.  The bar is each column's residual formed
+    on the host, as in test_cocg_columns_and_rows."""
+    freqs = (50.0, 80.0)[:nf]
+    nx, ny, nz = sides
+    m = M.anisotropic_blocks(nx=nx, ny=ny, nz_earth=nz - 2, nz_air=2, h=500.0, nodes=8, freqs=freqs, block=4, seed=5,
+                             full_tensor=True, dirichlet=True, nextd=2)
+    g = GpuVfem(m, emulate=0)
+    info = g.solve_frequencies(freqs, method=method, tol=1e-8, maxit=20000)
+    print(f"SpMV form {sides} {method} nf={nf}: nne={g.nne} its={info['iterations']}", flush=True)
+    assert info["converged"], info
+    x, bb = g.solution(2 * nf), g.rhs(2 * nf)
+    for i in range(nf):
+        g.set_frequency(i)
+        A, _ = reference_system(g)
+        for d in range(2):
+            b = bb[2 * i + d]
+            assert np.linalg.norm(b - A @ x[2 * i + d]) <= 1.1e-8 * np.linalg.norm(b)
