@@ -166,6 +166,17 @@ void mvf_default_solver_opts(mvf_solver_opts *o) {
   o->use_graph = 0;
 }
 
+// failure injection for the tests: the calling thread's next `skip` device
+// allocations succeed, the `fail` after them report no memory; returns the
+// failures of the last setting that were not used
+int32_t mvf_fail_allocs(int32_t skip, int32_t fail) {
+  AllocFail &f = alloc_fail();
+  const int32_t left = f.fail;
+  f.skip = skip;
+  f.fail = fail;
+  return left;
+}
+
 const char *mvf_last_error(const mvf_handle *h) { return h ? h->err.c_str() : mvf::g_host_err.c_str(); }
 
 void mvf_free(mvf_handle *h) {

@@ -1619,8 +1619,8 @@ void direct_invalidate(mvf_handle *h) {
   if (h->direct) ((DirectPlan *)h->direct)->factored = 0;
 }
 
-static int direct_plan(mvf_handle *h) {
-  if (h->direct) return 0;
+// fills h->direct: symbolic analysis, device buffers and their contents
+static int direct_plan_build(mvf_handle *h) {
   double t0 = now_s();
   const int64_t nne = h->nne, nnz = h->nnz, ne = h->geo.ne;
   const int me = h->et.ne;
@@ -1631,19 +1631,14 @@ static int direct_plan(mvf_handle *h) {
   MVF_HIP(h, hipMemcpy(rowptr.data(), h->d_rowptr, rowptr.size() * 8, hipMemcpyDeviceToHost));
   MVF_HIP(h, hipMemcpy(diagpos.data(), h->d_diagpos, diagpos.size() * 8, hipMemcpyDeviceToHost));
   DirectPlan *P = new DirectPlan();
+  h->direct = P;
   PlanArrays A;
   std::string err;
   int rc = build_plan_host(*P, h->geo.nx, h->geo.ny, h->geo.nz, me, gne.data(), nne, rowptr.data(), col.data(), A, err);
-  if (rc) {
-    delete P;
-    return set_err(h, rc, "direct plan: %s", err.c_str());
-  }
+  if (rc) return set_err(h, rc, "direct plan: %s", err.c_str());
   for (int d = 0; d <= P->maxdepth; d++)
-    if (P->levels[d].size() > 65535) {
-      delete P;
+    if (P->levels[d].size() > 65535)
       return set_err(h, MVF_E_UNSUPPORTED, "direct plan: %zu fronts in one level", P->levels[d].size());
-    }
-  h->direct = P;
   // smallest M/|K| over DOFs with mass, largest diagonal magnitudes
   {
     std::vector<double> K(nnz), M(nnz);
@@ -1709,6 +1704,14 @@ static int direct_plan(mvf_handle *h) {
   MVF_HIP(h, hipMemcpy(P->d_blk, blk.data(), sizeof(int2) * blk.size(), hipMemcpyHostToDevice));
   P->t_symbolic = now_s() - t0;
   return 0;
+}
+
+// a plan that could not be completed is given back, so that the next call starts anew
+static int direct_plan(mvf_handle *h) {
+  if (h->direct) return 0;
+  const int rc = direct_plan_build(h);
+  if (rc) direct_free(h);
+  return rc;
 }
 
 // numeric factorization of A_pc at angular frequency w (fl32(omega) as in the operator)

@@ -292,15 +292,34 @@ inline int set_err(mvf_handle *h, int code, const char *fmt, ...) {
     if (rc_) return rc_;   \
   } while (0)
 
+// hipMalloc with the failure injection of the tests (mvf_fail_allocs): of this
+// thread's next allocations the first `skip` succeed, then `fail` report no memory
+struct AllocFail {
+  int skip = 0, fail = 0;
+};
+inline AllocFail &alloc_fail() {
+  static thread_local AllocFail f;
+  return f;
+}
+inline hipError_t raw_malloc(void **p, size_t bytes) {
+  AllocFail &f = alloc_fail();
+  if (f.skip > 0) f.skip--;
+  else if (f.fail > 0) {
+    f.fail--;
+    return hipErrorOutOfMemory;
+  }
+  return hipMalloc(p, bytes);
+}
+
 template <typename T>
 inline int dalloc(mvf_handle *h, T **p, size_t n) {
   void *q = nullptr;
   size_t bytes = (n ? n : 1) * sizeof(T);
-  hipError_t e = hipMalloc(&q, bytes);
+  hipError_t e = raw_malloc(&q, bytes);
   if (e == hipErrorOutOfMemory) {
     (void)hipGetLastError();
     BufPool::trim_all();
-    e = hipMalloc(&q, bytes);
+    e = raw_malloc(&q, bytes);
   }
   if (e != hipSuccess)
     return set_err(h, MVF_E_MEMORY, "hipMalloc(%zu bytes) failed: %s", bytes, hipGetErrorString(e));

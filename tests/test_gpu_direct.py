@@ -16,8 +16,9 @@ import pytest
 import scipy.sparse as sp
 import scipy.sparse.linalg as spla
 
+from movfem_amd import _lib as L
 from movfem_amd import model as M
-from movfem_amd.vfem import GpuVfem
+from movfem_amd.vfem import GpuVfem, MvfError
 from tests.gauge import determined_dofs, inner_dofs
 
 pytestmark = pytest.mark.gpu
@@ -167,3 +168,37 @@ def test_direct_block_rows(nodes, sides, tile, need_gpu):
     for d in range(2):
         xr = lu.solve(b[d])
         assert np.linalg.norm(x[d][mask] - xr[mask]) <= 1e-6 * np.linalg.norm(xr[mask])
+
+
+def test_direct_out_of_memory(need_gpu):
+    """Every device allocation of a first direct solve fails in turn (reported on
+    the host; both tries).  The call returns MVF_E_MEMORY, and the next call on
+    the same handle solves: no half-built plan is left to run on."""
+    fail = L.lib().mvf_fail_allocs
+    m = M.random_small(8, 5, 4, 4, seed=33, nz_air=1, freqs=(10.0,))
+    opts = dict(method="gmres", precond="direct", tol=1e-10)
+    g = GpuVfem(m)
+    g.set_frequency(0)
+    mask = determined_dofs(m, g.gne())
+    _, _, _, b = g.global_vfem()
+    xr = g.solve(b, **opts)[0].reshape(2, -1)[:, mask]
+    g.close()
+    for skip in range(100):
+        g = GpuVfem(m)
+        g.set_frequency(0)
+        fail(skip, 2)
+        try:
+            g.solve(b, **opts)
+            code = 0
+        except MvfError as e:
+            code = e.code
+        unused = fail(0, 0)
+        assert (code, unused) in ((L.MVF_E_MEMORY, 0), (0, 2)), (skip, code, unused)
+        x, info = g.solve(b, **opts)
+        assert info["converged"], info
+        assert np.linalg.norm(x.reshape(2, -1)[:, mask] - xr) <= 1e-6 * np.linalg.norm(xr)
+        g.close()
+        if not code:
+            break
+    print(f"allocations failed in turn: {skip}", flush=True)
+    assert 20 <= skip < 99
