@@ -97,8 +97,10 @@ __device__ inline int64_t xcd_block(int64_t b, int64_t nb) {
 // hipMalloc and hipFree cost 50-300 us each and wait for the whole device, other
 // handles' streams included.  A handle's work is ordered on its stream, so a
 // buffer can be handed out again while earlier work on it is queued.  At most
-// kMax bytes are kept (the oldest go first), and an allocation that fails
-// anywhere empties every pool and is tried again.
+// kMax bytes are kept per handle (the oldest go first).  They go back to the device
+// when the handle closes and whenever one of this library's own allocations finds
+// no memory (dev_malloc empties every pool and tries again); another allocator in
+// the process cannot reach them.
 struct BufPool {
   static constexpr size_t kMax = (size_t)1 << 30;
   struct Buf {
@@ -311,16 +313,23 @@ inline hipError_t raw_malloc(void **p, size_t bytes) {
   return hipMalloc(p, bytes);
 }
 
+// every device allocation of the library: when memory runs out, what the handles
+// keep for reuse goes first
+inline hipError_t dev_malloc(void **p, size_t bytes) {
+  hipError_t e = raw_malloc(p, bytes);
+  if (e == hipErrorOutOfMemory) {
+    (void)hipGetLastError();
+    BufPool::trim_all();
+    e = raw_malloc(p, bytes);
+  }
+  return e;
+}
+
 template <typename T>
 inline int dalloc(mvf_handle *h, T **p, size_t n) {
   void *q = nullptr;
   size_t bytes = (n ? n : 1) * sizeof(T);
-  hipError_t e = raw_malloc(&q, bytes);
-  if (e == hipErrorOutOfMemory) {
-    (void)hipGetLastError();
-    BufPool::trim_all();
-    e = raw_malloc(&q, bytes);
-  }
+  hipError_t e = dev_malloc(&q, bytes);
   if (e != hipSuccess)
     return set_err(h, MVF_E_MEMORY, "hipMalloc(%zu bytes) failed: %s", bytes, hipGetErrorString(e));
   *p = (T *)q;
@@ -331,8 +340,9 @@ inline void dfree(void *p) {
   if (p) (void)hipFree(p);
 }
 
-// Temporary device buffers of one call: whatever is allocated through it is
-// freed when the call returns, on every return path (errors included).
+// Temporary device buffers of one call: whatever is allocated through it goes
+// back to the handle's pool when the call returns, on every return path (errors
+// included).
 struct DevScope {
   mvf_handle *h = nullptr;
   std::vector<BufPool::Buf> bufs;

@@ -615,7 +615,7 @@ static int nn_err(mvf_nn *n, int code, const char *fmt, ...) {
 template <typename T>
 static int nn_alloc(mvf_nn *n, T **p, size_t count) {
   void *q = nullptr;
-  hipError_t e = hipMalloc(&q, (count ? count : 1) * sizeof(T));
+  hipError_t e = dev_malloc(&q, (count ? count : 1) * sizeof(T));
   if (e != hipSuccess) return nn_err(n, MVF_E_MEMORY, "hipMalloc(%zu) failed", count * sizeof(T));
   n->owned.push_back(q);
   *p = (T *)q;

@@ -15,7 +15,10 @@ import pathlib
 import numpy as np
 import pytest
 
+from movfem_amd import _lib as L
 from movfem_amd import learned as Lm
+from movfem_amd import model as M
+from movfem_amd.vfem import GpuVfem
 from tests import unet_ref
 
 pytestmark = pytest.mark.gpu
@@ -141,3 +144,24 @@ def test_learned_guess_held_out(need_gpu):
         assert res <= 1.5e-8
     g.close()
     net.close()
+
+
+def test_network_takes_kept_buffers(need_gpu):
+    """Creating a network while a handle keeps work buffers for reuse: an allocation
+    that finds no memory (reported on the host, each of the first ones in turn)
+    gets the kept buffers freed and is tried again."""
+    import torch
+
+    m = M.anisotropic_blocks(nx=24, ny=24, nz_earth=18, nz_air=2, h=500.0, nodes=8, freqs=(1.0,), block=4, seed=5)
+    g = GpuVfem(m)
+    fail = L.lib().mvf_fail_allocs
+    for skip in (0, 1, 7, 30):
+        g.solve_frequencies([1.0, 2.0, 4.0], method="gmres", precond="direct", tol=1e-8, freqs_per_factor=3)
+        before = torch.cuda.mem_get_info()[0]
+        fail(skip, 1)
+        net = Lm.Net(nx=8, ny=8, nz=8, batch=1, seed=1)
+        assert fail(0, 0) == 0
+        # the handle kept GMRES vectors of eight columns: 2 x 31 x 128 bytes per DOF
+        assert torch.cuda.mem_get_info()[0] - before > 31 * 128 * g.nne
+        net.close()
+    g.close()
