@@ -833,6 +833,9 @@ int mvf_solve_frequencies(mvf_handle *h, const double *freqs_hz, int32_t nfreq, 
     dfree(h->d_x);
     dfree(h->d_b);
     h->d_x = h->d_b = nullptr;
+    h->xb_cap = 0;
+    h->last_freqs.clear();  // no solution to read out until the call succeeds
+    h->ncols_last = 0;
     MVF_TRY(dalloc(h, &h->d_x, need));
     MVF_TRY(dalloc(h, &h->d_b, need));
     h->xb_cap = need;

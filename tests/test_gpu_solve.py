@@ -10,8 +10,9 @@ import pytest
 import scipy.sparse as sp
 import scipy.sparse.linalg as spla
 
+from movfem_amd import _lib as L
 from movfem_amd import model as M
-from movfem_amd.vfem import GpuVfem
+from movfem_amd.vfem import GpuVfem, MvfError
 
 pytestmark = pytest.mark.gpu
 
@@ -191,3 +192,31 @@ def test_spmv_large_grids(sides, method, nf, need_gpu):
         for d in range(2):
             b = bb[2 * i + d]
             assert np.linalg.norm(b - A @ x[2 * i + d]) <= 1.1e-8 * np.linalg.norm(b)
+
+
+def test_solution_buffers_out_of_memory(need_gpu):
+    """The solution or right-hand-side buffer finds no memory (reported on the
+    host) when a call needs more columns: the call says so, nothing is left to
+    read out, and a call with the first column count solves again."""
+    fail = L.lib().mvf_fail_allocs
+    freqs = (20.0, 50.0, 90.0)
+    g = GpuVfem(M.random_small(8, 5, 4, 4, seed=51, freqs=freqs), emulate=0)
+    opts = dict(method="cocg", tol=1e-10, maxit=20000)
+    g.solve_frequencies(freqs[:1], **opts)
+    x0 = g.solution(2)
+    for skip in (0, 1):
+        g.close()
+        g = GpuVfem(M.random_small(8, 5, 4, 4, seed=51, freqs=freqs), emulate=0)
+        g.solve_frequencies(freqs[:1], **opts)
+        fail(skip, 2)
+        with pytest.raises(MvfError) as e:
+            g.solve_frequencies(freqs, **opts)
+        assert (e.value.code, fail(0, 0)) == (L.MVF_E_MEMORY, 0)
+        for read in (lambda: g.solution(2), lambda: g.rhs(2), lambda: g.readout(None, f=0)):
+            with pytest.raises(MvfError):
+                read()
+        g.solve_frequencies(freqs[:1], **opts)
+        # the relative residual is below 1e-10 in both solves
+        assert np.linalg.norm(g.solution(2) - x0) <= 1e-5 * np.linalg.norm(x0)
+        g.readout(None, f=0)
+    g.close()
