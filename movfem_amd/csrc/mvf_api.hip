@@ -394,20 +394,20 @@ int mvf_assemble(mvf_handle *h, int32_t precision, double *integrate_ms) {
   MVF_HIP(h, hipEventCreate(&ev[1]));
   int rc = 0;
   if (precision == 0) {
-    MVF_TRY(dalloc(h, &h->d_Ke, np * ne));
-    MVF_TRY(dalloc(h, &h->d_Me, np * ne));
-    MVF_HIP(h, hipEventRecord(ev[0], h->stream));
-    rc = integrate_elements(h, 0, ne, ff, h->d_Ke, h->d_Me);
+    rc = dalloc(h, &h->d_Ke, np * ne);
+    if (!rc) rc = dalloc(h, &h->d_Me, np * ne);
+    (void)hipEventRecord(ev[0], h->stream);
+    if (!rc) rc = integrate_elements(h, 0, ne, ff, h->d_Ke, h->d_Me);
     (void)hipEventRecord(ev[1], h->stream);
     if (!rc) rc = assemble_operators(h);
     dfree(h->d_Ke); dfree(h->d_Me);
     h->d_Ke = h->d_Me = nullptr;
   } else {
-    float *k32, *m32;
-    MVF_TRY(ds.alloc(h, &k32, np * ne));
-    MVF_TRY(ds.alloc(h, &m32, np * ne));
-    MVF_HIP(h, hipEventRecord(ev[0], h->stream));
-    rc = integrate_elements32(h, 0, ne, ff, k32, m32);
+    float *k32 = nullptr, *m32 = nullptr;
+    rc = ds.alloc(h, &k32, np * ne);
+    if (!rc) rc = ds.alloc(h, &m32, np * ne);
+    (void)hipEventRecord(ev[0], h->stream);
+    if (!rc) rc = integrate_elements32(h, 0, ne, ff, k32, m32);
     (void)hipEventRecord(ev[1], h->stream);
     if (!rc) rc = assemble_operators32(h, k32, m32);
     ds.drop(k32); ds.drop(m32);

@@ -220,3 +220,25 @@ def test_solution_buffers_out_of_memory(need_gpu):
         assert np.linalg.norm(g.solution(2) - x0) <= 1e-5 * np.linalg.norm(x0)
         g.readout(None, f=0)
     g.close()
+
+
+def test_assemble_out_of_memory(need_gpu):
+    """Re-assembly whose second element buffer finds no memory (reported on the
+    host): the call says so each time, loses no device memory (the first buffer
+    holds 22 MB) and leaves the operators as they were."""
+    import torch
+
+    fail = L.lib().mvf_fail_allocs
+    g = GpuVfem(M.random_small(27, 12, 12, 13, seed=51, freqs=(20.0,)), emulate=0)
+    ops = g.operators()
+    g.assemble()
+    before = torch.cuda.mem_get_info()[0]
+    for _ in range(20):
+        fail(1, 2)
+        with pytest.raises(MvfError) as e:
+            g.assemble()
+        assert (e.value.code, fail(0, 0)) == (L.MVF_E_MEMORY, 0)
+    assert torch.cuda.mem_get_info()[0] >= before - (64 << 20)
+    for a, b in zip(ops, g.operators()):
+        assert np.array_equal(a, b)
+    g.close()
