@@ -131,7 +131,8 @@ struct DirectPlan {
   int64_t gemm_launches = 0;
 };
 
-// events around the factorization's GEMM launches (ring drained at level ends)
+// events around the factorization's GEMM launches (half the ring is read when it
+// is full, the rest at the end)
 struct GemmTimer {
   static constexpr int kRing = 512;
   hipEvent_t ev[kRing][2];
@@ -1232,7 +1233,7 @@ __host__ __device__ inline GemmArgs gemm_args(int mode, const DNode &nd, int64_t
   return g;
 }
 
-// BIG selects the 128x128 tiles (levels whose fronts are large)
+// BIG selects the 128 x 64 tiles (levels whose fronts are large)
 template <int MODE, bool BIG>
 __global__ __launch_bounds__(BIG ? kBigThreads : 256, 2) void k_fa_gemm_mfma(const DNode *nodes, const int32_t *lev,
                                                                             int64_t step, int64_t K0, double2 *fac,
@@ -1715,7 +1716,7 @@ static int direct_plan(mvf_handle *h) {
 }
 
 // numeric factorization of A_pc at angular frequency w (fl32(omega) as in the operator)
-// levels whose largest front reaches this order use the 128x128 tiles
+// levels whose largest front reaches this order use the 128 x 64 tiles
 constexpr int64_t kBigFront = 512;
 
 template <int MODE>

@@ -663,10 +663,12 @@ __global__ __launch_bounds__(kBS) void k_cocg_step2(int64_t nne, const ColState 
 // `iters` COCG iterations in one cooperative launch: the SpMV with its fused
 // p^T A p partials, alpha, the x/r update with its partials, beta and the p
 // update, separated by three grid barriers per iteration.  Every block reduces
-// the partials itself (the same order as the one-block reduction kernels) and
-// keeps its own copy of the column state, so no further barrier is needed; block 0
-// writes the state back at the end.  Every block runs every iteration: inactive
-// columns only carry zero alpha and beta.
+// the partials itself (256 threads' strides where the one-block kernels have 1024,
+// so the sums' last bits differ) and keeps its own copy of the column state, so no
+// further barrier is needed; block 0 writes the state back at the end.  Every
+// block runs every iteration: inactive columns only carry zero alpha and beta.
+// Two waves per SIMD as the bound: at sixteen columns two registers more would
+// halve them (20-node 40 x 40 x 32, sixteen columns: 3126 -> 2365 us per iteration).
 template <int NC, int LPR, bool C64>
 __global__ __launch_bounds__(kBS, 2) void k_cocg_persist(int iters, int64_t nne, const int64_t *__restrict__ rowptr,
                                                       const int32_t *__restrict__ col, const double *__restrict__ K,
