@@ -49,8 +49,8 @@ FP32_PEAK_TFS = 157.3
 ELEM_FLOPS = {8: 21768, 20: 376731, 27: 744795}
 # HBM bytes per launch from rocprofv3 FETCH_SIZE and WRITE_SIZE runs, each scaled
 # by what the counter reads for a plain copy of known size (profiles/)
-TRAFFIC_MEASURED = {("halfspace8", "k_spmv"): 20.17e6, ("aniso20", "k_fa_gemm"): 3.43e9,
-                    ("aniso20", "k_spmv"): 7.45e9, ("aniso20", "k_elem_km"): 2.40e9}
+TRAFFIC_MEASURED = {("halfspace8", "k_spmv"): 17.6e6, ("aniso20", "k_fa_gemm"): 6.02e9,
+                    ("aniso20", "k_spmv"): 6.59e9, ("aniso20", "k_elem_km"): 2.40e9}
 
 
 def log(msg):
@@ -278,7 +278,8 @@ def main():
     gemm_n = sum(i["gemm_launches"] for i in infos)
     gemm_tfs = gemm_fl / (gemm_ms * 1e-3) / 1e12 if gemm_ms > 0 else 0.0
     roofline = {"bound": "mfma", "kernel": "k_fa_gemm_mfma (FP64 complex on v_mfma_f64_16x16x4, three real products "
-                "per complex one on the 128x64 tiles; achieved counts 8 real flops per complex multiply-add; MI355X "
+                "per complex one on the 128x64 tiles; achieved counts 8 real flops per complex multiply-add, of which "
+                "those tiles execute 6; MI355X "
                 "FP64 matrix peak = FP64 vector peak; launch durations include time shared with the panel kernels "
                 "the lookahead overlaps)",
                 "achieved": gemm_tfs, "peak": FP64_PEAK_TFS, "unit": "TFLOP/s", "frac": gemm_tfs / FP64_PEAK_TFS,
