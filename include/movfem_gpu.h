@@ -200,7 +200,7 @@ typedef struct mvf_solve_info {
   double spmv_ms[2];       /* summed kernel time */
   double spmv_bytes[2];    /* algorithmic bytes of one launch: nnz*(K+M+col) + nne*(rowptr + ncol*(x+y)) */
   int32_t spmv_ncol;       /* columns per launch (last batch) */
-  int32_t spmv_lpr;        /* lanes per matrix row of the FP64 SpMV (autotuned; 8 where the grouped form runs) */
+  int32_t spmv_lpr;        /* lanes per matrix row of the FP64 SpMV, chosen by the autotuner */
   /* MVF_PC_DIRECT */
   double factor_seconds;   /* numeric factorizations performed by this call, wall time */
   double factor_flops;     /* algorithmic real flops of one factorization */

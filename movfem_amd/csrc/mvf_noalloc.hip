@@ -86,12 +86,11 @@ extern "C" int mvf_solve_noalloc(mvf_handle *h, double *rhs_inout, const mvf_sol
   const int64_t n = h->nne;
   // staging: host-layout RHS/solution, then the interleaved b and x
   const size_t vec = (((size_t)n * 2 * sizeof(double2)) + 255) & ~(size_t)255;
-  // the lanes per row the handle's autotuner chose for two columns, if it ran
-  const int dot = o->method != MVF_KRYLOV_BICGSTAB;
-  const int lpr = h->spmv_lpr[dot][0] ? h->spmv_lpr[dot][0] : h->spmv_lpr[!dot][0];
-  Solver S{h, 2, {}, o->matrix == MVF_MATRIX_C64REF, lpr ? lpr : 16, n, nullptr};
+  Solver S{h, 2, {}, o->matrix == MVF_MATRIX_C64REF, 16, n, nullptr};
   S.w.w[0] = S.w.w[1] = (double)(float)h->omega;
-  S.grp = spmv_grouped_rows(h);
+  // the form the handle's autotuner chose for two columns, if it ran
+  const int dot = o->method != MVF_KRYLOV_BICGSTAB;
+  if (const int t = h->spmv_tuned[dot][0] ? h->spmv_tuned[dot][0] : h->spmv_tuned[!dot][0]) spmv_take(S, t);
   Workspace W;
   W.sizing = true;
   if (o->method == MVF_KRYLOV_BICGSTAB) {

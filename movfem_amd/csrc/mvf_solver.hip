@@ -100,7 +100,7 @@ __host__ __device__ constexpr int spmv_unroll() {
 // loaded before the current row's are summed; 8-node 64 x 64 x 48, four columns,
 // with the dot product: 156 us plain, 156 us grouped without the next row's loads
 // ahead, 126 us with them; capping the registers for a third wave per SIMD spills
-// and takes twice the time.  spmv_grouped_rows says where it is used.
+// and takes twice the time.  spmv_grouped_call says where it is used.
 template <typename VT, typename KT, typename MT, int NC, int LPR, bool C64, bool DOT, bool GRP>
 __device__ __forceinline__ void spmv_body(int64_t nne, const int64_t *__restrict__ rowptr,
                                           const int32_t *__restrict__ col, const KT *__restrict__ K,
@@ -1097,7 +1097,7 @@ struct Solver {
   int lpr;
   int64_t n;  // nne
   SpmvTimer *tm;
-  bool grp = false;  // rows for the grouped SpMV (spmv_grouped_rows)
+  bool grp = false;  // grouped FP64 SpMV, 4 or 8 lanes per row
   // device block the Krylov buffers are carved from; nullptr: allocated per call
   char *ws = nullptr;
   size_t ws_cap = 0;
@@ -1169,26 +1169,20 @@ static int spmv_blocks(int64_t n) {
   int64_t b = (n + kBS / 16 - 1) / (kBS / 16);
   return (int)(b < kSpmvBlocks ? b : kSpmvBlocks);
 }
-// The grouped form pays only where the plain form's gathers of x leave the L2s:
-// 8-node rows (one pass of eight lanes holds them) of systems above about 220k
-// DOFs, with four columns, or with two and no dot product (which costs the
-// grouped form's longer row chains more).  us plain / grouped, complex64, four
-// columns with the dot product: 199k DOFs 55.5 / 54.8 (44 / 50 without), 237k
-// 63 / 54, 570k 156 / 126, 2.3M 633 / 467; two columns without it: 199k 29.4 /
-// 33.5, 237k 33.5 / 32.2, 570k 95 / 86; with it 570k 98 / 103.  Longer rows leave
-// a second pass nearly empty (two columns with the dot product: 20-node 129k 41 /
-// 52, 27-node 69k 32 / 45), and float vectors halve the plain form's lines (8-node
-// 570k, four columns: 182 / 248).
-constexpr int kGrpLanes = 8;
-constexpr int64_t kGrpMinRows = 220000;
-static bool short_rows(const mvf_handle *h) {
-  return h->nnz <= (int64_t)kGrpLanes * spmv_unroll<kGrpLanes>() * h->nne;
-}
-static bool spmv_grouped_rows(const mvf_handle *h) { return h->nne >= kGrpMinRows && short_rows(h); }
-template <typename MT, int NC, bool DOT>
+// The grouped form gains where the plain form's gathers of x leave the L2s, and in
+// a band of small systems at four lanes; the autotuner decides.  us plain /
+// grouped, complex64, 8-node rows, four columns with the dot product: 8k DOFs 5.7 /
+// 5.8, 26k 11.1 / 9.8, 145k 39 / 45, 237k 57 / 54, 570k 150 / 126, 2.3M 609 / 467;
+// two columns without it: 199k 29.4 / 33.5, 237k 33.5 / 32.2, 570k 95 / 86.  Longer
+// rows take two passes, the second nearly empty (two columns with the dot product:
+// 20-node 129k 40 / 52, 27-node 69k 30 / 45), and float vectors halve the plain
+// form's lines (8-node 570k, four columns: 182 / 248), so they take the plain form.
+template <typename MT, int NC>
 constexpr bool spmv_grouped_call() {
-  return sizeof(MT) == 8 && (NC == 4 || (NC == 2 && !DOT));
+  return sizeof(MT) == 8 && (NC == 2 || NC == 4);
 }
+// rows that one pass of eight lanes holds (8-node systems)
+static bool short_rows(const mvf_handle *h) { return h->nnz <= (int64_t)8 * spmv_unroll<8>() * h->nne; }
 
 // workgroups of an SpMV (and of its partial sums): no more than its rows need.
 // The grouped form takes eight waves per SIMD at most.  The plain form with the
@@ -1199,8 +1193,8 @@ constexpr bool spmv_grouped_call() {
 // last workgroups to finish count more (sixteen columns, 145k: 191 / 153).
 template <typename MT, int NC, bool DOT>
 static int spmv_grid(const Solver &S) {
-  const bool grp = spmv_grouped_call<MT, NC, DOT>() && S.grp;
-  const int64_t lpr = grp ? kGrpLanes : sizeof(MT) == 8 ? S.lpr : 16;
+  const bool grp = spmv_grouped_call<MT, NC>() && S.grp;
+  const int64_t lpr = sizeof(MT) == 8 ? S.lpr : 16;
   const int most = grp ? 2048 : DOT ? 1024 : kSpmvBlocks;
   return (int)std::min<int64_t>(std::min(spmv_blocks(S.n), most), (S.n * lpr + kBS - 1) / kBS);
 }
@@ -1216,7 +1210,7 @@ static void spmv_launch(const Solver &S, const MT *K, const MT *M, const VT *x, 
   }
   // lanes per row: the autotuned choice for the FP64 operator, 16 otherwise
   const int lpr = sizeof(MT) == 8 ? S.lpr : 16;
-  constexpr bool grp = spmv_grouped_call<MT, NC, DOT>();
+  constexpr bool grp = spmv_grouped_call<MT, NC>();
   const unsigned grid = (unsigned)spmv_grid<MT, NC, DOT>(S);
 #define MVF_SPMV(L_, G_)                                                                                         \
   do {                                                                                                           \
@@ -1227,7 +1221,8 @@ static void spmv_launch(const Solver &S, const MT *K, const MT *M, const VT *x, 
       hipLaunchKernelGGL((k_spmv<VT, MT, MT, NC, L_, false, DOT, G_>), dim3(grid), dim3(kBS), 0, h->stream, S.n, \
                          h->d_rowptr, h->d_col, K, M, S.w, x, y, p, part);                                       \
   } while (0)
-  if (grp && S.grp) MVF_SPMV(kGrpLanes, grp);
+  if (grp && S.grp && lpr == 4) MVF_SPMV(4, grp);
+  else if (grp && S.grp) MVF_SPMV(8, grp);
   else if (sizeof(MT) == 8 && lpr == 4) MVF_SPMV(4, false);
   else if (sizeof(MT) == 8 && lpr == 8) MVF_SPMV(8, false);
   else if (sizeof(MT) == 8 && lpr == 32) MVF_SPMV(32, false);
@@ -1296,6 +1291,10 @@ static int cocg_persist_grid(mvf_handle *h, int64_t n, int &grid) {
   MVF_HIP(h, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, (const void *)k_cocg_persist<NC, LPR, C64>, kBS, 0));
   MVF_HIP(h, hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, h->device));
   int64_t g = (int64_t)per * ncu;
+  // small systems pay for the barriers by the block: one per CU (us per iteration
+  // at 256 / 512 blocks, four columns: 27-node 9k DOFs 108 / 175, 8-node 145k 153 /
+  // 213, 570k 379 / 377; sixteen: 20-node 129k 665 / 645, 590k 2737 / 2170)
+  if (n < 150000) g = std::min<int64_t>(g, ncu);
   // MVF_PERSIST_BLOCKS caps the grid: fewer blocks make the barriers and the
   // per-block reductions cheaper and leave fewer waves for the SpMV
   if (const char *e = getenv("MVF_PERSIST_BLOCKS")) {
@@ -1339,7 +1338,7 @@ static int cocg_persist(Solver &S, bool grid_only, int &grid, int iters, double 
                      : cocg_persist_run<NC, LPR_, false>(S, grid, iters, x, r, p, q, invd, spart, part, st, tol);  \
   } while (0)
   if constexpr (NC <= 4) {
-    if (short_rows(S.h)) MVF_PERSIST(kGrpLanes);
+    if (short_rows(S.h)) MVF_PERSIST(8);
     MVF_PERSIST(32);
   } else {
     switch (S.lpr) {
@@ -1757,17 +1756,32 @@ static int guess_scale(Solver &S, const double *b, double *x, double *alpha_out)
 
 constexpr int nc_slot(int nc) { return nc == 2 ? 0 : (nc == 4 ? 1 : (nc == 8 ? 2 : 3)); }
 
-// SpMV autotuner: the FP64 operator's lanes per row (4, 8, 16 or 32) timed
-// once per handle, column count and form (COCG runs the one with the dot product)
-// with HIP events (one warm-up and three timed launches each), the fastest kept
-// in the handle.  Rows of 8-node systems hold <= 33 entries, 20-node ~84, 27-node
-// ~104: the best width follows the row length and the column count.
+// the tuned form of a handle: lanes per row, negative for the grouped form
+static void spmv_take(Solver &S, int tuned) {
+  S.grp = tuned < 0;
+  S.lpr = tuned < 0 ? -tuned : tuned;
+}
+
+// SpMV autotuner: the FP64 operator's lanes per row (4, 8, 16 or 32, with two and
+// four columns also the grouped form at 4 and 8) timed once per handle, column
+// count and presence of the dot product (COCG runs it) with HIP events (one warm-up
+// and three timed launches each), the fastest kept in the handle.  Rows of 8-node
+// systems hold <= 33 entries, 20-node ~84, 27-node ~104: the best width follows the
+// row length, the column count and the size.  MVF_SPMV forces a form (4, 8, 16, 32;
+// -4, -8 grouped).
 template <int NC, bool DOT>
-static int tune_lpr(Solver &S) {
+static int tune_spmv(Solver &S) {
   mvf_handle *h = S.h;
-  int &slot = h->spmv_lpr[DOT][nc_slot(NC)];
+  int &slot = h->spmv_tuned[DOT][nc_slot(NC)];
+  constexpr int forms[] = {4, 8, 16, 32, -4, -8};
+  if (const char *e = getenv("MVF_SPMV"))
+    for (int t : forms)
+      if (atoi(e) == t && (t > 0 || spmv_grouped_call<double, NC>())) {
+        spmv_take(S, t);
+        return 0;
+      }
   if (slot) {
-    S.lpr = slot;
+    spmv_take(S, slot);
     return 0;
   }
   DevScope ds;
@@ -1782,12 +1796,11 @@ static int tune_lpr(Solver &S) {
   MVF_HIP(h, hipEventCreate(&e1));
   SpmvTimer *tm = S.tm;
   S.tm = nullptr;
-  const bool grp = S.grp;
-  S.grp = false;  // the plain form's width
   int best = 16;
   float best_ms = 1e30f;
-  for (int L : {4, 8, 16, 32}) {
-    S.lpr = L;
+  for (int t : forms) {
+    if (t < 0 && !spmv_grouped_call<double, NC>()) continue;
+    spmv_take(S, t);
     auto apply = [&]() { spmv_launch<double, double, NC, DOT>(S, h->d_K, h->d_M, xa, ya, DOT ? xa : nullptr, part); };
     apply();
     (void)hipEventRecord(e0, h->stream);
@@ -1796,16 +1809,15 @@ static int tune_lpr(Solver &S) {
     float ms = 0.f;
     if (hipEventSynchronize(e1) == hipSuccess && hipEventElapsedTime(&ms, e0, e1) == hipSuccess && ms < best_ms) {
       best_ms = ms;
-      best = L;
+      best = t;
     }
   }
   S.tm = tm;
-  S.grp = grp;
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   MVF_HIP(h, hipGetLastError());
   slot = best;
-  S.lpr = best;
+  spmv_take(S, best);
   return 0;
 }
 
@@ -1820,10 +1832,9 @@ static int solve_nc(mvf_handle *h, const double *omegas, int ncol, const mvf_sol
   tm->reset();
   Solver S{h, ncol, {}, o->matrix == MVF_MATRIX_C64REF, 16, (int64_t)h->nne, tm};
   for (int c = 0; c < NC; c++) S.w.w[c] = c < ncol ? (double)(float)omegas[c] : 0.0;
-  S.grp = spmv_grouped_rows(h);
   const bool cocg64 =
       o->precond != MVF_PC_DIRECT && o->precision != MVF_PREC_MIXED && o->method != MVF_KRYLOV_BICGSTAB;
-  int rc = !h->autotune ? 0 : cocg64 ? tune_lpr<NC, true>(S) : tune_lpr<NC, false>(S);
+  int rc = !h->autotune ? 0 : cocg64 ? tune_spmv<NC, true>(S) : tune_spmv<NC, false>(S);
   if (!rc && alpha_out) rc = guess_scale<NC>(S, b, x, alpha_out);
   if (rc) {
   } else if (o->precond == MVF_PC_DIRECT) rc = run_gmres_direct<NC>(S, o, b, x, info);
@@ -1841,7 +1852,7 @@ static int solve_nc(mvf_handle *h, const double *omegas, int ncol, const mvf_sol
   info->spmv_bytes[0] = nnz * ((S.c64 ? 4 : 8) + 8 + 4) + n * (8 + NC * (16 + 16));
   info->spmv_bytes[1] = nnz * (4 + 4 + 4) + n * (8 + NC * (8 + 8));
   info->spmv_ncol = NC;
-  info->spmv_lpr = NC == 4 && S.grp ? kGrpLanes : S.lpr;
+  info->spmv_lpr = S.lpr;
   return rc;
 }
 

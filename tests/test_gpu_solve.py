@@ -170,23 +170,49 @@ def test_cocg_columns_and_rows(nodes, sides, nf, matrix, need_gpu):
             assert r <= (1.1e-9 if matrix == "c64ref" else 1e-5), (i, d, r)
 
 
-@pytest.mark.parametrize("sides", [(44, 44, 36), (47, 50, 37)])  # 199k and 249k DOFs: on either side of the rule
-@pytest.mark.parametrize("method,nf", [("cocg", 2), ("cocg", 1), ("bicgstab", 1)])
-def test_spmv_large_grids(sides, method, nf, need_gpu):
-    """The SpMV's two forms at the sizes where the choice between them lies: four
-    and two columns with the dot product, two without it; the second grid's rows
-    fill no whole pass of the workgroups.  The bar is each column's residual formed
-    on the host, as in test_cocg_columns_and_rows."""
-    freqs = (50.0, 80.0)[:nf]
-    nx, ny, nz = sides
-    m = M.anisotropic_blocks(nx=nx, ny=ny, nz_earth=nz - 2, nz_air=2, h=500.0, nodes=8, freqs=freqs, block=4, seed=5,
-                             full_tensor=True, dirichlet=True, nextd=2)
+@pytest.mark.parametrize("form", [4, 8, 16, 32, -4, -8])  # lanes per row; negative: the grouped form
+@pytest.mark.parametrize("nodes,sides,method,nf", [
+    (8, (5, 4, 3), "cocg", 1),       # rows shorter than one pass, fewer rows than a workgroup takes
+    (8, (11, 9, 7), "cocg", 2),      # several workgroups, the last partly filled
+    (8, (11, 9, 7), "bicgstab", 2),  # without the dot product
+    (20, (4, 3, 3), "cocg", 2),      # ~84 entries: several passes
+    (20, (4, 3, 3), "bicgstab", 1),
+    (8, (5, 4, 3), "cocg", 3),       # eight columns: no grouped form, the autotuner's width instead
+])
+def test_spmv_forms(form, nodes, sides, method, nf, monkeypatch, need_gpu):
+    """Every form of the SpMV the autotuner can choose, forced: the residual of each
+    column, formed on the host, is at most the tolerance (as in
+    test_cocg_columns_and_rows)."""
+    monkeypatch.setenv("MVF_SPMV", str(form))
+    freqs = tuple(20.0 * 3.0 ** k for k in range(nf))
+    m = M.random_small(nodes, *sides, seed=41, full_tensor=True, freqs=freqs)
     g = GpuVfem(m, emulate=0)
-    info = g.solve_frequencies(freqs, method=method, tol=1e-8, maxit=20000)
-    print(f"SpMV form {sides} {method} nf={nf}: nne={g.nne} its={info['iterations']}", flush=True)
+    info = g.solve_frequencies(freqs, method=method, tol=1e-9, maxit=20000)
     assert info["converged"], info
+    assert nf == 3 or info["spmv_lpr"] == abs(form)
     x, bb = g.solution(2 * nf), g.rhs(2 * nf)
     for i in range(nf):
+        g.set_frequency(i)
+        A, _ = reference_system(g)
+        for d in range(2):
+            b = bb[2 * i + d]
+            assert np.linalg.norm(b - A @ x[2 * i + d]) <= 1.1e-9 * np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("form", [8, -8, 0])
+def test_spmv_large_grid(form, monkeypatch, need_gpu):
+    """249k DOFs, beyond the workgroups of either form (each takes several passes
+    over the rows, the last partly filled); form 0: the autotuner's choice."""
+    if form:
+        monkeypatch.setenv("MVF_SPMV", str(form))
+    freqs = (50.0, 80.0)
+    m = M.anisotropic_blocks(nx=47, ny=50, nz_earth=35, nz_air=2, h=500.0, nodes=8, freqs=freqs, block=4, seed=5,
+                             full_tensor=True, dirichlet=True, nextd=2)
+    g = GpuVfem(m, emulate=0)
+    info = g.solve_frequencies(freqs, method="cocg", tol=1e-8, maxit=20000)
+    assert info["converged"], info
+    x, bb = g.solution(4), g.rhs(4)
+    for i in range(2):
         g.set_frequency(i)
         A, _ = reference_system(g)
         for d in range(2):
